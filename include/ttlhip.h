@@ -326,6 +326,22 @@ int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B,
                 int b_dtype, int64_t ldb, void* C, int c_dtype, int64_t ldc,
                 int64_t M, int64_t N, int64_t K, int accumulate, void* stream);
 
+/* The same product with device memory for partial results: `scratch` is
+ * TTLH_MATMUL_SCRATCH_BYTES of caller-owned device memory, 16-byte aligned,
+ * zeroed once before its first use and then left to the library (NULL: none).
+ * Problems with few outputs then divide K among several workgroups per output
+ * block; sums are added in a fixed order, so results repeat exactly.  Launches
+ * that share a scratch must be ordered (one stream); while the stream is being
+ * captured the scratch is not used.  No counterpart in the reference (its
+ * kernels own a core's SRAM). */
+#define TTLH_MATMUL_SCRATCH_BYTES (4198400)
+
+int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,
+                        int b_dtype, int64_t ldb, void* C, int c_dtype,
+                        int64_t ldc, int64_t M, int64_t N, int64_t K,
+                        int accumulate, void* scratch, int64_t scratch_bytes,
+                        void* stream);
+
 /* ------------------------------------------------------------------------
  * Tile matmul with its store's elementwise program fused:
  *   out[y0 + i, x0 + j] = prog(round_bf16((A . B)[i, j]), operands...)

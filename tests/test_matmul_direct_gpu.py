@@ -1,0 +1,95 @@
+"""The register-direct GEMM kernels on the MI355X at the edges of their blocks:
+one tile of rows, columns that end inside a block, K shorter than the waves'
+stages, K divided among workgroups (scratch), outputs without vector
+alignment.  The reference is the float64 product of the same inputs.  Bounds
+as for the other GEMM kernels: fp32 sums of K products (1e-6 sqrt(K) of the
+largest result) and, for bf16 results, one rounding (2^-8 of the value)."""
+
+import math
+
+import pytest
+import torch
+
+from oracle import tile_ops as O
+from ttlhip import kernels as Kn
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): every block shape, whole and cut; K of one stage, of fewer stages
+# than waves, and long enough to be divided
+SHAPES = [(32, 32, 32), (32, 96, 96), (64, 4096, 96), (96, 2048, 160), (32, 11008, 288),
+          (160, 1024, 1056), (224, 544, 1504), (544, 288, 2080), (1056, 160, 3104),
+          (2080, 96, 2016)]
+
+
+def _check(got, a, b, bf16_out):
+    exact = a.cpu().double() @ b.cpu().double()
+    bound = 1e-6 * math.sqrt(a.shape[1]) * float(exact.abs().max())
+    if bf16_out:
+        bound = bound + exact.abs() * 2.0 ** -8
+    err = (got.cpu().double() - exact).abs()
+    assert bool((err <= bound).all()), float(err.max())
+
+
+def _operands(M, K, N, seed, dtype=torch.bfloat16):
+    std = K ** -0.25
+    return (O.seeded((M, K), "normal", seed, dtype, std=std).cuda(),
+            O.seeded((K, N), "normal", seed + 1, dtype, std=std).cuda())
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_bf16_blocks(M, K, N):
+    print(f"direct bf16 {M}x{K}x{N}", flush=True)
+    a, b = _operands(M, K, N, 3)
+    # a guard column on each side: results outside the block stay untouched,
+    # and the odd pitch takes the stores without vector alignment
+    buf = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device="cuda")
+    Kn.matmul(a, b, buf[:, 1:N + 1])
+    wide = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    for _ in range(3):  # the counters of the divided products reset themselves
+        wide.zero_()
+        Kn.matmul(a, b, wide)
+        _check(wide, a, b, True)
+    assert torch.equal(buf[:, 1:N + 1], wide)
+    assert bool((buf[:, 0] == 7).all()) and bool((buf[:, N + 1:] == 7).all())
+
+
+@pytest.mark.parametrize("M,K,N", [(32, 4096, 96), (96, 288, 1056)])
+def test_bf16_accumulate_f32(M, K, N):
+    a, b = _operands(M, K, N, 5)
+    c0 = O.seeded((M, N), "normal", 7, torch.float32).cuda()
+    c = c0.clone()
+    Kn.matmul(a, b, c, accumulate=True)
+    _check(c - c0, a, b, False)
+
+
+def test_divided_product_under_capture_and_on_two_streams():
+    # under capture K is not divided (a replay may run beside launches that use
+    # the scratch); two streams have a scratch each
+    a, b = _operands(32, 4096, 256, 9)
+    c = torch.zeros(32, 256, dtype=torch.bfloat16, device="cuda")
+    Kn.matmul(a, b, c)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    d = torch.zeros_like(c)
+    with torch.cuda.graph(g):
+        Kn.matmul(a, b, d)
+    for _ in range(3):
+        d.zero_()
+        g.replay()
+        Kn.matmul(a, b, c)
+        torch.cuda.synchronize()
+        _check(d, a, b, True)
+        _check(c, a, b, True)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[torch.zeros_like(c) for _ in range(8)] for _ in streams]
+    torch.cuda.synchronize()
+    for i in range(8):
+        for s, o in zip(streams, outs):
+            Kn.matmul(a, b, o[i], stream=s)
+    torch.cuda.synchronize()
+    for o in outs:
+        assert all(torch.equal(x, c) for x in o)
+    Kn.release_workspaces()
+    Kn.matmul(a, b, c)
+    _check(c, a, b, True)

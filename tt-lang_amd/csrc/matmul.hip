@@ -32,6 +32,7 @@
 #include "ttlh_bfp8.h"
 #include "ttlh_common.h"
 #include "ttlh_eltprog.h"
+#include "ttlh_matmul.h"
 
 namespace ttlh {
 namespace {
@@ -1828,9 +1829,11 @@ __global__ __launch_bounds__(256) void mm_f32_kernel(const MmArgsF p) {
 
 using namespace ttlh;
 
-extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B, int b_dtype,
-                           int64_t ldb, void* C, int c_dtype, int64_t ldc, int64_t M, int64_t N,
-                           int64_t K, int accumulate, void* stream) {
+namespace {
+
+int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dtype, int64_t ldb,
+                void* C, int c_dtype, int64_t ldc, int64_t M, int64_t N, int64_t K, int accumulate,
+                bool direct, void* scratch, void* stream) {
   clear_error();
   TTLH_REQUIRE(A && B && C, TTLH_EINVAL, "ttlh_matmul: null pointer");
   TTLH_REQUIRE(M > 0 && N > 0 && K > 0 && M % 32 == 0 && N % 32 == 0 && K % 32 == 0, TTLH_EINVAL,
@@ -1861,7 +1864,21 @@ extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* 
     a.c_dtype = c_dtype;
     a.accumulate = accumulate ? 1 : 0;
     int status = TTLH_OK;
-    if (launch_mm256<false>(a, s, &status)) return status;
+    // a 256-row block would be mostly padding for one or two tiles of rows
+    if (M > 64 && launch_mm256<false>(a, s, &status)) return status;
+    DirectArgs d = {};
+    d.A = A;
+    d.B = B;
+    d.C = C;
+    d.lda = lda;
+    d.ldb = ldb;
+    d.ldc = ldc;
+    d.M = a.M;
+    d.N = a.N;
+    d.K = a.K;
+    d.c_dtype = c_dtype;
+    d.accumulate = a.accumulate;
+    if (direct && launch_direct_bf16(d, scratch, s, &status)) return status;
     a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
     a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
     hipLaunchKernelGGL(mm_bf16_kernel<false>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0, s, a);
@@ -1882,6 +1899,28 @@ extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* 
   dim3 grid(static_cast<unsigned>((N + FBN - 1) / FBN), static_cast<unsigned>((M + FBM - 1) / FBM));
   hipLaunchKernelGGL(mm_f32_kernel, grid, dim3(256), 0, s, a);
   return check_launch("mm_f32_kernel");
+}
+
+}  // namespace
+
+extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B, int b_dtype,
+                           int64_t ldb, void* C, int c_dtype, int64_t ldc, int64_t M, int64_t N,
+                           int64_t K, int accumulate, void* stream) {
+  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, true,
+                     nullptr, stream);
+}
+
+extern "C" int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,
+                                   int b_dtype, int64_t ldb, void* C, int c_dtype, int64_t ldc,
+                                   int64_t M, int64_t N, int64_t K, int accumulate, void* scratch,
+                                   int64_t scratch_bytes, void* stream) {
+  clear_error();
+  TTLH_REQUIRE(!scratch || (scratch_bytes >= TTLH_MATMUL_SCRATCH_BYTES &&
+                            (reinterpret_cast<uintptr_t>(scratch) & 15) == 0),
+               TTLH_EINVAL, "ttlh_matmul_scratch: needs %d bytes, 16-byte aligned",
+               TTLH_MATMUL_SCRATCH_BYTES);
+  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, true,
+                     scratch, stream);
 }
 
 extern "C" int ttlh_matmul_eltwise(const void* A, int64_t lda, const void* B, int64_t ldb,
@@ -2037,6 +2076,7 @@ extern "C" int ttlh_matmul_bfp8w_ws(const void* A, int64_t lda, const void* Bq, 
   // pass 2: the bf16 GEMM.  The error text of a failing pass names it.
   int st = ttlh_bfp8_unpack(Bq, workspace, K, N, stream);
   if (st != TTLH_OK) return st;
-  return ttlh_matmul(A, TTLH_BF16, lda, workspace, TTLH_BF16, N, C, TTLH_BF16, ldc, M, N, K, 0,
-                     stream);
+  // (with the fused path's order of summation)
+  return matmul_with(A, TTLH_BF16, lda, workspace, TTLH_BF16, N, C, TTLH_BF16, ldc, M, N, K, 0,
+                     false, nullptr, stream);
 }

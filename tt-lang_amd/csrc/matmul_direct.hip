@@ -1,0 +1,393 @@
+// GEMM kernels that read their operands from global memory straight into the
+// MFMA registers, without LDS staging, for the problems that the 256x256 LDS
+// kernels (matmul.hip) leave most of the chip idle on: few rows of A (decode
+// steps, small batches) and outputs of few tiles.
+//
+// A workgroup owns one BM x BN output block and its WK waves split K between
+// them (wave w takes k stages w, w + WK, ...), so that a small output still
+// puts WK waves per block on the chip, each with its own loads in flight and
+// no barrier in the loop.  At the end the waves' partial blocks meet in LDS
+// and are summed in wave order: results repeat exactly.
+#include <algorithm>
+
+#include "ttlh_common.h"
+#include "ttlh_matmul.h"
+
+namespace ttlh {
+namespace {
+
+// Scratch: the arrival counters of at most 256 output blocks, then their parts
+// (at most 256 workgroups' blocks of 32 x 128).
+constexpr int kArrivedBytes = 1024;
+static_assert(TTLH_MATMUL_SCRATCH_BYTES >= kArrivedBytes + 256 * 32 * 128 * 4, "scratch size");
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+template <int N>
+struct WordVec;
+template <>
+struct WordVec<1> { typedef uint32_t type; };
+template <>
+struct WordVec<2> { typedef u32x2 type; };
+template <>
+struct WordVec<4> { typedef u32x4 type; };
+
+// A uniform base plus a 32-bit byte offset of the lane (one load instruction,
+// no 64-bit vector address arithmetic).
+template <typename T>
+__device__ __forceinline__ T gload(const void* base, uint32_t off) {
+  typedef const __attribute__((address_space(1))) T gT;
+  typedef const __attribute__((address_space(1))) char gchar;
+  return *reinterpret_cast<gT*>(reinterpret_cast<gchar*>(reinterpret_cast<uintptr_t>(base)) + off);
+}
+
+// A copy of a lane's byte offset that the compiler cannot widen to 64 bits
+// outside the loop (it would then add it with vector instructions instead of
+// using the load's scalar base).
+__device__ __forceinline__ uint32_t opaque(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// Output block of this workgroup.  Workgroup i runs on XCD i % 8: each XCD
+// takes a contiguous run of the block order, in which the row blocks of one
+// column of blocks follow each other (they share B through that XCD's L2).
+__device__ __forceinline__ void direct_block(const DirectArgs& p, int& bm, int& bn, int& split) {
+  const int n = gridDim.x, id = blockIdx.x;
+  const int per = n >> 3, rem = n & 7, x = id & 7;
+  const int i = x * per + min(x, rem) + (id >> 3);
+  const int j = i / p.grid_m;
+  bm = i - j * p.grid_m;
+  split = j / p.grid_n;
+  bn = j - split * p.grid_n;
+}
+
+// Four consecutive results of one row.  vec: the row pitch and the base allow
+// one store of all four.
+__device__ __forceinline__ void store4(const DirectArgs& p, int row, int col, f32x4 v) {
+  const int64_t off = static_cast<int64_t>(row) * p.ldc + col;
+  if (p.c_dtype == TTLH_BF16) {
+    uint16_t* c = static_cast<uint16_t*>(p.C) + off;
+    if (p.accumulate) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += bf16_to_f32(c[i]);
+    }
+    const u32x2 w = {cvt_pk_bf16x2(v[0], v[1]), cvt_pk_bf16x2(v[2], v[3])};
+    if (p.c_vec) {
+      *reinterpret_cast<u32x2*>(c) = w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i] = static_cast<uint16_t>(w[i >> 1] >> (16 * (i & 1)));
+    }
+  } else {
+    float* c = static_cast<float*>(p.C) + off;
+    if (p.accumulate) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += c[i];
+    }
+    if (p.c_vec) {
+      *reinterpret_cast<f32x4*>(c) = v;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i] = v[i];
+    }
+  }
+}
+
+// Four values of a part, to and from memory past the caches that other
+// workgroups' XCDs do not see: relaxed device-scope atomics, which write
+// through and read at the device's coherence point.
+__device__ __forceinline__ void put_part(float* d, f32x4 v) {
+  typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+  const u64x2 w = __builtin_bit_cast(u64x2, v);
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(d);
+  __hip_atomic_store(q, w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 get_part(const float* d) {
+  typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(d);
+  const u64x2 w = {__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                   __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+  return __builtin_bit_cast(f32x4, w);
+}
+
+// The sum over the waves' partial blocks in LDS (rows at a pitch of PITCH
+// floats), in wave order, and the store of the block.
+template <int BM, int BN, int PITCH, int WK, int THREADS>
+__device__ __forceinline__ void reduce_store(const DirectArgs& p, const float* part, int bm, int bn,
+                                             int split) {
+  constexpr int kChunks = BM * BN / 4;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const int block = bn * p.grid_m + bm;
+  float* mine = p.partial + static_cast<int64_t>(block * p.splits + split) * (BM * BN);
+  for (int c = threadIdx.x; c < kChunks; c += THREADS) {
+    const int r = c / (BN / 4), col = (c % (BN / 4)) * 4;
+    f32x4 s = *reinterpret_cast<const f32x4*>(part + r * PITCH + col);
+#pragma unroll
+    for (int w = 1; w < WK; ++w)
+      s += *reinterpret_cast<const f32x4*>(part + w * BM * PITCH + r * PITCH + col);
+    if (p.splits > 1)
+      put_part(mine + 4 * c, s);
+    else if (m0 + r < p.M && n0 + col < p.N)
+      store4(p, m0 + r, n0 + col, s);
+  }
+  if (p.splits == 1) return;
+  // The workgroup that arrives last at this block's counter adds the parts,
+  // in split order; nobody waits for anybody.  Every wave's parts are at the
+  // coherence point (vmcnt 0) before the barrier, so before thread 0 counts
+  // them in; a device-scope fence would do the same by writing back the whole
+  // L2 (measured: 20 us a launch).
+  __shared__ int last;
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(p.arrived + block, 1, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) == p.splits - 1;
+    if (last) __hip_atomic_store(p.arrived + block, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last) return;
+  const float* parts = p.partial + static_cast<int64_t>(block) * p.splits * (BM * BN);
+  for (int c = threadIdx.x; c < kChunks; c += THREADS) {
+    const int r = c / (BN / 4), col = (c % (BN / 4)) * 4;
+    f32x4 s = get_part(parts + 4 * c);
+    for (int w = 1; w < p.splits; ++w)
+      s += get_part(parts + static_cast<int64_t>(w) * (BM * BN) + 4 * c);
+    if (m0 + r < p.M && n0 + col < p.N) store4(p, m0 + r, n0 + col, s);
+  }
+}
+
+__device__ __forceinline__ uint32_t perm_lo(uint32_t x, uint32_t y) {
+  return __builtin_amdgcn_perm(y, x, 0x05040100u);  // lo16(x) | lo16(y) << 16
+}
+__device__ __forceinline__ uint32_t perm_hi(uint32_t x, uint32_t y) {
+  return __builtin_amdgcn_perm(y, x, 0x07060302u);
+}
+
+// ---------------------------------------------------------------------------
+// bf16 A and B.  Block of 16 MT rows x 16 NPL columns; a stage is 32 k.
+// v_mfma_f32_16x16x32_bf16 takes from lane l row / column l % 16 and k
+// 8 (l / 16) .. + 7.  A: one 16-byte load per lane and 16 rows.  B is stored
+// with n contiguous: the lane loads NPL adjacent columns of its eight k rows
+// (16 lanes cover the block's 32 NPL bytes of a row) and transposes them in
+// registers with v_perm_b32, column c of every lane feeding MFMA c, whose
+// columns are therefore NPL apart.  D stages are in flight per wave.
+template <int MT, int NPL, int D>
+struct BfStage {
+  typedef typename WordVec<NPL / 2>::type vec;
+  u32x4 a[MT];
+  vec b[8];
+};
+
+template <typename V>
+__device__ __forceinline__ uint32_t word(const V& v, int i) { return v[i]; }
+__device__ __forceinline__ uint32_t word(const uint32_t& v, int) { return v; }
+
+template <int MT, int NPL, int WK, int D, int OCC>
+__global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArgs p) {
+  constexpr int BM = 16 * MT, BN = 16 * NPL, PITCH = BN + 4;
+  __shared__ __attribute__((aligned(16))) float part[WK * BM * PITCH];
+  int bm, bn, split;
+  direct_block(p, bm, bn, split);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const uint16_t* A = static_cast<const uint16_t*>(p.A);
+  const uint16_t* B = static_cast<const uint16_t*>(p.B);
+
+  // lane offsets (bytes); rows past M and columns past N re-read the last
+  // ones, for results that are not stored
+  uint32_t a_off[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    a_off[i] = 2 * (static_cast<uint32_t>(min(m0 + 16 * i + l16, p.M - 1)) *
+                        static_cast<uint32_t>(p.lda) + 8 * kg);
+  const uint32_t b_off = 2 * (static_cast<uint32_t>(8 * kg) * static_cast<uint32_t>(p.ldb) +
+                              min(n0 + NPL * l16, p.N - NPL));
+
+  f32x4 acc[MT][NPL];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int stages = p.K / 32, first = split * WK + wave, step = p.splits * WK;
+  typedef BfStage<MT, NPL, D> Stage;
+  auto load = [&](Stage& s, int i) {  // the wave's i-th stage
+    const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 32;
+    const uint32_t bo = opaque(b_off);
+    const uint16_t* ak = A + k0;
+    const uint16_t* bk = B + k0 * p.ldb;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      s.b[j] = gload<typename Stage::vec>(bk + static_cast<int64_t>(j) * p.ldb, bo);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
+  };
+  auto compute = [&](const Stage& s) {
+#pragma unroll
+    for (int c = 0; c < NPL; ++c) {
+      u32x4 f;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t x = word(s.b[2 * d], c >> 1), y = word(s.b[2 * d + 1], c >> 1);
+        f[d] = (c & 1) ? perm_hi(x, y) : perm_lo(x, y);
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, f), acc[m][c], 0, 0, 0);
+    }
+  };
+
+  const int n = stages > first ? (stages - first + step - 1) / step : 0;
+  Stage st[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load(st[d], d);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int i = 0;
+  for (; i + 2 * D <= n; i += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      compute(st[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      load(st[d], i + D + d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    if (i + d < n) compute(st[d]);
+    if (i + D + d < n) load(st[d], i + D + d);
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (i + D + d < n) compute(st[d]);
+
+  // lane holds of MFMA (m, c): column NPL l16 + c, rows 16 m + 4 kg + r
+  float* mine = part + wave * BM * PITCH + (4 * kg) * PITCH + NPL * l16;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float* d = mine + (16 * m + r) * PITCH;
+      if constexpr (NPL == 2) {
+        *reinterpret_cast<f32x2*>(d) = f32x2{acc[m][0][r], acc[m][1][r]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < NPL; c += 4)
+          *reinterpret_cast<f32x4*>(d + c) =
+              f32x4{acc[m][c][r], acc[m][c + 1][r], acc[m][c + 2][r], acc[m][c + 3][r]};
+      }
+    }
+  __syncthreads();
+  reduce_store<BM, BN, PITCH, WK, 64 * WK>(p, part, bm, bn, split);
+}
+
+// ---------------------------------------------------------------------------
+// Choice of the kernel.
+
+// Parts of K for `blocks` output blocks of which the chip holds 256 at once
+// (one per CU): as many as fill it, at most four, while every wave keeps
+// `min_k` of K.  One part without scratch, or while the stream is being
+// captured: a replay may run beside other launches that use the scratch.
+int k_parts(int64_t blocks, int K, int min_k, void* scratch, hipStream_t s) {
+  int parts = 1;
+  while (parts < 4 && blocks * parts * 2 <= 256 && K >= min_k * parts * 2) parts *= 2;
+  if (parts == 1 || !scratch) return 1;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // not this launch's error
+    return 1;
+  }
+  return st == hipStreamCaptureStatusNone ? parts : 1;
+}
+
+void set_blocks(DirectArgs& a, int bm, int bn, int splits, void* scratch) {
+  a.grid_m = (a.M + bm - 1) / bm;
+  a.grid_n = (a.N + bn - 1) / bn;
+  a.splits = splits;
+  a.arrived = static_cast<int32_t*>(scratch);
+  a.partial = scratch ? reinterpret_cast<float*>(static_cast<char*>(scratch) + kArrivedBytes) : nullptr;
+}
+
+void set_c_vec(DirectArgs& a) {
+  const uintptr_t c = reinterpret_cast<uintptr_t>(a.C);
+  a.c_vec = a.ldc % 4 == 0 && c % (a.c_dtype == TTLH_BF16 ? 8 : 16) == 0;
+}
+
+int64_t blocks_of(const DirectArgs& a, int bm, int bn) {
+  return static_cast<int64_t>((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+}
+
+// lane offsets are 32-bit bytes
+bool offsets_fit(const DirectArgs& a, int elem) {
+  return static_cast<int64_t>(a.M) * a.lda * elem < (int64_t(1) << 32) &&
+         (24 * a.ldb + a.N) * elem < (int64_t(1) << 32);
+}
+
+#define TTLH_DIRECT(kernel, waves, name)                                                      \
+  do {                                                                                        \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME kernel, dim3(a.grid_m * a.grid_n * a.splits),          \
+                       dim3(64 * (waves)), 0, s, a);                                          \
+    *status = check_launch(name);                                                             \
+  } while (0)
+
+}  // namespace
+
+bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status) {
+  if (!offsets_fit(a, 2)) return false;
+  set_c_vec(a);
+  // Modelled time of each shape, us: per round of workgroups the chip holds
+  // at once, a fixed part and one per 32-k stage, both fitted to measurements
+  // of 32 problems from 32x512x512 to 4096x512x2048 (the choice was within 8%
+  // of the best measured shape on 28 of them, within 20% on all).
+  const double k = a.K / 32.0;
+  const auto rounds = [](int64_t blocks, int held) {
+    return static_cast<double>((blocks + held - 1) / held);
+  };
+  const int64_t b64 = blocks_of(a, 32, 64), b128 = blocks_of(a, 32, 128), m64 = blocks_of(a, 64, 128),
+                lds = blocks_of(a, 128, 128);
+  const int p64 = k_parts(b64, a.K, 1024, scratch, s);
+  const int p128 = b128 >= 80 ? std::min(2, k_parts(b128, a.K, 1024, scratch, s)) : 1;
+  const double t[6] = {
+      2 + 0.11 * k / p64 * rounds(b64 * p64, 256) + (p64 > 1 ? 2 : 0),
+      2 + 0.153 * k / p128 * rounds(b128 * p128, 256) + (p128 > 1 ? 2 : 0),
+      3 + k * (b128 <= 256 ? 0.17 : 0.267 * std::max(1.0, b128 / 512.0)),
+      3 + 0.237 * k * rounds(m64, 256),
+      (6 + 0.4 * k) * rounds(m64, 512),
+      10 + 0.57 * k * std::max(1.0, 0.65 * rounds(lds, 256)),  // 128x128 through LDS (matmul.hip)
+  };
+  switch (std::min_element(t, t + 6) - t) {
+    case 0:
+      set_blocks(a, 32, 64, p64, scratch);
+      TTLH_DIRECT((mm_direct_kernel<2, 4, 8, 3, 3>), 8, "mm_direct_kernel");
+      return true;
+    case 1:
+      set_blocks(a, 32, 128, p128, scratch);
+      TTLH_DIRECT((mm_direct_kernel<2, 8, 8, 2, 2>), 8, "mm_direct_kernel");
+      return true;
+    case 2:
+      set_blocks(a, 32, 128, 1, nullptr);
+      TTLH_DIRECT((mm_direct_kernel<2, 8, 4, 3, 2>), 4, "mm_direct_kernel");
+      return true;
+    case 3:
+      set_blocks(a, 64, 128, 1, nullptr);
+      TTLH_DIRECT((mm_direct_kernel<4, 8, 4, 2, 2>), 4, "mm_direct_kernel");
+      return true;
+    case 4:
+      set_blocks(a, 64, 128, 1, nullptr);
+      TTLH_DIRECT((mm_direct_kernel<4, 8, 2, 2, 1>), 2, "mm_direct_kernel");
+      return true;
+    default:
+      return false;
+  }
+}
+
+}  // namespace ttlh

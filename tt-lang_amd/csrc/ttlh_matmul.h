@@ -1,0 +1,28 @@
+// Register-direct GEMM kernels (matmul_direct.hip), chosen and launched for
+// the entry points in matmul.hip.
+#pragma once
+
+#include "ttlh_common.h"
+
+namespace ttlh {
+
+struct DirectArgs {
+  const void* A;  // bf16, row-major
+  const void* B;  // bf16, row-major [K, N]
+  void* C;
+  int64_t lda, ldb, ldc;
+  int32_t M, N, K;
+  int32_t c_dtype, accumulate, c_vec;  // c_vec: four results are one aligned store
+  int32_t grid_m, grid_n;
+  int32_t splits;    // workgroups per output block, each a part of K
+  float* partial;    // splits > 1: fp32 blocks of the parts
+  int32_t* arrived;  // ... and a counter per output block, 0 between launches
+};
+
+// Launches the product (M, N, K multiples of 32) and returns true with
+// the launch's status in *status, or returns false, having launched nothing,
+// where the caller's other kernels take the problem.  `scratch`: null, or
+// TTLH_MATMUL_SCRATCH_BYTES of device memory (see ttlh_matmul_scratch).
+bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status);
+
+}  // namespace ttlh

@@ -61,6 +61,7 @@ class Instr(C.Structure):
 # ttlh_reduce kinds and dimension bits
 REDUCE_SUM, REDUCE_MAX = 0, 1
 REDUCE_DIM0, REDUCE_DIM1 = 1, 2
+MATMUL_SCRATCH_BYTES = 4198400
 
 
 class Operand(C.Structure):
@@ -101,6 +102,8 @@ SIGNATURES = {
                                         _i64, _i64, _vp]),
     "ttlh_matmul": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64, _i64,
                            _int, _vp]),
+    "ttlh_matmul_scratch": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64,
+                                   _i64, _int, _vp, _i64, _vp]),
     "ttlh_matmul_eltwise": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, C.POINTER(Instr),
                                    C.POINTER(Operand), _int, _int, _vp, _int, _i64, _i64, _i64,
                                    _vp]),

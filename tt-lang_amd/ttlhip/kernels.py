@@ -68,10 +68,33 @@ def _workspace(device: torch.device, stream, nbytes: int) -> torch.Tensor:
     return ws
 
 
+# The matmul's scratch (partial sums of products that divide K among several
+# workgroups, and their counters): a fixed 4 MiB per (device, stream), zeroed
+# once and left to the library.  Never allocated while the stream is being
+# captured; the library does not use it there either, so no graph holds it.
+_MATMUL_SCRATCH: dict = {}
+
+
+def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Tensor]:
+    key = (device.index, sp)
+    t = _MATMUL_SCRATCH.get(key)
+    if t is None:
+        s = stream if stream is not None else torch.cuda.current_stream()
+        if s.device.index != device.index:
+            return None  # the zeroing would not be ordered before the launch
+        with torch.cuda.stream(s):
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            t = torch.zeros(L.MATMUL_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+        t = _MATMUL_SCRATCH.setdefault(key, t)
+    return t
+
+
 def release_workspaces() -> None:
     """Drop the cached workspaces (their memory returns to torch's caching
     allocator once the work queued on them has finished)."""
     _WORKSPACES.clear()
+    _MATMUL_SCRATCH.clear()
 
 
 def _axis_range(lo: int, n: int, mask: int, off: int):
@@ -298,9 +321,12 @@ def matmul(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, accumulate: bool =
     K2, N = b.shape
     if K2 != K or tuple(c.shape) != (M, N):
         raise ValueError(f"matmul shapes {tuple(a.shape)} @ {tuple(b.shape)} -> {tuple(c.shape)}")
-    L.call("ttlh_matmul", a.data_ptr(), L.dtype_code(a.dtype), a.stride(0), b.data_ptr(),
+    sp = L.stream_ptr(stream)
+    scratch = _matmul_scratch(c.device, stream, sp)
+    L.call("ttlh_matmul_scratch", a.data_ptr(), L.dtype_code(a.dtype), a.stride(0), b.data_ptr(),
            L.dtype_code(b.dtype), b.stride(0), c.data_ptr(), L.dtype_code(c.dtype), c.stride(0),
-           M, N, K, int(bool(accumulate)), L.stream_ptr(stream))
+           M, N, K, int(bool(accumulate)), scratch.data_ptr() if scratch is not None else 0,
+           L.MATMUL_SCRATCH_BYTES, sp)
 
 
 # Ops the fused GEMM epilogue (ttlh_matmul_eltwise) runs: + - * / max min
