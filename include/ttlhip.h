@@ -326,14 +326,18 @@ int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B,
                 int b_dtype, int64_t ldb, void* C, int c_dtype, int64_t ldc,
                 int64_t M, int64_t N, int64_t K, int accumulate, void* stream);
 
-/* The same product with device memory for partial results: `scratch` is
- * TTLH_MATMUL_SCRATCH_BYTES of caller-owned device memory, 16-byte aligned,
+/* The same product with device memory for partial results, and with packed
+ * weights: b_dtype may also be TTLH_BFP8 or TTLH_BFP4 (B the tile array of a
+ * K x N matrix, 8-byte aligned, ldb ignored; A and C bf16, accumulate 0).
+ * `scratch` is TTLH_MATMUL_SCRATCH_BYTES of caller-owned device memory, 16-byte aligned,
  * zeroed once before its first use and then left to the library (NULL: none).
  * Problems with few outputs then divide K among several workgroups per output
  * block; sums are added in a fixed order, so results repeat exactly.  Launches
  * that share a scratch must be ordered (one stream); while the stream is being
  * captured the scratch is not used.  No counterpart in the reference (its
  * kernels own a core's SRAM). */
+#define TTLH_BFP8 8
+#define TTLH_BFP4 4
 #define TTLH_MATMUL_SCRATCH_BYTES (4198400)
 
 int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,

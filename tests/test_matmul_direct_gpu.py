@@ -10,6 +10,7 @@ import math
 import pytest
 import torch
 
+from oracle import bfp8 as OB
 from oracle import tile_ops as O
 from ttlhip import kernels as Kn
 
@@ -93,3 +94,54 @@ def test_divided_product_under_capture_and_on_two_streams():
     Kn.release_workspaces()
     Kn.matmul(a, b, c)
     _check(c, a, b, True)
+
+
+def _packed(w, bits):
+    return OB.pack_c(w) if bits == 8 else OB.pack4_c(w)
+
+
+def _unpacked(q, K, N, bits):
+    return OB.unpack_c(q, K, N) if bits == 8 else OB.unpack4_c(q, K, N)
+
+
+def _matmul_packed(a, q, c, bits):
+    if bits == 8:
+        Kn.matmul_bfp8w(a, q, c, two_pass=False)
+    else:
+        Kn.matmul_bfp4w(a, q, c)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M,K,N", [s for s in SHAPES if s[0] < 512] + [(480, 160, 1504)])
+def test_packed_weights(M, K, N, bits):
+    print(f"direct packed {bits} {M}x{K}x{N}", flush=True)
+    a = O.seeded((M, K), "normal", 21, torch.bfloat16, std=K ** -0.5).cuda()
+    q = _packed(O.seeded((K, N), "normal", 22, torch.float32), bits)
+    w = _unpacked(q, K, N, bits)
+    qd = q.cuda()
+    c = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    for _ in range(2):
+        c.zero_()
+        _matmul_packed(a, qd, c, bits)
+        _check(c, a, w, True)
+    off = torch.empty(q.numel() + 8, dtype=torch.uint8, device="cuda")[8:]
+    off.copy_(qd)  # tiles on 8 bytes, not 16
+    d = torch.empty_like(c)
+    _matmul_packed(a, off, d, bits)
+    assert torch.equal(c, d)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("K", [96, 352])
+def test_packed_decode_is_exact(K, bits):
+    # rows of the identity read the weights themselves: random bytes with every
+    # finite exponent, subnormal results among them
+    N, per = 160, 1088 if bits == 8 else 576
+    g = torch.Generator().manual_seed(31)
+    q = torch.randint(0, 256, ((K // 32) * (N // 32), per), generator=g, dtype=torch.uint8)
+    q[:, :64] = torch.randint(0, 255, (q.shape[0], 64), generator=g, dtype=torch.uint8)
+    q = q.flatten()
+    c = torch.empty(K, N, dtype=torch.bfloat16, device="cuda")
+    _matmul_packed(torch.eye(K, dtype=torch.bfloat16, device="cuda"), q.cuda(), c, bits)
+    w = _unpacked(q, K, N, bits)
+    assert torch.equal(c.cpu().float(), w.float())

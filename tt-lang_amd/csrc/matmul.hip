@@ -1833,7 +1833,7 @@ namespace {
 
 int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dtype, int64_t ldb,
                 void* C, int c_dtype, int64_t ldc, int64_t M, int64_t N, int64_t K, int accumulate,
-                bool direct, void* scratch, void* stream) {
+                void* scratch, void* stream) {
   clear_error();
   TTLH_REQUIRE(A && B && C, TTLH_EINVAL, "ttlh_matmul: null pointer");
   TTLH_REQUIRE(M > 0 && N > 0 && K > 0 && M % 32 == 0 && N % 32 == 0 && K % 32 == 0, TTLH_EINVAL,
@@ -1878,7 +1878,7 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
     d.K = a.K;
     d.c_dtype = c_dtype;
     d.accumulate = a.accumulate;
-    if (direct && launch_direct_bf16(d, scratch, s, &status)) return status;
+    if (launch_direct_bf16(d, scratch, s, &status)) return status;
     a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
     a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
     hipLaunchKernelGGL(mm_bf16_kernel<false>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0, s, a);
@@ -1901,13 +1901,62 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
   return check_launch("mm_f32_kernel");
 }
 
+// bf16 A times packed weights (bits 8: bfloat8_b, 4: bfloat4_b), decoded on
+// their way to the MFMAs
+int matmul_block(const char* fn, int bits, const void* A, int64_t lda, const void* Bq, void* C,
+                 int64_t ldc, int64_t M, int64_t N, int64_t K, void* scratch, void* stream) {
+  clear_error();
+  TTLH_REQUIRE(A && Bq && C, TTLH_EINVAL, "%s: null pointer", fn);
+  TTLH_REQUIRE(M > 0 && N > 0 && K > 0 && M % 32 == 0 && N % 32 == 0 && K % 32 == 0, TTLH_EINVAL,
+               "%s: M, N, K must be positive multiples of 32", fn);
+  TTLH_REQUIRE(M < (1 << 30) && N < (1 << 30) && K < (1 << 30), TTLH_EUNSUPPORTED,
+               "%s: dimension too large", fn);
+  TTLH_REQUIRE(lda >= K && ldc >= N && lda % 8 == 0, TTLH_EINVAL,
+               "%s: bad leading dims", fn);
+  TTLH_REQUIRE((reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(Bq) & 7) == 0,
+               TTLH_EINVAL, "%s: A must be 16-byte and Bq 8-byte aligned", fn);
+  MmArgs a = {};
+  a.A = static_cast<const uint16_t*>(A);
+  a.Bq = static_cast<const uint8_t*>(Bq);
+  a.bq_tiles_n = static_cast<int32_t>(N / 32);
+  a.C = C;
+  a.lda = lda;
+  a.ldb = N;
+  a.ldc = ldc;
+  a.M = static_cast<int32_t>(M);
+  a.N = static_cast<int32_t>(N);
+  a.K = static_cast<int32_t>(K);
+  a.c_dtype = TTLH_BF16;
+  a.accumulate = 0;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  int status = TTLH_OK;
+  if (bits == 8 && M > 64 && launch_mm256<true>(a, s, &status)) return status;
+  DirectArgs d = {};
+  d.A = A;
+  d.B = Bq;
+  d.C = C;
+  d.lda = lda;
+  d.ldc = ldc;
+  d.M = a.M;
+  d.N = a.N;
+  d.K = a.K;
+  d.c_dtype = TTLH_BF16;
+  if (launch_direct_block(d, bits, scratch, s, &status)) return status;
+  TTLH_REQUIRE(bits == 8, TTLH_EUNSUPPORTED, "%s: row stride too large", fn);
+  a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
+  a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
+  hipLaunchKernelGGL(mm_bf16_kernel<true>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0,
+                     s, a);
+  return check_launch("mm_bf16_kernel<bfp8>");
+}
+
 }  // namespace
 
 extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B, int b_dtype,
                            int64_t ldb, void* C, int c_dtype, int64_t ldc, int64_t M, int64_t N,
                            int64_t K, int accumulate, void* stream) {
-  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, true,
-                     nullptr, stream);
+  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, nullptr,
+                     stream);
 }
 
 extern "C" int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,
@@ -1919,8 +1968,14 @@ extern "C" int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, cons
                             (reinterpret_cast<uintptr_t>(scratch) & 15) == 0),
                TTLH_EINVAL, "ttlh_matmul_scratch: needs %d bytes, 16-byte aligned",
                TTLH_MATMUL_SCRATCH_BYTES);
-  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, true,
-                     scratch, stream);
+  if (b_dtype == TTLH_BFP8 || b_dtype == TTLH_BFP4) {
+    TTLH_REQUIRE(a_dtype == TTLH_BF16 && c_dtype == TTLH_BF16 && !accumulate, TTLH_EUNSUPPORTED,
+                 "ttlh_matmul_scratch: packed weights take bf16 A and C and no accumulation");
+    return matmul_block(b_dtype == TTLH_BFP8 ? "ttlh_matmul_bfp8w" : "ttlh_matmul_bfp4w",
+                        b_dtype == TTLH_BFP8 ? 8 : 4, A, lda, B, C, ldc, M, N, K, scratch, stream);
+  }
+  return matmul_with(A, a_dtype, lda, B, b_dtype, ldb, C, c_dtype, ldc, M, N, K, accumulate, scratch,
+                     stream);
 }
 
 extern "C" int ttlh_matmul_eltwise(const void* A, int64_t lda, const void* B, int64_t ldb,
@@ -2021,36 +2076,7 @@ extern "C" int ttlh_matmul_eltwise(const void* A, int64_t lda, const void* B, in
 
 extern "C" int ttlh_matmul_bfp8w(const void* A, int64_t lda, const void* Bq, void* C, int64_t ldc,
                                  int64_t M, int64_t N, int64_t K, void* stream) {
-  clear_error();
-  TTLH_REQUIRE(A && Bq && C, TTLH_EINVAL, "ttlh_matmul_bfp8w: null pointer");
-  TTLH_REQUIRE(M > 0 && N > 0 && K > 0 && M % 32 == 0 && N % 32 == 0 && K % 32 == 0, TTLH_EINVAL,
-               "ttlh_matmul_bfp8w: M, N, K must be positive multiples of 32");
-  TTLH_REQUIRE(M < (1 << 30) && N < (1 << 30) && K < (1 << 30), TTLH_EUNSUPPORTED,
-               "ttlh_matmul_bfp8w: dimension too large");
-  TTLH_REQUIRE(lda >= K && ldc >= N && lda % 8 == 0, TTLH_EINVAL,
-               "ttlh_matmul_bfp8w: bad leading dims");
-  TTLH_REQUIRE((reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(Bq) & 7) == 0,
-               TTLH_EINVAL, "ttlh_matmul_bfp8w: A must be 16-byte and Bq 8-byte aligned");
-  MmArgs a = {};
-  a.A = static_cast<const uint16_t*>(A);
-  a.Bq = static_cast<const uint8_t*>(Bq);
-  a.bq_tiles_n = static_cast<int32_t>(N / 32);
-  a.C = C;
-  a.lda = lda;
-  a.ldb = N;
-  a.ldc = ldc;
-  a.M = static_cast<int32_t>(M);
-  a.N = static_cast<int32_t>(N);
-  a.K = static_cast<int32_t>(K);
-  a.c_dtype = TTLH_BF16;
-  a.accumulate = 0;
-  int status = TTLH_OK;
-  if (launch_mm256<true>(a, static_cast<hipStream_t>(stream), &status)) return status;
-  a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
-  a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
-  hipLaunchKernelGGL(mm_bf16_kernel<true>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0,
-                     static_cast<hipStream_t>(stream), a);
-  return check_launch("mm_bf16_kernel<bfp8>");
+  return matmul_block("ttlh_matmul_bfp8w", 8, A, lda, Bq, C, ldc, M, N, K, nullptr, stream);
 }
 
 extern "C" int64_t ttlh_matmul_bfp8w_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -2076,7 +2102,6 @@ extern "C" int ttlh_matmul_bfp8w_ws(const void* A, int64_t lda, const void* Bq, 
   // pass 2: the bf16 GEMM.  The error text of a failing pass names it.
   int st = ttlh_bfp8_unpack(Bq, workspace, K, N, stream);
   if (st != TTLH_OK) return st;
-  // (with the fused path's order of summation)
-  return matmul_with(A, TTLH_BF16, lda, workspace, TTLH_BF16, N, C, TTLH_BF16, ldc, M, N, K, 0,
-                     false, nullptr, stream);
+  return ttlh_matmul(A, TTLH_BF16, lda, workspace, TTLH_BF16, N, C, TTLH_BF16, ldc, M, N, K, 0,
+                     stream);
 }

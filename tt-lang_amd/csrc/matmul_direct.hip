@@ -1,7 +1,8 @@
 // GEMM kernels that read their operands from global memory straight into the
 // MFMA registers, without LDS staging, for the problems that the 256x256 LDS
 // kernels (matmul.hip) leave most of the chip idle on: few rows of A (decode
-// steps, small batches) and outputs of few tiles.
+// steps, small batches) and outputs of few tiles, with bf16 or block-float
+// weights.
 //
 // A workgroup owns one BM x BN output block and its WK waves split K between
 // them (wave w takes k stages w, w + WK, ...), so that a small output still
@@ -24,6 +25,7 @@ static_assert(TTLH_MATMUL_SCRATCH_BYTES >= kArrivedBytes + 256 * 32 * 128 * 4, "
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4a8 __attribute__((aligned(8)));  // packed tiles may be 8-byte aligned
 
 template <int N>
 struct WordVec;
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, kg = lane >> 4;
   const int m0 = bm * BM, n0 = bn * BN;
-  const uint16_t* A = static_cast<const uint16_t*>(p.A);
+  const uint16_t* A = static_cast<const uint16_t*>(p.A) + static_cast<int64_t>(m0) * p.lda;
   const uint16_t* B = static_cast<const uint16_t*>(p.B);
 
   // lane offsets (bytes); rows past M and columns past N re-read the last
@@ -204,7 +206,7 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
   uint32_t a_off[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
-    a_off[i] = 2 * (static_cast<uint32_t>(min(m0 + 16 * i + l16, p.M - 1)) *
+    a_off[i] = 2 * (static_cast<uint32_t>(min(16 * i + l16, p.M - 1 - m0)) *
                         static_cast<uint32_t>(p.lda) + 8 * kg);
   const uint32_t b_off = 2 * (static_cast<uint32_t>(8 * kg) * static_cast<uint32_t>(p.ldb) +
                               min(n0 + NPL * l16, p.N - NPL));
@@ -291,6 +293,196 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
 }
 
 // ---------------------------------------------------------------------------
+// bf16 A, block-float B (BITS 8: bfloat8_b, 4: bfloat4_b).  Block of 16 MT
+// rows x 32 NT columns; a stage is one tile row (32 k).  Lane l loads face row
+// l of each tile (16 or 8 bytes, contiguous over the wave) and its exponent
+// byte l, so the 16 elements that it decodes share one shift; it writes them
+// as bf16 to the wave's own LDS, from where ds_read_b64_tr_b16 gives the
+// MFMA's B operand (lane l of 16: column l of four 32-byte row pieces).
+// Decoding bounds this kernel (3.6 VALU instructions an element), not the
+// packed bytes' 8 to 9 us.
+template <int MT, int NT, int BITS>
+struct BqStage {
+  u32x4 a[MT];
+  u32x4 q[NT];     // element bytes of face row `lane` (bfloat4_b: 8 bytes)
+  uint32_t e[NT];  // its exponent
+};
+
+// two elements (bytes 0, 1 or 2, 3 of w; m: their magnitudes) as bf16 bits.
+// v_cvt_f32_ubyte is written out: from shifts and masks the compiler extracts
+// every byte first.
+__device__ __forceinline__ uint32_t decode_pair(uint32_t w, uint32_t m, int shift, bool high) {
+  float x, y;
+  if (high) {
+    asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(x) : "v"(m));
+    asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(y) : "v"(m));
+  } else {
+    asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(x) : "v"(m));
+    asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(y) : "v"(m));
+  }
+  // exact: at most 7 significant bits, the low half of the pattern is zero
+  x = __builtin_amdgcn_ldexpf(x, shift);
+  y = __builtin_amdgcn_ldexpf(y, shift);
+  const uint32_t v = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
+  const uint32_t sign = __builtin_amdgcn_perm(w, w, high ? 0x030C020Cu : 0x010C000Cu);
+  return (sign & 0x80008000u) | v;
+}
+
+// eight nibbles (column order) -> eight bytes: sign in bit 7, magnitude below
+__device__ __forceinline__ u32x2 spread_nibbles(uint32_t w) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;  // even, odd columns
+  const uint32_t x = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+  const uint32_t y = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+  return u32x2{(x | (x << 4)) & 0x87878787u, (y | (y << 4)) & 0x87878787u};
+}
+
+template <int MT, int NT, int BITS, int WK, int D, int OCC>
+__global__ __launch_bounds__(64 * WK, OCC) void mm_direct_bq_kernel(const DirectArgs p) {
+  constexpr int BM = 16 * MT, BN = 32 * NT, PITCH = BN + 4;
+  constexpr int kTile = BITS == 8 ? TTLH_BFP8_TILE_BYTES : TTLH_BFP4_TILE_BYTES;
+  constexpr int kBias = BITS == 8 ? 133 : 129;
+  // decoded stage: k row r at position (r & 3) + 4 (r >> 3) + 16 ((r >> 2) & 1),
+  // which puts the rows of one transpose read on consecutive positions; the
+  // pitch is an odd number of 32-byte pieces, so 32 lanes' pieces fall in
+  // different banks
+  constexpr int kRow = 64 * NT + 32, kStageLds = 32 * kRow;
+  constexpr int kPart = BM * PITCH * 4;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[WK * (kPart > kStageLds ? kPart : kStageLds)];
+  int bm, bn, split;
+  direct_block(p, bm, bn, split);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int m0 = bm * BM;
+  const uint16_t* A = static_cast<const uint16_t*>(p.A) + static_cast<int64_t>(m0) * p.lda;
+  const uint8_t* Q = static_cast<const uint8_t*>(p.B);
+
+  uint32_t a_off[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    a_off[i] = 2 * (static_cast<uint32_t>(min(16 * i + l16, p.M - 1 - m0)) *
+                        static_cast<uint32_t>(p.lda) + 8 * kg);
+  const int tiles_n = p.N / 32;
+  // tiles past the last column re-read the last one
+  uint32_t q_off[NT], e_off[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    e_off[t] = static_cast<uint32_t>(min(bn * NT + t, tiles_n - 1)) * kTile + lane;
+    q_off[t] = e_off[t] + 64 + (BITS == 8 ? 15 : 7) * lane;
+  }
+  // face row `lane`: k row 16 (face / 2) + lane % 16, columns 16 (face % 2) ..
+  const int kr = 16 * (lane >> 5) + l16;
+  uint8_t* const put = lds + wave * kStageLds +
+                       ((kr & 3) + 4 * (kr >> 3) + 16 * ((kr >> 2) & 1)) * kRow +
+                       32 * ((lane >> 4) & 1);
+  // transpose read of k rows 8 kg + 4 half .. + 3: lane addresses row l16 / 4,
+  // columns 4 (l16 % 4) ..
+  uint8_t* const get = lds + wave * kStageLds + (4 * kg + (l16 >> 2)) * kRow + 8 * (l16 & 3);
+
+  f32x4 acc[MT][2 * NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int stages = p.K / 32, first = split * WK + wave, step = p.splits * WK;
+  typedef BqStage<MT, NT, BITS> Stage;
+  auto load = [&](Stage& s, int i) {
+    const int64_t st = min(first + i * step, stages - 1);
+    const uint16_t* ak = A + st * 32;
+    const uint8_t* qk = Q + st * (static_cast<int64_t>(tiles_n) * kTile);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if constexpr (BITS == 8) {
+        s.q[t] = gload<u32x4a8>(qk, opaque(q_off[t]));
+      } else {
+        const u32x2 v = gload<u32x2>(qk, opaque(q_off[t]));
+        s.q[t].x = v.x;
+        s.q[t].y = v.y;
+      }
+      s.e[t] = gload<uint8_t>(qk, opaque(e_off[t]));
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
+  };
+  typedef short i16x4 __attribute__((ext_vector_type(4)));
+  typedef short i16x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+  auto compute = [&](const Stage& s) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      u32x4 v = s.q[t];
+      if constexpr (BITS == 4) {
+        const u32x2 x = spread_nibbles(v.x), y = spread_nibbles(v.y);
+        v = u32x4{x.x, x.y, y.x, y.y};
+      }
+      const int shift = static_cast<int>(s.e[t]) - kBias;
+      uint32_t o[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t m = v[i] & 0x7f7f7f7fu;
+        o[2 * i] = decode_pair(v[i], m, shift, false);
+        o[2 * i + 1] = decode_pair(v[i], m, shift, true);
+      }
+      *reinterpret_cast<u32x4*>(put + 64 * t) = u32x4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<u32x4*>(put + 64 * t + 16) = u32x4{o[4], o[5], o[6], o[7]};
+    }
+    // (the wave reads what it wrote itself: LDS operations of one wave
+    // complete in order, so no barrier)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j) {
+      const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 32 * j));
+      const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 16 * kRow + 32 * j));
+      const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, w), acc[m][j], 0, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+  };
+
+  const int n = stages > first ? (stages - first + step - 1) / step : 0;
+  Stage st[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load(st[d], d);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int i = 0;
+  for (; i + 2 * D <= n; i += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      compute(st[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      load(st[d], i + D + d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    if (i + d < n) compute(st[d]);
+    if (i + D + d < n) load(st[d], i + D + d);
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (i + D + d < n) compute(st[d]);
+
+  __syncthreads();  // the stage buffers become the partial blocks
+  float* part = reinterpret_cast<float*>(lds);
+  float* d = part + wave * BM * PITCH + (4 * kg) * PITCH + l16;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[(16 * m + r) * PITCH + 16 * j] = acc[m][j][r];
+  __syncthreads();
+  reduce_store<BM, BN, PITCH, WK, 64 * WK>(p, part, bm, bn, split);
+}
+
+// ---------------------------------------------------------------------------
 // Choice of the kernel.
 
 // Parts of K for `blocks` output blocks of which the chip holds 256 at once
@@ -326,10 +518,9 @@ int64_t blocks_of(const DirectArgs& a, int bm, int bn) {
   return static_cast<int64_t>((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
 }
 
-// lane offsets are 32-bit bytes
+// lane offsets, inside a row block of A and a stage of B, are 32-bit bytes
 bool offsets_fit(const DirectArgs& a, int elem) {
-  return static_cast<int64_t>(a.M) * a.lda * elem < (int64_t(1) << 32) &&
-         (24 * a.ldb + a.N) * elem < (int64_t(1) << 32);
+  return 128 * a.lda * elem < (int64_t(1) << 32) && (24 * a.ldb + a.N) * elem < (int64_t(1) << 32);
 }
 
 #define TTLH_DIRECT(kernel, waves, name)                                                      \
@@ -388,6 +579,27 @@ bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status)
     default:
       return false;
   }
+}
+
+bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status) {
+  const int64_t row = static_cast<int64_t>(a.N / 32) *
+                      (bits == 8 ? TTLH_BFP8_TILE_BYTES : TTLH_BFP4_TILE_BYTES);
+  if (128 * a.lda * 2 >= (int64_t(1) << 32) || row >= (int64_t(1) << 32)) return false;
+  set_c_vec(a);
+  // A wave decodes the weights of its columns once for all its rows, so 64
+  // rows are taken as soon as such blocks fill most of the CUs: 64 x 4096 x
+  // 11008 20.6 us against 25.0, 1024^3 8.4 against 10.2; fewer blocks are
+  // faster in 32 rows: 512^3 4.8 against 5.6.
+  if (blocks_of(a, 64, 64) >= 160 && a.M > 32) {
+    set_blocks(a, 64, 64, 1, nullptr);
+    if (bits == 8) TTLH_DIRECT((mm_direct_bq_kernel<4, 2, 8, 4, 2, 2>), 4, "mm_direct_bq_kernel");
+    else TTLH_DIRECT((mm_direct_bq_kernel<4, 2, 4, 4, 2, 2>), 4, "mm_direct_bq_kernel");
+    return true;
+  }
+  set_blocks(a, 32, 64, k_parts(blocks_of(a, 32, 64), a.K, 1024, scratch, s), scratch);
+  if (bits == 8) TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>), 8, "mm_direct_bq_kernel");
+  else TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>), 8, "mm_direct_bq_kernel");
+  return true;
 }
 
 }  // namespace ttlh

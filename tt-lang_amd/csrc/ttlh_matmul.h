@@ -8,7 +8,7 @@ namespace ttlh {
 
 struct DirectArgs {
   const void* A;  // bf16, row-major
-  const void* B;  // bf16, row-major [K, N]
+  const void* B;  // bf16 row-major [K, N], or the packed block-float tiles
   void* C;
   int64_t lda, ldb, ldc;
   int32_t M, N, K;
@@ -19,10 +19,11 @@ struct DirectArgs {
   int32_t* arrived;  // ... and a counter per output block, 0 between launches
 };
 
-// Launches the product (M, N, K multiples of 32) and returns true with
+// Each launches the product (M, N, K multiples of 32) and returns true with
 // the launch's status in *status, or returns false, having launched nothing,
 // where the caller's other kernels take the problem.  `scratch`: null, or
 // TTLH_MATMUL_SCRATCH_BYTES of device memory (see ttlh_matmul_scratch).
 bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status);
+bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status);
 
 }  // namespace ttlh

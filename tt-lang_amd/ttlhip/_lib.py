@@ -62,6 +62,8 @@ class Instr(C.Structure):
 REDUCE_SUM, REDUCE_MAX = 0, 1
 REDUCE_DIM0, REDUCE_DIM1 = 1, 2
 MATMUL_SCRATCH_BYTES = 4198400
+# b_dtype codes of packed weights (ttlh_matmul_scratch)
+TTLH_BFP8, TTLH_BFP4 = 8, 4
 
 
 class Operand(C.Structure):

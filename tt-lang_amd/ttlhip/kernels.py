@@ -492,10 +492,21 @@ def bfp8_unpack(q: torch.Tensor, rows: int, cols: int, stream=None) -> torch.Ten
 
 
 # At and above this many rows of A the weight tiles are dequantised once into a
-# bf16 workspace and multiplied by the bf16 GEMM (ttlh_matmul_bfp8w_ws); below
-# it the fused kernel, which decodes each tile once per 256-row block of A, is
-# used (ttlh_matmul_bfp8w).
+# bf16 workspace and multiplied by the bf16 GEMM; below it the kernels that
+# decode on the way to the MFMAs, once per 32 or 64 rows of A, are used.  At
+# 512 x 4096 x 4096 the two take the same time (38 us decoding, 8 to 10 us for
+# the unpack and 29 for the GEMM), at 256 x 4096 x 11008 decoding takes 53 us
+# against 25 + 62.
 BFP8_TWO_PASS_MIN_M = 512
+BFP4_TWO_PASS_MIN_M = 512
+
+
+def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> None:
+    sp = L.stream_ptr(stream)
+    scratch = _matmul_scratch(c.device, stream, sp)
+    L.call("ttlh_matmul_scratch", a.data_ptr(), L.TTLH_BF16, a.stride(0), bq.data_ptr(), code, N,
+           c.data_ptr(), L.TTLH_BF16, c.stride(0), M, N, K, 0,
+           scratch.data_ptr() if scratch is not None else 0, L.MATMUL_SCRATCH_BYTES, sp)
 
 
 def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None,
@@ -516,8 +527,7 @@ def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
     if two_pass is None:  # the two-pass decode reads Bq in 16-byte words
         two_pass = M >= BFP8_TWO_PASS_MIN_M and bq.data_ptr() % 16 == 0
     if not two_pass:
-        L.call("ttlh_matmul_bfp8w", a.data_ptr(), a.stride(0), bq.data_ptr(), c.data_ptr(),
-               c.stride(0), M, N, K, L.stream_ptr(stream))
+        _matmul_packed(a, bq, L.TTLH_BFP8, c, M, N, K, stream)
         return
     nbytes = int(L.load().ttlh_matmul_bfp8w_workspace_bytes(M, N, K))
     ws = _workspace(c.device, stream, nbytes)
@@ -560,9 +570,9 @@ def bfp4_unpack(q: torch.Tensor, rows: int, cols: int, stream=None) -> torch.Ten
 
 
 def matmul_bfp4w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None) -> None:
-    """c[M,N] = a[M,K] (bf16) @ dequant(bq)[K,N] with bfloat4_b weights; the
-    dequantised weights go through a bf16 workspace (the cached one of c's
-    device and the stream)."""
+    """c[M,N] = a[M,K] (bf16) @ dequant(bq)[K,N] with bfloat4_b weights; from
+    BFP4_TWO_PASS_MIN_M rows on, the dequantised weights go through a bf16
+    workspace (the cached one of c's device and the stream)."""
     _check_device(a, "matmul_bfp4w A")
     _check_device(c, "matmul_bfp4w C")
     M, K = a.shape
@@ -573,6 +583,12 @@ def matmul_bfp4w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
         raise ValueError("matmul_bfp4w: Bq must be device uint8 tiles of a K x N matrix")
     if a.stride(1) != 1 or c.stride(1) != 1:
         raise ValueError("matmul_bfp4w: A and C must be row-major")
+    # (operands off their alignment go to the two passes at any M, which refuse
+    # them)
+    if (M < BFP4_TWO_PASS_MIN_M and bq.data_ptr() % 8 == 0 and a.data_ptr() % 16 == 0
+            and a.stride(0) % 8 == 0):
+        _matmul_packed(a, bq, L.TTLH_BFP4, c, M, N, K, stream)
+        return
     ws = _workspace(c.device, stream, K * N * 2)
     L.call("ttlh_matmul_bfp4w_ws", a.data_ptr(), a.stride(0), bq.data_ptr(), c.data_ptr(),
            c.stride(0), M, N, K, ws.data_ptr(), K * N * 2, L.stream_ptr(stream))
