@@ -55,6 +55,28 @@ def test_bf16_blocks(M, K, N):
     assert bool((buf[:, 0] == 7).all()) and bool((buf[:, N + 1:] == 7).all())
 
 
+@pytest.mark.parametrize("M,K,N", [(32, 32, 32), (64, 2048, 96), (96, 160, 224), (32, 4096, 32),
+                                   (544, 96, 608), (1056, 64, 1504), (1760, 96, 1792)])
+def test_f32_blocks(M, K, N):
+    print(f"direct f32 {M}x{K}x{N}", flush=True)
+    a, b = _operands(M, K, N, 13, torch.float32)
+    buf = torch.full((M, N + 3), 7.0, device="cuda")
+    Kn.matmul(a, b, buf[:, 1:N + 1])
+    wide = torch.zeros(M, N, device="cuda")
+    for _ in range(2):
+        Kn.matmul(a, b, wide)
+        _check(wide, a, b, False)
+    assert torch.equal(buf[:, 1:N + 1], wide)
+    assert bool((buf[:, 0] == 7).all()) and bool((buf[:, N + 1:] == 7).all())
+    Kn.matmul(a, b, wide, accumulate=True)
+    torch.testing.assert_close(wide, 2 * buf[:, 1:N + 1], rtol=1e-6, atol=1e-6)
+    # operands off the vector alignment take the kernel through LDS
+    oa, ob = torch.empty(M, K + 1, device="cuda"), torch.empty(K, N + 1, device="cuda")
+    oa[:, 1:], ob[:, 1:] = a, b
+    Kn.matmul(oa[:, 1:], ob[:, 1:], wide)
+    _check(wide, a, b, False)
+
+
 @pytest.mark.parametrize("M,K,N", [(32, 4096, 96), (96, 288, 1056)])
 def test_bf16_accumulate_f32(M, K, N):
     a, b = _operands(M, K, N, 5)

@@ -1759,8 +1759,8 @@ bool launch_mm256(MmArgs a, hipStream_t s, int* status) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32: 64x64 blocks, 4 waves (2x2) of 32x32 v_mfma_f32_32x32x2f32 tiles,
-// BK = 32 through LDS (A row-major, B row-major; the f32 MFMA operands are
+// fp32 operands without the alignment of mm_direct_f32_kernel: 64x64 blocks,
+// 4 waves (2x2) of 32x32 v_mfma_f32_32x32x2f32 tiles, BK = 32 through LDS (A row-major, B row-major; the f32 MFMA operands are
 // single elements, read with ds_read_b32).
 struct MmArgsF {
   const float* A;
@@ -1847,6 +1847,19 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
   TTLH_REQUIRE(a_dtype == b_dtype && (a_dtype == TTLH_BF16 || a_dtype == TTLH_F32),
                TTLH_EUNSUPPORTED, "ttlh_matmul: A and B must both be bf16 or both f32");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  int status = TTLH_OK;
+  DirectArgs d = {};
+  d.A = A;
+  d.B = B;
+  d.C = C;
+  d.lda = lda;
+  d.ldb = ldb;
+  d.ldc = ldc;
+  d.M = static_cast<int32_t>(M);
+  d.N = static_cast<int32_t>(N);
+  d.K = static_cast<int32_t>(K);
+  d.c_dtype = c_dtype;
+  d.accumulate = accumulate ? 1 : 0;
   if (a_dtype == TTLH_BF16) {
     TTLH_REQUIRE((reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(B) & 15) == 0 && lda % 8 == 0 && ldb % 8 == 0,
@@ -1863,27 +1876,15 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
     a.K = static_cast<int32_t>(K);
     a.c_dtype = c_dtype;
     a.accumulate = accumulate ? 1 : 0;
-    int status = TTLH_OK;
     // a 256-row block would be mostly padding for one or two tiles of rows
     if (M > 64 && launch_mm256<false>(a, s, &status)) return status;
-    DirectArgs d = {};
-    d.A = A;
-    d.B = B;
-    d.C = C;
-    d.lda = lda;
-    d.ldb = ldb;
-    d.ldc = ldc;
-    d.M = a.M;
-    d.N = a.N;
-    d.K = a.K;
-    d.c_dtype = c_dtype;
-    d.accumulate = a.accumulate;
     if (launch_direct_bf16(d, scratch, s, &status)) return status;
     a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
     a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
     hipLaunchKernelGGL(mm_bf16_kernel<false>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0, s, a);
     return check_launch("mm_bf16_kernel");
   }
+  if (launch_direct_f32(d, scratch, s, &status)) return status;
   MmArgsF a;
   a.A = static_cast<const float*>(A);
   a.B = static_cast<const float*>(B);

@@ -1,8 +1,7 @@
 // GEMM kernels that read their operands from global memory straight into the
 // MFMA registers, without LDS staging, for the problems that the 256x256 LDS
 // kernels (matmul.hip) leave most of the chip idle on: few rows of A (decode
-// steps, small batches) and outputs of few tiles, with bf16 or block-float
-// weights.
+// steps, small batches), outputs of few tiles, block-float weights, and fp32.
 //
 // A workgroup owns one BM x BN output block and its WK waves split K between
 // them (wave w takes k stages w, w + WK, ...), so that a small output still
@@ -24,6 +23,7 @@ static_assert(TTLH_MATMUL_SCRATCH_BYTES >= kArrivedBytes + 256 * 32 * 128 * 4, "
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x4 u32x4a8 __attribute__((aligned(8)));  // packed tiles may be 8-byte aligned
 
@@ -483,6 +483,126 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_bq_kernel(const Direct
 }
 
 // ---------------------------------------------------------------------------
+// fp32.  A wave owns 32 MT x 32 NT outputs and runs v_mfma_f32_32x32x2f32,
+// whose operands are one element a lane (row / column lane % 32, k lane / 32):
+// the k order inside a group of eight is free, so MFMA s of the group takes
+// k = 4 (lane / 32) + s and a lane's A elements are one 16-byte load; B needs
+// no transpose, the lane loads NT adjacent columns of a k row.
+template <int MT, int NT>
+struct FStage {
+  f32x4 a[2][MT];       // two groups of eight k
+  float b[2][4][NT];
+};
+
+template <int MT, int NT, int WM, int WN, int WK, int OCC>
+__global__ __launch_bounds__(64 * WM * WN * WK, OCC) void mm_direct_f32_kernel(const DirectArgs p) {
+  constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, PITCH = BN + 4, D = 2;
+  constexpr int kWaves = WM * WN * WK;
+  __shared__ __attribute__((aligned(16))) float part[WK * BM * PITCH];
+  int bm, bn, split;
+  direct_block(p, bm, bn, split);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
+  const int l32 = lane & 31, h = lane >> 5;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const float* A = static_cast<const float*>(p.A) + static_cast<int64_t>(m0) * p.lda;
+  const float* B = static_cast<const float*>(p.B);
+  uint32_t a_off[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    a_off[i] = 4 * (static_cast<uint32_t>(min(32 * (wm * MT + i) + l32, p.M - 1 - m0)) *
+                        static_cast<uint32_t>(p.lda) + 4 * h);
+  const uint32_t b_off = 4 * (static_cast<uint32_t>(4 * h) * static_cast<uint32_t>(p.ldb) +
+                              min(n0 + 32 * NT * wn + NT * l32, p.N - NT));
+
+  f32x16 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  const int stages = p.K / 16, first = split * WK + wk, step = p.splits * WK;
+  typedef FStage<MT, NT> Stage;
+  auto load = [&](Stage& s, int i) {  // stage of 16 k
+    const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 16;
+    const uint32_t bo = opaque(b_off);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const float* bk = B + (k0 + 8 * g) * p.ldb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float* src = bk + static_cast<int64_t>(j) * p.ldb;
+        if constexpr (NT == 2) {
+          const f32x2 v = gload<f32x2>(src, bo);
+          s.b[g][j][0] = v[0];
+          s.b[g][j][1] = v[1];
+        } else {
+          s.b[g][j][0] = gload<float>(src, bo);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) s.a[g][m] = gload<f32x4>(A + k0 + 8 * g, opaque(a_off[m]));
+    }
+  };
+  auto compute = [&](const Stage& s) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int c = 0; c < NT; ++c)
+            acc[m][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[g][m][j], s.b[g][j][c], acc[m][c],
+                                                             0, 0, 0);
+  };
+
+  const int n = stages > first ? (stages - first + step - 1) / step : 0;
+  Stage st[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    load(st[d], d);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int i = 0;
+  for (; i + 2 * D <= n; i += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      compute(st[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      load(st[d], i + D + d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    if (i + d < n) compute(st[d]);
+    if (i + D + d < n) load(st[d], i + D + d);
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (i + D + d < n) compute(st[d]);
+
+  // lane holds of MFMA (m, c): column NT l32 + c, rows 8 (r / 4) + 4 h + r % 4
+  float* d = part + wk * BM * PITCH + (32 * MT * wm + 4 * h) * PITCH + 32 * NT * wn + NT * l32;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float* dst = d + (32 * m + 8 * (r >> 2) + (r & 3)) * PITCH;
+      if constexpr (NT == 2)
+        *reinterpret_cast<f32x2*>(dst) = f32x2{acc[m][0][r], acc[m][1][r]};
+      else
+        *dst = acc[m][0][r];
+    }
+  __syncthreads();
+  reduce_store<BM, BN, PITCH, WK, 64 * kWaves>(p, part, bm, bn, split);
+}
+
+// ---------------------------------------------------------------------------
 // Choice of the kernel.
 
 // Parts of K for `blocks` output blocks of which the chip holds 256 at once
@@ -599,6 +719,33 @@ bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, i
   set_blocks(a, 32, 64, k_parts(blocks_of(a, 32, 64), a.K, 1024, scratch, s), scratch);
   if (bits == 8) TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>), 8, "mm_direct_bq_kernel");
   else TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>), 8, "mm_direct_bq_kernel");
+  return true;
+}
+
+bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status) {
+  // 16-byte loads of A, 8-byte loads of B
+  if ((reinterpret_cast<uintptr_t>(a.A) & 15) || a.lda % 4 || (reinterpret_cast<uintptr_t>(a.B) & 7) ||
+      a.ldb % 2 || !offsets_fit(a, 4))
+    return false;
+  set_c_vec(a);
+  // 128x128 blocks where they fill whole rounds of the CUs: 2048^3 126 us
+  // against 142 to 145 in smaller blocks, but 1504^3 (144 blocks) 93 against
+  // 68.  Few outputs go in 32x32 blocks with K over eight (and more) waves:
+  // 256 x 2048 x 256 8.3 us, 12.9 without the parts.
+  const int64_t big = blocks_of(a, 128, 128), small = blocks_of(a, 32, 32);
+  if (4 * big >= 3 * 256 * ((big + 255) / 256)) {
+    set_blocks(a, 128, 128, 1, nullptr);
+    TTLH_DIRECT((mm_direct_f32_kernel<2, 2, 2, 2, 2, 2>), 8, "mm_direct_f32_kernel");
+  } else if (small <= 128) {
+    set_blocks(a, 32, 32, k_parts(small, a.K, 256, scratch, s), scratch);
+    TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4>), 8, "mm_direct_f32_kernel");
+  } else if (small <= 512) {
+    set_blocks(a, 32, 32, 1, nullptr);
+    TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 4, 4>), 4, "mm_direct_f32_kernel");
+  } else {
+    set_blocks(a, 32, 64, 1, nullptr);
+    TTLH_DIRECT((mm_direct_f32_kernel<1, 2, 1, 1, 8, 3>), 8, "mm_direct_f32_kernel");
+  }
   return true;
 }
 

@@ -7,8 +7,8 @@
 namespace ttlh {
 
 struct DirectArgs {
-  const void* A;  // bf16, row-major
-  const void* B;  // bf16 row-major [K, N], or the packed block-float tiles
+  const void* A;  // bf16 or f32, row-major
+  const void* B;  // bf16 or f32 row-major [K, N], or the packed block-float tiles
   void* C;
   int64_t lda, ldb, ldc;
   int32_t M, N, K;
@@ -24,6 +24,7 @@ struct DirectArgs {
 // where the caller's other kernels take the problem.  `scratch`: null, or
 // TTLH_MATMUL_SCRATCH_BYTES of device memory (see ttlh_matmul_scratch).
 bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status);
+bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status);
 bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status);
 
 }  // namespace ttlh
