@@ -11,7 +11,9 @@ missing GPU raises.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
+import struct
 from pathlib import Path
 
 import torch  # noqa: F401  (must precede the library load, see module docstring)
@@ -84,30 +86,49 @@ class RowReduce(C.Structure):
     ]
 
 
-# every symbol include/ttlhip.h declares, with its ctypes signature
+# The structs' layouts for struct.pack, which builds a launch's argument arrays
+# in a microsecond where one ctypes object per step takes about one each.
+INSTR_FMT, OPERAND_FMT, ROW_REDUCE_FMT = "3Bxff", "Qii6q", "QQiiQifQiiq"
+assert struct.calcsize("=" + INSTR_FMT) == C.sizeof(Instr)
+assert struct.calcsize("=" + OPERAND_FMT) == C.sizeof(Operand)
+assert struct.calcsize("=" + ROW_REDUCE_FMT) == C.sizeof(RowReduce)
+
+
+@functools.lru_cache(maxsize=128)
+def array_struct(fmt: str, n: int) -> struct.Struct:
+    return struct.Struct("=" + fmt * n)
+
+
+def f32(v: float) -> float:
+    """v as a C float holds it: beyond the range infinite, not an error."""
+    return C.c_float(v).value
+
+
+# every symbol include/ttlhip.h declares, with its ctypes signature (arrays of
+# Instr, Operand and RowReduce as plain pointers: ctypes arrays or packed bytes)
 _i64, _vp, _int = C.c_int64, C.c_void_p, C.c_int
 SIGNATURES = {
-    "ttlh_eltwise": (_int, [C.POINTER(Instr), C.POINTER(Operand), _int, _vp, _int, _i64, _i64,
+    "ttlh_eltwise": (_int, [_vp, _vp, _int, _vp, _int, _i64, _i64,
                             _i64, _i64, _i64, _vp]),
     "ttlh_tilize": (_int, [_vp, _i64, _vp, _i64, _i64, _int, _vp]),
     "ttlh_untilize": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "ttlh_transpose_bf16": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "ttlh_reduce_workspace_bytes": (_i64, [_int, _i64, _i64]),
-    "ttlh_reduce": (_int, [C.POINTER(Instr), C.POINTER(Operand), _int, _int, _int, _vp, _int,
+    "ttlh_reduce": (_int, [_vp, _vp, _int, _int, _int, _vp, _int,
                            C.c_float, _vp, _int, _i64, _int, _i64, _i64, _i64, _i64, _vp, _i64,
                            _vp]),
-    "ttlh_reduce_noalloc": (_int, [C.POINTER(Instr), C.POINTER(Operand), _int, _int, _int, _vp,
+    "ttlh_reduce_noalloc": (_int, [_vp, _vp, _int, _int, _int, _vp,
                                    _int, C.c_float, _vp, _int, _i64, _int, _i64, _i64, _i64, _i64,
                                    _vp]),
-    "ttlh_reduce_rows_eltwise": (_int, [C.POINTER(RowReduce), _int, C.POINTER(Instr),
-                                        C.POINTER(Operand), _int, _vp, _int, _i64, _i64, _i64,
+    "ttlh_reduce_rows_eltwise": (_int, [_vp, _int, _vp,
+                                        _vp, _int, _vp, _int, _i64, _i64, _i64,
                                         _i64, _i64, _vp]),
     "ttlh_matmul": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64, _i64,
                            _int, _vp]),
     "ttlh_matmul_scratch": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64,
                                    _i64, _int, _vp, _i64, _vp]),
-    "ttlh_matmul_eltwise": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, C.POINTER(Instr),
-                                   C.POINTER(Operand), _int, _int, _vp, _int, _i64, _i64, _i64,
+    "ttlh_matmul_eltwise": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp,
+                                   _vp, _int, _int, _vp, _int, _i64, _i64, _i64,
                                    _vp]),
     "ttlh_bfp8_pack_host": (_int, [_vp, _vp, _i64, _i64]),
     "ttlh_bfp8_unpack_host": (_int, [_vp, _vp, _i64, _i64]),
@@ -164,25 +185,47 @@ def check(fn: str, status: int) -> None:
 
 def call(fn: str, *args) -> None:
     """Calls entry point `fn` and raises on a non-zero status."""
-    check(fn, getattr(load(), fn)(*args))
+    status = getattr(_lib or load(), fn)(*args)
+    if status != TTLH_OK:
+        check(fn, status)
+
+
+_device_seen = False
 
 
 def require_device() -> None:
-    if not torch.cuda.is_available():
-        raise RuntimeError(
-            "tt-lang_amd executes on an AMD GPU (MI355X, gfx950); no HIP device is visible "
-            "and there is no CPU fallback"
-        )
+    global _device_seen
+    if not _device_seen:
+        if not torch.cuda.is_available():
+            raise RuntimeError(
+                "tt-lang_amd executes on an AMD GPU (MI355X, gfx950); no HIP device is visible "
+                "and there is no CPU fallback"
+            )
+        _device_seen = True
 
 
 def stream_ptr(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    if stream is not None:
+        return int(stream.cuda_stream)
+    if not torch.cuda.is_initialized():
+        return int(torch.cuda.current_stream().cuda_stream)
+    # the current stream of the current device, without building a Stream object
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def synchronize() -> None:
+    """torch.cuda.synchronize() without its device-guard bookkeeping (10 us)."""
+    if torch.cuda.is_initialized():
+        torch._C._cuda_synchronize()
+    else:
+        torch.cuda.synchronize()
+
+
+_DTYPE_CODES = {torch.bfloat16: TTLH_BF16, torch.float32: TTLH_F32}
 
 
 def dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.bfloat16:
-        return TTLH_BF16
-    if dt == torch.float32:
-        return TTLH_F32
-    raise TypeError(f"tt-lang_amd kernels take bfloat16 or float32 tensors, got {dt}")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise TypeError(f"tt-lang_amd kernels take bfloat16 or float32 tensors, got {dt}")
+    return code

@@ -10,6 +10,7 @@ torch.cuda.synchronize() themselves.
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -118,22 +119,114 @@ def _axis_range(lo: int, n: int, mask: int, off: int):
     return vals_lo + off, vals_hi + off
 
 
-def _operand_struct(m: OperandMap, y0: int, x0: int, h: int, w: int) -> L.Operand:
+_READS = (L.FORM_LOAD, L.FORM_PUSH, L.FORM_BIN, L.FORM_BIN_REV)  # steps with an operand
+_NO_OPERAND = (0,) * 9
+_OPERAND_BYTES = struct.calcsize("=" + L.OPERAND_FMT)
+
+
+def _operand_fields(m: OperandMap, y0: int, x0: int, h: int, w: int) -> tuple:
+    """The ttlh_operand of `m`, every address checked against the tensor."""
     t = m.tensor
-    _check_device(t, "eltwise operand")
+    if not t.is_cuda or t.dim() != 2:
+        _check_device(t, "eltwise operand")
     rows, cols = t.shape
-    rs = t.stride(0) if rows > 1 else 0
-    cs = t.stride(1) if cols > 1 else 0
+    rs, cs = t.stride()
     if rows > 1:
         r = _axis_range(y0, h, m.row_mask, m.row_off)
         if r and (r[0] < 0 or r[1] >= rows):
             raise ValueError(f"eltwise operand rows {r} out of range for shape {tuple(t.shape)}")
+    else:
+        rs = 0
     if cols > 1:
         r = _axis_range(x0, w, m.col_mask, m.col_off)
         if r and (r[0] < 0 or r[1] >= cols):
             raise ValueError(f"eltwise operand cols {r} out of range for shape {tuple(t.shape)}")
-    return L.Operand(t.data_ptr(), L.dtype_code(t.dtype), 0, rs, cs, m.row_mask, m.col_mask,
-                     m.row_off, m.col_off)
+    else:
+        cs = 0
+    return (t.data_ptr(), L.dtype_code(t.dtype), 0, rs, cs, m.row_mask, m.col_mask, m.row_off,
+            m.col_off)
+
+
+def _pack(fmt: str, n: int, values: list, floats: Sequence[int]) -> bytes:
+    """n structs of `fmt` from their fields; `floats`: the float fields'
+    positions in one struct."""
+    try:
+        return L.array_struct(fmt, n).pack(*values)
+    except OverflowError:  # a Python float beyond fp32
+        per = len(values) // n
+        for k in range(n):
+            for i in floats:
+                values[k * per + i] = L.f32(values[k * per + i])
+        return L.array_struct(fmt, n).pack(*values)
+
+
+def _program_bytes(prog: StackProgram, operands: Sequence[Optional[OperandMap]], region,
+                   skip: int = -1):
+    """(ttlh_instr array, ttlh_operand array, n) of a program; the operand of
+    step `skip` is left empty."""
+    steps = prog.steps
+    n = len(steps)
+    if len(operands) != n:
+        raise ValueError(f"{n} steps but {len(operands)} operand slots")
+    y0, x0, h, w = region
+    pv: list = []
+    ov: list = []
+    for k, s in enumerate(steps):
+        form = s.form
+        pv += (s.op, form, s.rnd, s.imm, s.imm2)
+        if form in _READS and k != skip:
+            m = operands[k]
+            if m is None:
+                raise ValueError(f"step {k} needs an operand")
+            ov += _operand_fields(m, y0, x0, h, w)
+        else:
+            ov += _NO_OPERAND
+    return (_pack(L.INSTR_FMT, n, pv, (3, 4)), L.array_struct(L.OPERAND_FMT, n).pack(*ov), n)
+
+
+def _check_eltwise_out(out: torch.Tensor, region) -> None:
+    _check_device(out, "eltwise output")
+    if out.stride(1) != 1:
+        raise ValueError("eltwise output must have unit column stride")
+    y0, x0, h, w = region
+    if y0 < 0 or x0 < 0 or y0 + h > out.shape[0] or x0 + w > out.shape[1]:
+        raise ValueError(f"region {(y0, x0, h, w)} outside output {tuple(out.shape)}")
+
+
+_PTR = struct.Struct("=Q")
+
+
+class BoundProgram:
+    """A program's argument bytes for operands of one geometry, checked once
+    when built; `index[k]` is the number of step k's operand in the tensor list
+    that later calls give pointers of."""
+
+    def __init__(self, prog: StackProgram, operands: Sequence[Optional[OperandMap]], region,
+                 index: Sequence[Optional[int]]):
+        self.instrs, self.ops, self.n = _program_bytes(prog, operands, region)
+        self.slots = [(k * _OPERAND_BYTES, index[k]) for k, s in enumerate(prog.steps)
+                      if s.form in _READS]
+
+    def operands(self, ptrs: Sequence[int]) -> bytes:
+        b = bytearray(self.ops)
+        for at, i in self.slots:
+            _PTR.pack_into(b, at, ptrs[i])
+        return bytes(b)
+
+
+class BoundEltwise:
+    """eltwise(prog, operands, out, region) for later calls on tensors of the
+    same geometry: launch(pointers, stream pointer)."""
+
+    def __init__(self, prog, operands, out: torch.Tensor, region, index, out_index: int):
+        _check_eltwise_out(out, region)
+        self.program = BoundProgram(prog, operands, region, index)
+        self.out_index = out_index
+        self.tail = (L.dtype_code(out.dtype), out.stride(0), *region)
+
+    def launch(self, ptrs: Sequence[int], sp: int) -> None:
+        p = self.program
+        L.call("ttlh_eltwise", p.instrs, p.operands(ptrs), p.n, ptrs[self.out_index], *self.tail, sp)
 
 
 def eltwise(prog: StackProgram, operands: Sequence[Optional[OperandMap]], out: torch.Tensor,
@@ -142,23 +235,12 @@ def eltwise(prog: StackProgram, operands: Sequence[Optional[OperandMap]], out: t
 
     operands[k] is the operand of step k (None for steps without one).
     """
-    _check_device(out, "eltwise output")
-    if out.stride(1) != 1:
-        raise ValueError("eltwise output must have unit column stride")
-    n = len(prog.steps)
-    if len(operands) != n:
-        raise ValueError(f"{n} steps but {len(operands)} operand slots")
-    y0, x0, h, w = region if region is not None else (0, 0, out.shape[0], out.shape[1])
-    if y0 < 0 or x0 < 0 or y0 + h > out.shape[0] or x0 + w > out.shape[1]:
-        raise ValueError(f"region {(y0, x0, h, w)} outside output {tuple(out.shape)}")
-    instrs = (L.Instr * n)()
-    ops = (L.Operand * n)()
-    for k, (s, m) in enumerate(zip(prog.steps, operands)):
-        instrs[k] = L.Instr(s.op, s.form, s.rnd, 0, s.imm, s.imm2)
-        if s.form in (L.FORM_LOAD, L.FORM_PUSH, L.FORM_BIN, L.FORM_BIN_REV):
-            if m is None:
-                raise ValueError(f"step {k} needs an operand")
-            ops[k] = _operand_struct(m, y0, x0, h, w)
+    if region is None:
+        _check_device(out, "eltwise output")
+        region = (0, 0, out.shape[0], out.shape[1])
+    _check_eltwise_out(out, region)
+    y0, x0, h, w = region
+    instrs, ops, n = _program_bytes(prog, operands, region)
     L.call("ttlh_eltwise", instrs, ops, n, out.data_ptr(), L.dtype_code(out.dtype),
            out.stride(0), y0, x0, h, w, L.stream_ptr(stream))
 
@@ -185,9 +267,6 @@ def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: s
     if not dset or not dset <= {0, 1}:
         raise ValueError(f"reduce dims must be a non-empty subset of [0, 1], got {list(dims)}")
     dbits = (L.REDUCE_DIM0 if 0 in dset else 0) | (L.REDUCE_DIM1 if 1 in dset else 0)
-    n = len(prog.steps)
-    if len(operands) != n:
-        raise ValueError(f"{n} steps but {len(operands)} operand slots")
     y0, x0, h, w = region
     if h <= 0 or w <= 0 or y0 < 0 or x0 < 0:
         raise ValueError(f"bad reduce region {tuple(region)}")
@@ -198,14 +277,7 @@ def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: s
     if oy < 0 or ox < 0 or oy + rows > out.shape[0] or ox + cols > out.shape[1]:
         raise ValueError(f"reduce result ({rows}x{cols} at {(oy, ox)}) outside output "
                          f"{tuple(out.shape)}")
-    instrs = (L.Instr * n)()
-    ops = (L.Operand * n)()
-    for k, (s, m) in enumerate(zip(prog.steps, operands)):
-        instrs[k] = L.Instr(s.op, s.form, s.rnd, 0, s.imm, s.imm2)
-        if s.form in (L.FORM_LOAD, L.FORM_PUSH, L.FORM_BIN, L.FORM_BIN_REV):
-            if m is None:
-                raise ValueError(f"step {k} needs an operand")
-            ops[k] = _operand_struct(m, y0, x0, h, w)
+    instrs, ops, n = _program_bytes(prog, operands, region)
     sp, sdt = 0, 0
     if scaler is not None:
         if not scaler.is_cuda or scaler.numel() < 1:
@@ -226,22 +298,6 @@ def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: s
            L.stream_ptr(stream))
 
 
-def _program_structs(prog: StackProgram, operands: Sequence[Optional[OperandMap]], region):
-    y0, x0, h, w = region
-    n = len(prog.steps)
-    if len(operands) != n:
-        raise ValueError(f"{n} steps but {len(operands)} operand slots")
-    instrs = (L.Instr * n)()
-    ops = (L.Operand * n)()
-    for k, (s, m) in enumerate(zip(prog.steps, operands)):
-        instrs[k] = L.Instr(s.op, s.form, s.rnd, 0, s.imm, s.imm2)
-        if s.form in (L.FORM_LOAD, L.FORM_PUSH, L.FORM_BIN, L.FORM_BIN_REV):
-            if m is None:
-                raise ValueError(f"step {k} needs an operand")
-            ops[k] = _operand_struct(m, y0, x0, h, w)
-    return instrs, ops, n
-
-
 @dataclass
 class RowReduce:
     """One row reduction of reduce_rows_eltwise(): the arguments of a
@@ -258,6 +314,74 @@ class RowReduce:
     scale: float = 1.0
 
 
+class BoundRows:
+    """reduce_rows_eltwise(reds, prog, operands, out, region) for later calls
+    on tensors of the same geometry: launch(pointers, stream pointer).
+    `red_index[j]` = (operand numbers, result number, scaler number or None,
+    the scaler's byte offset in that tensor) of reduction j in the tensor list,
+    `index` / `out_index` the program's."""
+
+    def __init__(self, reds: Sequence[RowReduce], prog, operands, out: torch.Tensor, region,
+                 red_index, index, out_index: int):
+        y0, x0, h, w = region
+        if h <= 0 or w <= 0 or y0 < 0 or x0 < 0:
+            raise ValueError(f"bad region {tuple(region)}")
+        _check_eltwise_out(out, region)
+        self.heads = []      # per reduction: fields that no pointer changes
+        self.programs = []
+        for r, (ri, ro, rs, rs_at) in zip(reds, red_index):
+            _check_device(r.out, "reduce output")
+            if r.out.stride(1) != 1:
+                raise ValueError("reduce output must have unit column stride")
+            if r.kind not in ("sum", "max"):
+                raise ValueError(f"reduce kind must be 'sum' or 'max', got {r.kind!r}")
+            oy, ox = r.out_origin
+            cols = 32 if r.out_pad else 1
+            if oy < 0 or ox < 0 or oy + h > r.out.shape[0] or ox + cols > r.out.shape[1]:
+                raise ValueError(f"reduce result ({h}x{cols} at {(oy, ox)}) outside output "
+                                 f"{tuple(r.out.shape)}")
+            sdt = 0
+            if r.scaler is not None:
+                if not r.scaler.is_cuda or r.scaler.numel() < 1:
+                    raise ValueError("reduce scaler must be a non-empty device tensor")
+                sdt = L.dtype_code(r.scaler.dtype)
+            p = BoundProgram(r.prog, r.operands, region, ri)
+            ld = r.out.stride(0)
+            at = (oy * ld + ox) * r.out.element_size()
+            self.programs.append(p)
+            self.heads.append((p.n, L.REDUCE_SUM if r.kind == "sum" else L.REDUCE_MAX, rs, rs_at, sdt,
+                               L.f32(r.scale), ro, at, L.dtype_code(r.out.dtype),
+                               int(bool(r.out_pad)), ld))
+        self.program = BoundProgram(prog, operands, region, index)
+        self.out_index = out_index
+        self.tail = (L.dtype_code(out.dtype), out.stride(0), *region)
+        # the reductions' instructions: one buffer that never changes
+        blob = b"".join([p.instrs for p in self.programs] + [bytes(4)])
+        self.instrs = (C.c_char * len(blob)).from_buffer_copy(blob)
+
+    def launch(self, ptrs: Sequence[int], sp: int) -> bool:
+        """False, having launched nothing, where the library refuses the
+        combination."""
+        blob = b"".join([p.operands(ptrs) for p in self.programs] + [bytes(8)])
+        ops = (C.c_char * len(blob)).from_buffer_copy(blob)  # alive until the call returns
+        prog_at, in_at = C.addressof(self.instrs), C.addressof(ops)
+        values: list = []
+        for p, (n, kind, rs, rs_at, sdt, scale, ro, at, odt, pad, ld) in zip(self.programs,
+                                                                              self.heads):
+            values += (prog_at, in_at, n, kind, 0 if rs is None else ptrs[rs] + rs_at, sdt, scale,
+                       ptrs[ro] + at, odt, pad, ld)
+            prog_at += len(p.instrs)
+            in_at += len(p.ops)
+        p, n_red = self.program, len(self.heads)
+        st = L.load().ttlh_reduce_rows_eltwise(
+            L.array_struct(L.ROW_REDUCE_FMT, n_red).pack(*values), n_red, p.instrs,
+            p.operands(ptrs), p.n, ptrs[self.out_index], *self.tail, sp)
+        if st == L.TTLH_EUNSUPPORTED:
+            return False
+        L.check("ttlh_reduce_rows_eltwise", st)
+        return True
+
+
 def reduce_rows_eltwise(reds: Sequence[RowReduce], prog: StackProgram,
                         operands: Sequence[Optional[OperandMap]], out: torch.Tensor, region,
                         stream=None) -> bool:
@@ -268,46 +392,20 @@ def reduce_rows_eltwise(reds: Sequence[RowReduce], prog: StackProgram,
     own row from registers.  Returns False, having launched nothing, where
     the library refuses the combination (TTLH_EUNSUPPORTED); the caller then
     makes the separate calls."""
-    y0, x0, h, w = region
-    if h <= 0 or w <= 0 or y0 < 0 or x0 < 0:
-        raise ValueError(f"bad region {tuple(region)}")
-    _check_device(out, "eltwise output")
-    if out.stride(1) != 1:
-        raise ValueError("eltwise output must have unit column stride")
-    if y0 + h > out.shape[0] or x0 + w > out.shape[1]:
-        raise ValueError(f"region {tuple(region)} outside output {tuple(out.shape)}")
-    keep = []  # ctypes arrays the structs point into, alive until the call returns
-    rr = (L.RowReduce * len(reds))()
-    for j, r in enumerate(reds):
-        _check_device(r.out, "reduce output")
-        if r.out.stride(1) != 1:
-            raise ValueError("reduce output must have unit column stride")
-        if r.kind not in ("sum", "max"):
-            raise ValueError(f"reduce kind must be 'sum' or 'max', got {r.kind!r}")
-        oy, ox = r.out_origin
-        cols = 32 if r.out_pad else 1
-        if oy < 0 or ox < 0 or oy + h > r.out.shape[0] or ox + cols > r.out.shape[1]:
-            raise ValueError(f"reduce result ({h}x{cols} at {(oy, ox)}) outside output "
-                             f"{tuple(r.out.shape)}")
-        instrs, ops, n = _program_structs(r.prog, r.operands, region)
-        keep += [instrs, ops]
-        sp, sdt = 0, 0
-        if r.scaler is not None:
-            if not r.scaler.is_cuda or r.scaler.numel() < 1:
-                raise ValueError("reduce scaler must be a non-empty device tensor")
-            sp, sdt = r.scaler.data_ptr(), L.dtype_code(r.scaler.dtype)
-        optr = r.out.data_ptr() + (oy * r.out.stride(0) + ox) * r.out.element_size()
-        rr[j] = L.RowReduce(instrs, ops, n, L.REDUCE_SUM if r.kind == "sum" else L.REDUCE_MAX,
-                            sp, sdt, float(r.scale), optr, L.dtype_code(r.out.dtype),
-                            int(bool(r.out_pad)), r.out.stride(0))
-    instrs, ops, n = _program_structs(prog, operands, region)
-    st = L.load().ttlh_reduce_rows_eltwise(rr, len(reds), instrs, ops, n, out.data_ptr(),
-                                           L.dtype_code(out.dtype), out.stride(0), y0, x0, h, w,
-                                           L.stream_ptr(stream))
-    if st == L.TTLH_EUNSUPPORTED:
-        return False
-    L.check("ttlh_reduce_rows_eltwise", st)
-    return True
+    tensors: List[torch.Tensor] = []
+
+    def number(t) -> Optional[int]:
+        if t is None:
+            return None
+        tensors.append(t)
+        return len(tensors) - 1
+
+    def numbers(maps):
+        return [None if m is None else number(m.tensor) for m in maps]
+
+    red_index = [(numbers(r.operands), number(r.out), number(r.scaler), 0) for r in reds]
+    bound = BoundRows(reds, prog, operands, out, region, red_index, numbers(operands), number(out))
+    return bound.launch([t.data_ptr() for t in tensors], L.stream_ptr(stream))
 
 
 def matmul(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, accumulate: bool = False,
@@ -397,15 +495,7 @@ def matmul_eltwise(a: torch.Tensor, b: torch.Tensor, prog: StackProgram,
     if K2 != K or (h, w) != (M, N) or y0 + h > out.shape[0] or x0 + w > out.shape[1]:
         raise ValueError(f"matmul_eltwise shapes {tuple(a.shape)} @ {tuple(b.shape)} -> region "
                          f"{tuple(region)} of {tuple(out.shape)}")
-    n = len(prog.steps)
-    instrs = (L.Instr * n)()
-    ops = (L.Operand * n)()
-    for k, (s, m) in enumerate(zip(prog.steps, operands)):
-        instrs[k] = L.Instr(s.op, s.form, s.rnd, 0, s.imm, s.imm2)
-        if k != prod_step and s.form in (L.FORM_LOAD, L.FORM_PUSH, L.FORM_BIN, L.FORM_BIN_REV):
-            if m is None:
-                raise ValueError(f"step {k} needs an operand")
-            ops[k] = _operand_struct(m, y0, x0, h, w)
+    instrs, ops, n = _program_bytes(prog, operands, region, skip=prod_step)
     L.call("ttlh_matmul_eltwise", a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), M, N, K,
            instrs, ops, n, prod_step, out.data_ptr(), L.dtype_code(out.dtype), out.stride(0),
            y0, x0, L.stream_ptr(stream))

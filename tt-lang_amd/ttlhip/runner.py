@@ -21,6 +21,7 @@ import torch
 
 import ttnn
 
+from . import _lib as L
 from . import dsl
 from . import profile
 from . import plan as P
@@ -56,10 +57,10 @@ class KernelRunner:
     # -- cache key -----------------------------------------------------------
     @staticmethod
     def _key_of(v):
-        if hasattr(v, "_tensor") and isinstance(v._tensor, torch.Tensor):
-            return ("T", tuple(v.shape), str(v.dtype))
+        if isinstance(getattr(v, "_tensor", None), torch.Tensor):
+            return ("T", v.shape, v.dtype)
         if isinstance(v, torch.Tensor):
-            return ("t", tuple(v.shape), str(v.dtype))
+            return ("t", v.shape, v.dtype)
         try:
             hash(v)
             return ("v", v)
@@ -72,11 +73,13 @@ class KernelRunner:
         # k(a, a, out) and k(a, b, out) must not share a plan.
         first: Dict[int, Any] = {}
         alias = []
-        for p, v in list(enumerate(args)) + sorted(kwargs.items()):
+        for p, v in enumerate(args):
             alias.append(first.setdefault(id(v), p))
-        return (tuple(self._key_of(a) for a in args),
-                tuple(sorted((k, self._key_of(v)) for k, v in kwargs.items())),
-                tuple(alias))
+        for p, v in sorted(kwargs.items()):
+            alias.append(first.setdefault(id(v), p))
+        key = self._key_of
+        named = tuple([(k, key(v)) for k, v in sorted(kwargs.items())]) if kwargs else ()
+        return tuple([key(a) for a in args]), named, tuple(alias)
 
     @staticmethod
     def _check_layouts(args, kwargs) -> None:
@@ -251,5 +254,5 @@ class KernelRunner:
             return None
         P.execute(plan, amap)
         if self.sync:
-            torch.cuda.synchronize()
+            L.synchronize()
         return None
