@@ -836,11 +836,11 @@ class SdpaWorkload(PlanWorkload):
                        "drop-in")
 
     def kernel_name(self):
-        # the eight-wave kernel serves D = 128, non-causal, positive scale,
-        # S % 256 == 0; the ping-pong kernel the other multiples of 256
-        if self.D == 128 and self.S % 256 == 0:
+        # the eight-wave kernel serves D = 128, non-causal, S % 256 == 0 and
+        # more than 256 blocks of 128 queries
+        if self.D == 128 and self.S % 256 == 0 and self.B * self.H * self.S // 128 > 256:
             return "sdpa_w8_kernel"
-        return "sdpa_pp_kernel" if self.S % 256 == 0 else "sdpa_fwd_kernel"
+        return "sdpa_fwd_kernel"
 
     def work_per_step(self):
         return 4.0 * self.B * self.H * self.S * self.S * self.D

@@ -246,3 +246,32 @@ def test_sdpa_other_kernels_with_slow_loads(S, D, causal):
            D, 0.1, int(causal), L.stream_ptr())
     torch.cuda.synchronize()
     _check(out.cpu(), O.sdpa_ref(q, k, v, 0.1, causal))
+
+
+@pytest.mark.parametrize("B,H,S,D,causal", [(1, 2, 160, 128, True), (1, 2, 192, 64, False),
+                                            (1, 1, 1056, 128, True), (2, 16, 1024, 64, True),
+                                            (1, 32, 1120, 128, True), (1, 65, 544, 64, False),
+                                            (3, 24, 480, 128, True)])
+def test_sdpa_block_forms(B, H, S, D, causal):
+    # sdpa_fwd_kernel's forms (one and two groups of waves, whole and ragged
+    # sequences) and the causal block order: 3 to 33 KV blocks, so the groups'
+    # shares are equal and unequal, heads that an XCD's share divides and not
+    print(f"sdpa forms {B}x{H}x{S}x{D} causal={causal}", flush=True)
+    q, k, v = _qkv(B, H, S, D, 41)
+    _check(_run(q, k, v, 1.0 / math.sqrt(D), causal=causal),
+           O.sdpa_ref(q, k, v, 1.0 / math.sqrt(D), causal=causal))
+
+
+@pytest.mark.parametrize("S", [256, 2048])
+def test_sdpa_scores_of_minus_infinity(S):
+    # keys whose scores are -inf drop out, a whole KV block of them too
+    # (the first one, and in the second group's share)
+    g = torch.Generator().manual_seed(5)
+    q = torch.rand(1, 2, S, 128, generator=g).bfloat16() + 0.5  # positive
+    k, v = (torch.randn(1, 2, S, 128, generator=g).bfloat16() for _ in range(2))
+    k[:, :, :128, 3] = -float("inf")
+    k[:, :, 200:230, 3] = -float("inf")
+    got = _run(q, k, v, 0.09)
+    keep = torch.isfinite(k[0, 0, :, 3])
+    ref = O.sdpa_ref(q, k[:, :, keep], v[:, :, keep], 0.09)
+    _check(got, ref)

@@ -21,19 +21,25 @@
 // 4k + i / 4 addresses, so lanes addressing 4 kv rows x 16 d columns receive
 // 4 consecutive kv of one d column each.
 //
-// Three kernels share that per-wave math:
+// Two kernels share that per-wave math:
 //  * sdpa_w8_kernel (D = 128, non-causal, S a multiple of 256): 8 waves of
 //    32 queries, two per SIMD, each interleaving the MFMAs of a KV block with
 //    the softmax of the previous one, the second wave's VALU issuing under
 //    the first one's MFMAs; Q pre-scaled and the S accumulation started from
 //    -m, so the softmax is one exp2 per score; a persistent grid of one
 //    workgroup per CU (details at its definition);
-//  * sdpa_pp_kernel (other cases with S a multiple of 256): 8 waves, 256
-//    queries per workgroup, the two groups of four waves in ping-pong, one
-//    issuing the MFMAs of a block while the other runs the softmax of the
-//    previous one;
-//  * sdpa_fwd_kernel (S a multiple of 128): 4 waves, 128 queries, each wave
-//    running both parts in turn, two workgroups per CU.
+//  * sdpa_fwd_kernel (everything else): 128 queries per workgroup, K and V
+//    blocks of 64 rows, in two forms.  One group of four waves, two workgroups
+//    per CU, drifts apart so that one's softmax runs under the other's MFMAs;
+//    it is the faster one wherever the blocks fill the chip's 512 places.  With
+//    fewer, a CU would hold one group with nothing to hide its latencies, so
+//    two groups share the workgroup's queries, taking the even and the odd KV
+//    blocks, and their results meet in LDS: 1 x 8 x 4000 x 128 causal 107 ->
+//    76 us, 1 x 16 x 992 x 128 31 -> 24.  Either is bound by the latencies of
+//    its chain S -> softmax -> O (40% of the MFMA time of a block is waiting).
+//    A third kernel, which ran the two groups in ping-pong over 256 queries, was
+//    slower than these in every case it took (1 x 32 x 2048 x 128 causal 71 us
+//    against 58, 4 x 32 x 4096 x 64 682 against 646).
 //
 // K and V are staged in LDS as loaded (row-major, 16-byte stores).  gfx950's
 // LDS serves 256 bytes (64 banks) per cycle: a ds_read_b128 is conflict-free
@@ -42,8 +48,8 @@
 // D + 32 elements (V: 4 rows x 4 chunks per 32 lanes of a transpose read)
 // meet that.  The next block's K and V are fetched into registers while the
 // current block computes.
-// Softmax runs in the log2 domain: exp2(fma(s, scale log2 e, -m)) in the
-// other two kernels, with the block max taken on the raw scores (sign of the
+// Softmax runs in the log2 domain: exp2(fma(s, scale log2 e, -m)) in
+// sdpa_fwd_kernel, with the block max taken on the raw scores (sign of the
 // scale handled by taking the min instead); the causal mask touches only the blocks
 // that straddle the diagonal.  P is rounded to bf16 for the MFMA; O is
 // divided by l at the end.  Workgroup ids are regrouped so the query blocks
@@ -77,6 +83,7 @@ struct SdpaArgs {
   int32_t S;
   int32_t nqb;        // query blocks per (b, h)
   int32_t nbh;        // B * H
+  int32_t heads_together;  // causal: heads whose blocks are dispatched longest first
   float scale_log2;   // scale * log2(e)
 };
 
@@ -115,7 +122,7 @@ constexpr int kVPitch = D + 32;  // V rows in LDS (elements)
 template <int D, bool RAGGED = false>
 __device__ __forceinline__ void load_rows(const uint16_t* X, int64_t base, int kv0, u32x4 (&r)[D / 32],
                                           int end = 0) {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x & (kThreads - 1);
   constexpr int kChunksPerRow = D / 8;
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) {
@@ -132,7 +139,7 @@ __device__ __forceinline__ void load_rows(const uint16_t* X, int64_t base, int k
 
 template <int D, int PITCH>
 __device__ __forceinline__ void store_rows(const u32x4 (&r)[D / 32], uint16_t* dst) {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x & (kThreads - 1);
   constexpr int kChunksPerRow = D / 8;
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) {
@@ -161,6 +168,22 @@ __device__ __forceinline__ void block_coords(const SdpaArgs& p, int& bh, int& qb
   }
   bh = id / p.nqb;
   qb = id - bh * p.nqb;
+}
+
+// Causal: block qb has qb + 1 units of work, and the workgroups are dispatched
+// in order as CUs fall free, so the longest go first: of `heads_together` heads
+// (as many as share an XCD's L2 with their K and V), all last blocks, then all
+// last but one, and so on.
+template <bool CAUSAL>
+__device__ __forceinline__ void ordered_block(const SdpaArgs& p, int& bh, int& qb) {
+  block_coords(p, bh, qb);
+  if constexpr (CAUSAL) {
+    const int id = bh * p.nqb + qb, span = p.heads_together * p.nqb;
+    const int g = id / span, r = id - g * span;
+    const int heads = min(p.heads_together, p.nbh - g * p.heads_together);
+    qb = p.nqb - 1 - r / heads;
+    bh = g * p.heads_together + r % heads;
+  }
 }
 
 template <int D, bool CAUSAL, bool RAGGED = false>
@@ -194,21 +217,32 @@ struct Sdpa {
     }
   }
 
-  __device__ __forceinline__ float expo(float v) const {
-    return __builtin_amdgcn_exp2f(__builtin_fmaf(v, sc, -m));
+  __device__ __forceinline__ float expo(float v, float mx) const {
+    return __builtin_amdgcn_exp2f(__builtin_fmaf(v, sc, -mx));
   }
 
-  // One KV block kb: the next block's K and V are fetched into registers
-  // while this one computes S, the softmax and O += V(kb)^T P^T from LDS
-  // buffer kb & 1, then stored into the other buffer (last read before the
-  // previous barrier).
-  __device__ __forceinline__ void step(int kb) {
-    const uint16_t* Kc = Ks[kb & 1];
-    const uint16_t* Vc = Vs[kb & 1];
-    if (kb + 1 < nkv) {
-      load_rows<D, RAGGED>(p.K, base, (kb + 1) * BKV, stk, p.S);
-      load_rows<D, RAGGED>(p.V, base, (kb + 1) * BKV, stv, p.S);
+  static constexpr float kLazy = 8.0f;
+
+  // One KV block kb = it * GROUPS + group, if there is one: the group's next
+  // block's K and V are fetched into registers while this one computes S, the
+  // softmax and O += V(kb)^T P^T from the group's LDS buffer it & 1, then
+  // stored into the other buffer (last read before the previous barrier).
+  template <int GROUPS>
+  __device__ __forceinline__ void step(int it, int group) {
+    const int kb = it * GROUPS + group, next = kb + GROUPS;
+    if (next < nkv) {
+      load_rows<D, RAGGED>(p.K, base, next * BKV, stk, p.S);
+      load_rows<D, RAGGED>(p.V, base, next * BKV, stv, p.S);
     }
+    if (kb < nkv) block(kb, Ks[it & 1], Vs[it & 1]);
+    if (next < nkv) {
+      store_rows<D, kKPitch<D>>(stk, Ks[(it + 1) & 1]);
+      store_rows<D, kVPitch<D>>(stv, Vs[(it + 1) & 1]);
+    }
+    __syncthreads();
+  }
+
+  __device__ __forceinline__ void block(int kb, const uint16_t* Kc, const uint16_t* Vc) {
     f32x16 cur[2];
     scores(Kc, cur);
 
@@ -227,53 +261,60 @@ struct Sdpa {
           if (masked(kv)) cur[t][r] = sc >= 0.0f ? -INFINITY : INFINITY;
         }
     }
-    // block extreme of the raw scores: max if the scale is positive, else min
-    float ex = cur[0][0];
+    // block extreme of the raw scores: max if the scale is positive, else
+    // min (four chains, so that no add or max waits for all before it)
+    float e4[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) e4[c] = cur[c >> 1][8 * (c & 1)];
     if (sc >= 0.0f) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) ex = fmaxf(ex, cur[t][r]);
-      ex = fmaxf(ex, __shfl_xor(ex, 32));
+        for (int r = 1; r < 8; ++r) e4[c] = fmaxf(e4[c], cur[c >> 1][8 * (c & 1) + r]);
+      e4[0] = xor32_max(fmaxf(fmaxf(e4[0], e4[1]), fmaxf(e4[2], e4[3])));
     } else {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) ex = fminf(ex, cur[t][r]);
-      ex = fminf(ex, __shfl_xor(ex, 32));
+        for (int r = 1; r < 8; ++r) e4[c] = fminf(e4[c], cur[c >> 1][8 * (c & 1) + r]);
+      e4[0] = xor32_min(fminf(fminf(e4[0], e4[1]), fminf(e4[2], e4[3])));
     }
-    const float m_new = fmaxf(m, ex * sc);
-    // rescale O only when some lane's running max moved
-    if (__any(m_new != m)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the first block
+    // The running max moves, and O is rescaled, only when a lane's block max
+    // exceeds it by more than 8 (log2 units): P <= 2^8 until then.
+    const float m_blk = e4[0] * sc;
+    if (__any(m_blk > m + kLazy)) {
+      const float m_new = fmaxf(m, m_blk);
+      const float alpha = m_new == m ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // 0 at first
       l *= alpha;
 #pragma unroll
       for (int j = 0; j < ND; ++j) o[j] *= alpha;
       m = m_new;
     }
-    float rs = 0.0f;
+    // (a lane that has seen only masked or -inf scores keeps m = -inf: its
+    // exponentials are 0)
+    const float mm = m == -INFINITY ? 0.0f : m;
+    float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (diag) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int kv = kb * BKV + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-          const float e = masked(kv) ? 0.0f : expo(cur[t][r]);
+          const float e = masked(kv) ? 0.0f : expo(cur[t][r], mm);
           cur[t][r] = e;
-          rs += e;
+          r4[r & 3] += e;
         }
     } else {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float e = expo(cur[t][r]);
+          const float e = expo(cur[t][r], mm);
           cur[t][r] = e;
-          rs += e;
+          r4[r & 3] += e;
         }
     }
-    rs += __shfl_xor(rs, 32);
-    l += rs;
+    l += xor32_add((r4[0] + r4[1]) + (r4[2] + r4[3]));
 
     // P^T operands: chunk c (16 kv) = tile c/2, accumulators 8(c%2) .. +8
     bf16x8 pb[4];
@@ -301,11 +342,6 @@ struct Sdpa {
                                                        0, 0, 0);
       }
     }
-    if (kb + 1 < nkv) {
-      store_rows<D, kKPitch<D>>(stk, Ks[(kb + 1) & 1]);
-      store_rows<D, kVPitch<D>>(stv, Vs[(kb + 1) & 1]);
-    }
-    __syncthreads();
   }
 };
 
@@ -313,15 +349,16 @@ struct Sdpa {
 // the sequence (S % 32 == 0 keeps each wave wholly in or out): they read a
 // clamped Q row, take part in the K / V staging and barriers, store nothing.
 // The last KV block reads rows past S as zeros and masks their scores.
-template <int D, bool CAUSAL, bool RAGGED = false>
-__global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(const SdpaArgs p) {
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[2][BKV * kKPitch<D>];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[2][BKV * kVPitch<D>];
-  Sdpa<D, CAUSAL, RAGGED> w{p, Ks, Vs};
+template <int D, bool CAUSAL, bool RAGGED, int GROUPS>
+__global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel(const SdpaArgs p) {
+  __shared__ __attribute__((aligned(16))) uint16_t Ks[GROUPS][2][BKV * kKPitch<D>];
+  __shared__ __attribute__((aligned(16))) uint16_t Vs[GROUPS][2][BKV * kVPitch<D>];
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  Sdpa<D, CAUSAL, RAGGED> w{p, Ks[group], Vs[group]};
   int bh;
-  block_coords(p, bh, w.qb);
+  ordered_block<CAUSAL>(p, bh, w.qb);
   w.lane = threadIdx.x & 63;
-  w.wave = threadIdx.x >> 6;
+  w.wave = (threadIdx.x >> 6) & 3;
   w.l32 = w.lane & 31;
   w.h = w.lane >> 5;
   w.base = static_cast<int64_t>(bh) * p.S * D;
@@ -337,9 +374,11 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(const SdpaArgs p)
   }
   const int qload = RAGGED ? min(w.q, p.S - 1) : w.q;  // a wave past S reads a valid row
 
-  // prologue: K(0), V(0) into LDS; Q^T into VGPRs
-  load_rows<D, RAGGED>(p.K, w.base, 0, w.stk, p.S);
-  load_rows<D, RAGGED>(p.V, w.base, 0, w.stv, p.S);
+  // prologue: the group's first K and V block into LDS; Q^T into VGPRs
+  if (group < w.nkv) {
+    load_rows<D, RAGGED>(p.K, w.base, group * BKV, w.stk, p.S);
+    load_rows<D, RAGGED>(p.V, w.base, group * BKV, w.stv, p.S);
+  }
 #pragma unroll
   for (int dc = 0; dc < D / 16; ++dc)
     w.qop[dc] = *reinterpret_cast<const bf16x8*>(p.Q + w.base + static_cast<int64_t>(qload) * D +
@@ -348,15 +387,45 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(const SdpaArgs p)
   for (int j = 0; j < D / 32; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) w.o[j][r] = 0.0f;
-  store_rows<D, kKPitch<D>>(w.stk, Ks[0]);
-  store_rows<D, kVPitch<D>>(w.stv, Vs[0]);
+  if (group < w.nkv) {
+    store_rows<D, kKPitch<D>>(w.stk, w.Ks[0]);
+    store_rows<D, kVPitch<D>>(w.stv, w.Vs[0]);
+  }
   // Q^T must have landed before the loop: otherwise the compiler, merging
   // the first iteration's state (Q loads in flight) with later ones, makes
   // every S MFMA of every block wait on the next block's K/V prefetch
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
 
-  for (int kb = 0; kb < w.nkv; ++kb) w.step(kb);
+  const int steps = (w.nkv + GROUPS - 1) / GROUPS;
+  for (int it = 0; it < steps; ++it) w.template step<GROUPS>(it, group);
+
+  if constexpr (GROUPS == 2) {
+    // Group 1 leaves its max, sum and O in LDS (every group is past its last
+    // read of K and V); group 0's wave w, which holds the same queries in the
+    // same lanes as wave w + 4, adds them.
+    float* part = reinterpret_cast<float*>(&Ks[0][0][0]) + (w.wave * (16 * (D / 32) + 2)) * 64 + w.lane;
+    static_assert(sizeof(Ks) >= 4 * 64 * (16 * (D / 32) + 2) * sizeof(float), "partial O fits K");
+    if (group == 1) {
+      part[0] = w.m;
+      part[64] = w.l;
+#pragma unroll
+      for (int j = 0; j < D / 32; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[(2 + 16 * j + r) * 64] = w.o[j][r];
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = part[0], mt = fmaxf(w.m, m1);
+    const float a0 = w.m == mt ? 1.0f : __builtin_amdgcn_exp2f(w.m - mt);
+    const float a1 = m1 == mt ? 1.0f : __builtin_amdgcn_exp2f(m1 - mt);
+    w.l = w.l * a0 + part[64] * a1;
+#pragma unroll
+    for (int j = 0; j < D / 32; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        w.o[j][r] = w.o[j][r] * a0 + part[(2 + 16 * j + r) * 64] * a1;
+  }
   if (RAGGED && w.q >= p.S) return;  // wave-uniform (S % 32 == 0); no barrier follows
 
   // O[q][d], d = 32j + 8u + 4h + i: four contiguous bf16 per (j, u)
@@ -373,340 +442,12 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(const SdpaArgs p)
     }
 }
 
-// ---------------------------------------------------------------------------
-// Ping-pong variant: 512 threads = two groups of four waves, 256 queries per
-// workgroup (wave w owns rows 32 w .. 32 w + 31; group g = w / 4).  Each wave
-// alternates two phases per KV block i:
-//   X(i): O^T += V(i-1)^T P(i-1)^T and S^T = K(i) Q^T  (32 MFMAs, no softmax)
-//   Y(i): softmax of S(i) -> P(i), running max / sum, O rescale (VALU only)
-// and group 1 runs one phase behind group 0, so on every SIMD (which holds one
-// wave of each group) one wave issues MFMAs while the other does the softmax:
-// the matrix core and the VALU overlap across waves.  A workgroup barrier
-// separates the phases.  LDS holds two stages; stage i = {K(i), V(i-1)} (the
-// operands of X(i)) in buffer i & 1.  Every wave loads its share of stage
-// i + 1 into registers one phase before writing it to LDS, right after the
-// last reader of that buffer has passed a barrier.
-constexpr int PP_BQ = 256;
-constexpr int PP_THREADS = 512;
-
 template <int N, typename F>
 __device__ __forceinline__ void sd_static_for(F&& f) {
   if constexpr (N > 0) {
     sd_static_for<N - 1>(f);
     f(std::integral_constant<int, N - 1>());
   }
-}
-
-
-template <int D>
-__device__ __forceinline__ void pp_load(const uint16_t* X, int64_t base, int kv0,
-                                        u32x4 (&r)[D / 64]) {
-  const int t = threadIdx.x;
-  constexpr int kChunksPerRow = D / 8;
-#pragma unroll
-  for (int i = 0; i < D / 64; ++i) {
-    const int c = t + i * PP_THREADS;
-    const int row = c / kChunksPerRow, dc = (c % kChunksPerRow) * 8;
-    r[i] = *reinterpret_cast<gu32x4*>(
-        reinterpret_cast<uintptr_t>(X + base + static_cast<int64_t>(kv0 + row) * D + dc));
-  }
-}
-
-template <int D, int PITCH>
-__device__ __forceinline__ void pp_store(const u32x4 (&r)[D / 64], uint16_t* dst) {
-  const int t = threadIdx.x;
-  constexpr int kChunksPerRow = D / 8;
-#pragma unroll
-  for (int i = 0; i < D / 64; ++i) {
-    const int c = t + i * PP_THREADS;
-    const int row = c / kChunksPerRow, dc = (c % kChunksPerRow) * 8;
-    *reinterpret_cast<u32x4*>(dst + row * PITCH + dc) = r[i];
-  }
-}
-
-// phase boundary: this wave's LDS accesses are complete, then a workgroup
-// barrier with no memory fence (global loads stay in flight); the empty asm
-// statements keep the compiler from moving memory accesses across it and the
-// scheduling barriers keep MFMAs and VALU work in their phase
-__device__ __forceinline__ void pp_boundary() {
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-template <int D, bool CAUSAL>
-struct SdpaPP {
-  static constexpr int ND = D / 32;
-  static constexpr int NDC = D / 16;
-
-  const SdpaArgs& p;
-  uint16_t (*Ks)[BKV * kKPitch<D>];
-  uint16_t (*Vs)[BKV * kVPitch<D>];
-  int64_t base;
-  int qb, wave, lane, l32, h, q, n;
-  float sc;
-  bf16x8 qop[NDC];
-  f32x16 o[ND];
-  f32x16 cur[2];
-  bf16x8 pb[4];
-  float m, l;
-  u32x4 stk[D / 64], stv[D / 64];
-
-  // stage j = {K(j) if j < n, V(j - 1) if j >= 1} into registers / into LDS
-  __device__ __forceinline__ void load_stage(int j) {
-    if (j < n) pp_load<D>(p.K, base, j * BKV, stk);
-    if (j >= 1 && j <= n) pp_load<D>(p.V, base, (j - 1) * BKV, stv);
-  }
-  __device__ __forceinline__ void write_stage(int j) {
-    if (j < n) pp_store<D, kKPitch<D>>(stk, Ks[j & 1]);
-    if (j >= 1 && j <= n) pp_store<D, kVPitch<D>>(stv, Vs[j & 1]);
-  }
-
-  // X(i): DO_O adds V(i-1)^T P(i-1)^T, DO_S computes S(i); operands from
-  // LDS buffer i & 1.  The MFMAs (S and O alternating when both run) form a
-  // software pipeline: the LDS fragments of MFMA m + kPipe are requested
-  // right after MFMA m issues, so LDS latency hides behind kPipe MFMAs; the
-  // scheduling barriers keep that order.
-  static constexpr int kPipe = 6;
-
-  template <bool DO_O, bool DO_S, int M>
-  __device__ __forceinline__ void x_frag(const uint16_t* Kc, const uint16_t* Vc, bf16x8& f) {
-    constexpr bool kIsO = DO_O && DO_S ? (M & 1) != 0 : DO_O;
-    constexpr int k = DO_O && DO_S ? (M >> 1) : M;
-    if constexpr (kIsO) {
-      constexpr int j = k >> 2, c = k & 3;
-      const int d0 = 32 * j + 16 * ((lane >> 4) & 1);
-      const i16x4 lo = read_v4<D>(Vc, 16 * c + 4 * h, d0, lane);
-      const i16x4 hi = read_v4<D>(Vc, 16 * c + 4 * h + 8, d0, lane);
-      const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      f = __builtin_bit_cast(bf16x8, w);
-    } else {
-      constexpr int t = k / NDC, dc = k % NDC;
-      f = *reinterpret_cast<const bf16x8*>(Kc + (32 * t + l32) * kKPitch<D> + dc * 16 + 8 * h);
-    }
-  }
-
-  template <bool DO_O, bool DO_S, int M>
-  __device__ __forceinline__ void x_mfma(const bf16x8& f) {
-    constexpr bool kIsO = DO_O && DO_S ? (M & 1) != 0 : DO_O;
-    constexpr int k = DO_O && DO_S ? (M >> 1) : M;
-    if constexpr (kIsO) {
-      constexpr int j = k >> 2, c = k & 3;
-      o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, pb[c], o[j], 0, 0, 0);
-    } else {
-      constexpr int t = k / NDC, dc = k % NDC;
-      cur[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, qop[dc], cur[t], 0, 0, 0);
-    }
-  }
-
-  template <bool DO_O, bool DO_S>
-  __device__ __forceinline__ void x_phase(int i) {
-    const uint16_t* Kc = Ks[i & 1];
-    const uint16_t* Vc = Vs[i & 1];
-    constexpr int T = (DO_S ? 2 * NDC : 0) + (DO_O ? 4 * ND : 0);
-    if constexpr (DO_S) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) cur[t][r] = 0.0f;
-    }
-    bf16x8 fr[T];
-    sd_static_for<(kPipe < T ? kPipe : T)>([&](auto mc) {
-      x_frag<DO_O, DO_S, decltype(mc)::value>(Kc, Vc, fr[decltype(mc)::value]);
-    });
-    __builtin_amdgcn_sched_barrier(0);
-    sd_static_for<T>([&](auto mc) {
-      constexpr int m = decltype(mc)::value;
-      x_mfma<DO_O, DO_S, m>(fr[m]);
-      if constexpr (m + kPipe < T) x_frag<DO_O, DO_S, m + kPipe>(Kc, Vc, fr[m + kPipe]);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  }
-
-  __device__ __forceinline__ float expo(float v) const {
-    return __builtin_amdgcn_exp2f(__builtin_fmaf(v, sc, -m));
-  }
-
-  // Y(i): online softmax of S(i) into P(i) (masking and extreme rules as in
-  // Sdpa::step).  The running max m moves lazily: only when a lane's block
-  // maximum exceeds it by more than kLazy (log2 units), so O and l are rarely
-  // rescaled; until then P = exp2(s - m) <= 2^kLazy, which fp32 O / l and the
-  // bf16 P operands hold without loss (the final O / l is unchanged by the
-  // choice of m).
-  static constexpr float kLazy = 8.0f;
-
-  __device__ __forceinline__ void y_phase(int kb) {
-    const bool diag = CAUSAL && kb * BKV + BKV - 1 > qb * PP_BQ + wave * 32;
-    // element (t, r) holds kv = kb*BKV + 4h + (32t + 8(r/4) + r%4): masked
-    // when that offset exceeds lim (compared against literal constants)
-    const int lim = q - kb * BKV - 4 * h;
-    if (diag) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (32 * t + 8 * (r >> 2) + (r & 3) > lim) cur[t][r] = sc >= 0.0f ? -INFINITY : INFINITY;
-    }
-    // block extreme as a 4-way tree (short dependency chains)
-    float ex;
-    if (sc >= 0.0f) {
-      float p4[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = u >> 1, r0 = 8 * (u & 1);
-        p4[u] = fmaxf(fmaxf(fmaxf(cur[t][r0], cur[t][r0 + 1]), fmaxf(cur[t][r0 + 2], cur[t][r0 + 3])),
-                      fmaxf(fmaxf(cur[t][r0 + 4], cur[t][r0 + 5]), fmaxf(cur[t][r0 + 6], cur[t][r0 + 7])));
-      }
-      ex = xor32_max(fmaxf(fmaxf(p4[0], p4[1]), fmaxf(p4[2], p4[3])));
-    } else {
-      float p4[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = u >> 1, r0 = 8 * (u & 1);
-        p4[u] = fminf(fminf(fminf(cur[t][r0], cur[t][r0 + 1]), fminf(cur[t][r0 + 2], cur[t][r0 + 3])),
-                      fminf(fminf(cur[t][r0 + 4], cur[t][r0 + 5]), fminf(cur[t][r0 + 6], cur[t][r0 + 7])));
-      }
-      ex = xor32_min(fminf(fminf(p4[0], p4[1]), fminf(p4[2], p4[3])));
-    }
-    const float m_blk = ex * sc;
-    const bool grow = m_blk > m + kLazy;
-    if (__any(grow)) {
-      const float m_new = grow ? m_blk : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 1 where m stays, 0 at first
-      l *= alpha;
-#pragma unroll
-      for (int j = 0; j < ND; ++j) o[j] *= alpha;
-      m = m_new;
-    }
-    if (diag) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          cur[t][r] = 32 * t + 8 * (r >> 2) + (r & 3) > lim ? 0.0f : expo(cur[t][r]);
-    } else {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) cur[t][r] = expo(cur[t][r]);
-    }
-    // row sum as four independent partial sums (short dependency chains)
-    float rs4[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int t = c >> 1, r0 = 8 * (c & 1);
-      u32x4 w;
-      w.x = pk_bf16(cur[t][r0 + 0], cur[t][r0 + 1]);
-      w.y = pk_bf16(cur[t][r0 + 2], cur[t][r0 + 3]);
-      w.z = pk_bf16(cur[t][r0 + 4], cur[t][r0 + 5]);
-      w.w = pk_bf16(cur[t][r0 + 6], cur[t][r0 + 7]);
-      pb[c] = __builtin_bit_cast(bf16x8, w);
-      rs4[c] = ((cur[t][r0] + cur[t][r0 + 1]) + (cur[t][r0 + 2] + cur[t][r0 + 3])) +
-               ((cur[t][r0 + 4] + cur[t][r0 + 5]) + (cur[t][r0 + 6] + cur[t][r0 + 7]));
-    }
-    l += xor32_add((rs4[0] + rs4[1]) + (rs4[2] + rs4[3]));
-  }
-
-  // group 0: X(i), write stage i+1 | load stage i+2, Y(i).  The first and
-  // last X phases (S only, O only) are peeled so the steady loop has one body.
-  __device__ __forceinline__ void run_group0() {
-    x_phase<false, true>(0);
-    write_stage(1);
-    pp_boundary();
-    load_stage(2);
-    y_phase(0);
-    pp_boundary();
-    for (int i = 1; i < n; ++i) {
-      x_phase<true, true>(i);
-      write_stage(i + 1);
-      pp_boundary();
-      load_stage(i + 2);
-      y_phase(i);
-      pp_boundary();
-    }
-    x_phase<true, false>(n);
-    pp_boundary();
-  }
-  // group 1, one phase behind: Y(i-1), write stage i+1 | load stage i+2, X(i)
-  __device__ __forceinline__ void run_group1() {
-    write_stage(1);
-    pp_boundary();
-    load_stage(2);
-    x_phase<false, true>(0);
-    pp_boundary();
-    for (int i = 1; i < n; ++i) {
-      y_phase(i - 1);
-      write_stage(i + 1);
-      pp_boundary();
-      load_stage(i + 2);
-      x_phase<true, true>(i);
-      pp_boundary();
-    }
-    y_phase(n - 1);
-    pp_boundary();
-    x_phase<true, false>(n);
-  }
-};
-
-// the workgroup's queries: query blocks of one (b, h) kept on one XCD
-__device__ __forceinline__ void pp_block_coords(const SdpaArgs& p, int& bh, int& qb) {
-  block_coords(p, bh, qb);
-}
-
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(PP_THREADS, 1) void sdpa_pp_kernel(const SdpaArgs p) {
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[2][BKV * kKPitch<D>];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[2][BKV * kVPitch<D>];
-  SdpaPP<D, CAUSAL> w{p, Ks, Vs};
-  int bh;
-  pp_block_coords(p, bh, w.qb);
-  w.lane = threadIdx.x & 63;
-  w.wave = threadIdx.x >> 6;
-  w.l32 = w.lane & 31;
-  w.h = w.lane >> 5;
-  w.base = static_cast<int64_t>(bh) * p.S * D;
-  w.q = w.qb * PP_BQ + w.wave * 32 + w.l32;
-  w.sc = p.scale_log2;
-  w.m = -INFINITY;
-  w.l = 0.0f;
-  w.n = CAUSAL ? (w.qb * PP_BQ + PP_BQ) / BKV : p.S / BKV;
-
-  // prologue: Q^T into VGPRs, stage 0 (K(0)) into LDS, stage 1 into registers
-#pragma unroll
-  for (int dc = 0; dc < D / 16; ++dc)
-    w.qop[dc] = *reinterpret_cast<const bf16x8*>(p.Q + w.base + static_cast<int64_t>(w.q) * D +
-                                                 dc * 16 + 8 * w.h);
-  w.load_stage(0);
-  // Q^T and K(0) must have landed before any later load is issued: the
-  // stage loads are conditional, so a partial wait after them would leave Q
-  // "possibly in flight" on some path, and the compiler would then make every
-  // S MFMA wait for the stage prefetch in flight at that point
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm_sdpa(0));
-  w.write_stage(0);
-  w.load_stage(1);
-#pragma unroll
-  for (int j = 0; j < D / 32; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) w.o[j][r] = 0.0f;
-  pp_boundary();
-
-  if (w.wave < 4) w.run_group0();
-  else w.run_group1();
-
-  const float inv = 1.0f / w.l;
-  uint16_t* orow = p.O + w.base + static_cast<int64_t>(w.q) * D;
-#pragma unroll
-  for (int j = 0; j < D / 32; ++j)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int d = 32 * j + 8 * u + 4 * w.h;
-      const u32x2 v = {pk_bf16(w.o[j][4 * u] * inv, w.o[j][4 * u + 1] * inv),
-                       pk_bf16(w.o[j][4 * u + 2] * inv, w.o[j][4 * u + 3] * inv)};
-      *reinterpret_cast<u32x2*>(orow + d) = v;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1199,8 +940,18 @@ __global__ __launch_bounds__(W8_THREADS, 1) void sdpa_w8_kernel(const SdpaArgs p
 }
 
 template <int D, bool CAUSAL>
-int launch(const SdpaArgs& a, hipStream_t s) {
-  if (D == W8_D && !CAUSAL && a.S % W8_BQ == 0) {
+int launch(SdpaArgs a, hipStream_t s) {
+  // heads dispatched together: a divisor of an XCD's share of the heads whose
+  // K and V (2 x 2 S D bytes a head) fit its 4 MiB L2
+  const int share = a.nbh % 8 == 0 ? a.nbh / 8 : 1;
+  const int64_t fit = (int64_t(4) << 20) / (int64_t(4) * a.S * D);
+  a.heads_together = 1;
+  for (int g = 1; g <= share && g <= fit; ++g)
+    if (share % g == 0) a.heads_together = g;
+  const int64_t blocks = static_cast<int64_t>(a.nbh) * a.nqb;
+  // (256 blocks of 128 queries and fewer leave sdpa_w8_kernel half the CUs:
+  // 1 x 8 x 2048 x 128 46.6 us against 40 to 42 in sdpa_fwd_kernel)
+  if (D == W8_D && !CAUSAL && a.S % W8_BQ == 0 && blocks > 256) {
     SdpaArgs b = a;
     b.nqb = a.S / W8_BQ;
     // persistent: one workgroup per CU (at most), each walking its blocks
@@ -1213,18 +964,22 @@ int launch(const SdpaArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(sdpa_w8_kernel, dim3(grid), dim3(W8_THREADS), 0, s, b);
     return check_launch("sdpa_w8_kernel");
   }
-  if (a.S % PP_BQ == 0) {
-    SdpaArgs b = a;
-    b.nqb = a.S / PP_BQ;
-    hipLaunchKernelGGL((sdpa_pp_kernel<D, CAUSAL>), dim3(b.nbh * b.nqb), dim3(PP_THREADS), 0, s, b);
-    return check_launch("sdpa_pp_kernel");
-  }
-  if (a.S % BQ != 0) {  // a ragged tail (S % 32 == 0)
-    hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, true>), dim3(a.nbh * a.nqb), dim3(kThreads), 0,
-                       s, a);
-    return check_launch("sdpa_fwd_kernel");
-  }
-  hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL>), dim3(a.nbh * a.nqb), dim3(kThreads), 0, s, a);
+  // Two groups of waves: up to one workgroup per CU, and under the causal mask
+  // up to two rounds of long blocks, whose shares of a CU would differ most (512
+  // blocks of S = 2016: 62 us against 69; of S = 480: 28 against 24; 384
+  // blocks without the mask: 84 against 72).  Two KV blocks do not pay for the
+  // second group.
+  const bool two = a.S > 128 && (blocks <= 256 || (CAUSAL && blocks <= 512 && a.S >= 1024));
+  const dim3 grid(static_cast<uint32_t>(blocks));
+  const bool ragged = a.S % BQ != 0;  // S % 32 == 0 only
+  if (two && ragged)
+    hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, true, 2>), grid, dim3(2 * kThreads), 0, s, a);
+  else if (two)
+    hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, false, 2>), grid, dim3(2 * kThreads), 0, s, a);
+  else if (ragged)
+    hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, true, 1>), grid, dim3(kThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, false, 1>), grid, dim3(kThreads), 0, s, a);
   return check_launch("sdpa_fwd_kernel");
 }
 
