@@ -944,6 +944,72 @@ __global__ __launch_bounds__(256) void reduce_cols_kernel(const RedArgs a) {
   }
 }
 
+// Column reduce of a plain bf16 operand.  A workgroup takes 64 columns (eight
+// lanes, one 128-byte line of a row: with 32 columns a line is asked for twice,
+// and a CU asks for about one line every ten clocks whatever it uses of it) and
+// its share of the rows, 64 rows a pass, eight passes in flight.  The lanes of a
+// wave that hold the same columns halve their eight sums three times over, the
+// waves meet in LDS.  Workgroups of neighbouring strips are on one XCD.
+constexpr int kStripCols = 64, kStripThreads = 512;
+
+template <int KIND>
+__global__ __launch_bounds__(kStripThreads) void reduce_cols_strip_kernel(const uint16_t* base,
+                                                                          int64_t rs, int64_t strips,
+                                                                          const RedArgs a) {
+  constexpr int R = kStripThreads / 8, W = kStripThreads / 64, D = 8;
+  __shared__ float part[W][kStripCols];
+  const int n = gridDim.x, id = blockIdx.x, per = n >> 3, rem = n & 7, xcd = id & 7;
+  const int i0 = xcd * per + min(xcd, rem) + (id >> 3);
+  const int split = i0 / static_cast<int>(strips), strip = i0 - split * static_cast<int>(strips);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t col = int64_t(strip) * kStripCols + 8 * (lane & 7);
+  const int64_t rb = split * a.rows_per_split;
+  const int64_t re = rb + a.rows_per_split < a.h ? rb + a.rows_per_split : a.h;
+  float acc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) acc[k] = red_identity(KIND);
+  if (col < a.w) {  // w % 8 == 0: all eight columns
+    int64_t row = rb + (t >> 3);
+    uintptr_t q = reinterpret_cast<uintptr_t>(base + col) + 2 * rs * row;
+    const int64_t step = 2 * rs * R;
+    u32x4 c[D];  // slots past the last row are neither fetched nor read
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+      if (row + i * R < re) c[i] = ld16<false>(q + i * step);
+    const float s = red_scale(a);  // after the first row loads are in flight
+    for (; row < re; row += D * R, q += D * step) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        if (row + i * R < re) {
+          const f32x8 v = unpack_bf16x8(c[i]);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) acc[k] = red_acc_k<KIND>(acc[k], v[k], s);
+        }
+        if (row + (i + D) * R < re) c[i] = ld16<false>(q + (i + D) * step);
+      }
+    }
+  }
+  const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+  float v4[4], v2[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    v4[k] = red_combine_k<KIND>(b5 ? acc[4 + k] : acc[k],
+                                __shfl_xor(b5 ? acc[k] : acc[4 + k], 32, 64));
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    v2[k] = red_combine_k<KIND>(b4 ? v4[2 + k] : v4[k], __shfl_xor(b4 ? v4[k] : v4[2 + k], 16, 64));
+  part[wave][8 * (lane & 7) + (b5 ? 4 : 0) + (b4 ? 2 : 0) + (b3 ? 1 : 0)] =
+      red_combine_k<KIND>(b3 ? v2[1] : v2[0], __shfl_xor(b3 ? v2[0] : v2[1], 8, 64));
+  __syncthreads();
+  const int64_t oc = int64_t(strip) * kStripCols + t;
+  if (t >= kStripCols || oc >= a.w) return;
+  float r = part[0][t];
+#pragma unroll
+  for (int w = 1; w < W; ++w) r = red_combine_k<KIND>(r, part[w][t]);
+  if (a.splits == 1) red_write<TTLH_REDUCE_DIM0>(a, oc, r);
+  else a.ws[split * a.w + oc] = r;
+}
+
 // p[0], p[stride], ..., p[(n - 1) stride] combined in that order, eight
 // loads in flight
 __device__ __forceinline__ float red_strided(int kind, const float* p, int64_t n, int64_t stride) {
@@ -1832,6 +1898,36 @@ int reduce_impl(const char* who, const ttlh_instr* prog, const ttlh_operand* in,
   {
     a.rows_per_split = red_rows_per_split(h, w);
     a.splits = static_cast<int32_t>((h + a.rows_per_split - 1) / a.rows_per_split);
+    const EltOperand& o0 = a.e.ops[0];
+    const int64_t strips = (w + kStripCols - 1) / kStripCols;
+    if (mode == 1 && plain_row(o0) && strips < (int64_t(1) << 24)) {
+      // Shares of at least 1024 rows, at most eight (and at most the
+      // workspace's), while all make up to 512 workgroups: one launch below
+      // 2048 rows (512 x 4096: 3.9 us, 5.5 in two shares, 9.7 in 32-row shares of
+      // 512 columns by the kernel below), 4096^2 in four 11.5 us (one 17, eight
+      // 13; 15 below), 8192^2 in four 27 (two 31; 47 below).
+      const int64_t fill = strips < 512 ? 512 / strips : 1;
+      int64_t sp = h / 1024 < fill ? h / 1024 : fill;
+      if (sp > 8) sp = 8;
+      if (sp > a.splits) sp = a.splits;
+      if (sp < 1) sp = 1;
+      a.rows_per_split = (h + sp - 1) / sp;
+      a.splits = static_cast<int32_t>((h + a.rows_per_split - 1) / a.rows_per_split);
+      const uint16_t* const base = static_cast<const uint16_t*>(o0.ptr) +
+                                   (a.e.y0 + o0.roff) * o0.rs + a.e.x0 + o0.coff;
+      const dim3 sgrid(static_cast<uint32_t>(strips * a.splits));
+      if (kind == TTLH_REDUCE_SUM)
+        hipLaunchKernelGGL(reduce_cols_strip_kernel<TTLH_REDUCE_SUM>, sgrid, dim3(kStripThreads), 0,
+                           s, base, int64_t(o0.rs), strips, a);
+      else
+        hipLaunchKernelGGL(reduce_cols_strip_kernel<TTLH_REDUCE_MAX>, sgrid, dim3(kStripThreads), 0,
+                           s, base, int64_t(o0.rs), strips, a);
+      const int rc = check_launch("reduce_cols_strip_kernel");
+      if (rc != TTLH_OK || a.splits == 1) return rc;
+      hipLaunchKernelGGL(reduce_cols_finish_kernel, dim3(static_cast<uint32_t>((w + 31) / 32)),
+                         block, 0, s, a);
+      return check_launch("reduce_cols_finish_kernel");
+    }
     const int vw = pi.vec ? 8 : 1;
     const dim3 grid(static_cast<uint32_t>((w + 64 * vw - 1) / (64 * vw)),
                     static_cast<uint32_t>(a.splits));

@@ -10,6 +10,7 @@ torch.cuda.synchronize() themselves.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import struct
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
@@ -54,9 +55,9 @@ def _check_device(t: torch.Tensor, what: str) -> None:
 _WORKSPACES: dict = {}
 
 
-def _workspace(device: torch.device, stream, nbytes: int) -> torch.Tensor:
-    sp = L.stream_ptr(stream)
-    key = (device.index, sp)
+def _workspace(device: torch.device, stream, nbytes: int,
+               sp: Optional[int] = None) -> torch.Tensor:
+    key = (device.index, L.stream_ptr(stream) if sp is None else sp)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -245,6 +246,11 @@ def eltwise(prog: StackProgram, operands: Sequence[Optional[OperandMap]], out: t
            out.stride(0), y0, x0, h, w, L.stream_ptr(stream))
 
 
+@functools.lru_cache(maxsize=1024)
+def _reduce_workspace_bytes(dbits: int, h: int, w: int) -> int:
+    return int(L.load().ttlh_reduce_workspace_bytes(dbits, h, w))
+
+
 def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: str,
            dims: Sequence[int], out: torch.Tensor, region, out_origin=(0, 0),
            out_pad: bool = False, scaler: Optional[torch.Tensor] = None, scale: float = 1.0,
@@ -263,7 +269,7 @@ def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: s
         raise ValueError("reduce output must have unit column stride")
     if kind not in ("sum", "max"):
         raise ValueError(f"reduce kind must be 'sum' or 'max', got {kind!r}")
-    dset = set(int(d) for d in dims)
+    dset = {int(d) for d in dims}
     if not dset or not dset <= {0, 1}:
         raise ValueError(f"reduce dims must be a non-empty subset of [0, 1], got {list(dims)}")
     dbits = (L.REDUCE_DIM0 if 0 in dset else 0) | (L.REDUCE_DIM1 if 1 in dset else 0)
@@ -290,12 +296,13 @@ def reduce(prog: StackProgram, operands: Sequence[Optional[OperandMap]], kind: s
                L.dtype_code(out.dtype), out.stride(0), int(bool(out_pad)), y0, x0, h, w,
                L.stream_ptr(stream))
         return
-    ws_bytes = int(L.load().ttlh_reduce_workspace_bytes(dbits, h, w))
-    ws = _workspace(out.device, stream, ws_bytes) if ws_bytes else None
+    stp = L.stream_ptr(stream)
+    ws_bytes = _reduce_workspace_bytes(dbits, h, w)
+    ws = _workspace(out.device, stream, ws_bytes, stp) if ws_bytes else None
     L.call("ttlh_reduce", instrs, ops, n, kcode,
            dbits, sp, sdt, float(scale), optr, L.dtype_code(out.dtype), out.stride(0),
            int(bool(out_pad)), y0, x0, h, w, ws.data_ptr() if ws is not None else 0, ws_bytes,
-           L.stream_ptr(stream))
+           stp)
 
 
 @dataclass
