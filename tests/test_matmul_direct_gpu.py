@@ -12,6 +12,7 @@ import torch
 
 from oracle import bfp8 as OB
 from oracle import tile_ops as O
+from ttlhip import _lib as L
 from ttlhip import kernels as Kn
 
 pytestmark = pytest.mark.gpu
@@ -53,6 +54,39 @@ def test_bf16_blocks(M, K, N):
         _check(wide, a, b, True)
     assert torch.equal(buf[:, 1:N + 1], wide)
     assert bool((buf[:, 0] == 7).all()) and bool((buf[:, N + 1:] == 7).all())
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 224, 256, 352])
+def test_bf16_blocks_of_128(K):
+    # mm_mid_kernel: every number of stages around its ring of four buffers,
+    # blocks cut in both directions, accumulation and fp32 results
+    M, N = 2080, 1952
+    print(f"mid bf16 K={K}", flush=True)
+    a, b = _operands(M, K, N, 11)
+    c = torch.full((M, N + 2), 7.0, dtype=torch.bfloat16, device="cuda")
+    Kn.matmul(a, b, c[:, :N])
+    _check(c[:, :N], a, b, True)
+    assert bool((c[:, N:] == 7).all())
+    odd = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device="cuda")
+    Kn.matmul(a, b, odd[:, 1:N + 1])
+    assert torch.equal(odd[:, 1:N + 1], c[:, :N])
+    assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())
+    f = O.seeded((M, N), "normal", 12, torch.float32).cuda()
+    f0 = f.clone()
+    Kn.matmul(a, b, f, accumulate=True)
+    _check(f - f0, a, b, False)
+
+
+def test_bf16_blocks_of_128_with_slow_operand_loads():
+    # A and B in pinned host memory: every stage's loads take far longer than
+    # a stage, so a wait that covered too few of them would read a stale stage
+    a, b = _operands(2080, 352, 1952, 17)
+    pa, pb = a.cpu().pin_memory(), b.cpu().pin_memory()
+    c = torch.zeros(2080, 1952, dtype=torch.bfloat16, device="cuda")
+    L.call("ttlh_matmul", pa.data_ptr(), L.TTLH_BF16, 352, pb.data_ptr(), L.TTLH_BF16, 1952,
+           c.data_ptr(), L.TTLH_BF16, 1952, 2080, 1952, 352, 0, L.stream_ptr())
+    torch.cuda.synchronize()
+    _check(c, a, b, True)
 
 
 @pytest.mark.parametrize("M,K,N", [(32, 32, 32), (64, 2048, 96), (96, 160, 224), (32, 4096, 32),

@@ -26,6 +26,7 @@
 //  - the epilogue rounds once to the output dtype (RNE).
 // fp32 inputs take a simpler v_mfma_f32_32x32x2f32 kernel (64x64 blocks).
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -55,6 +56,7 @@ struct MmArgs {
   int32_t M, N, K;
   int32_t c_dtype, accumulate;
   int32_t grid_m, grid_n;  // output blocks along M / N
+  int32_t c_pairs;         // mm_mid_kernel: two columns of C are one aligned store
 };
 
 // XCD-aware block order: MI355X dispatches workgroup i to XCD i % 8.  Regroup
@@ -1378,6 +1380,157 @@ bool launch_mm_dma_as(const MmArgs& a, hipStream_t s, int* status) {
 }
 
 // ---------------------------------------------------------------------------
+// The same pipeline in 128x128 blocks, for problems whose 256x256 blocks would
+// leave CUs idle: four waves of 64x64 (2x2 MFMA tiles), 32-k stages of 16 KB in
+// four LDS buffers, two workgroups per CU.  A wave feeds each fragment to two
+// MFMAs instead of four, so the LDS reads (128 bytes a clock and CU at full MFMA
+// rate) take as long as the MFMAs; the second workgroup's MFMAs run under one's
+// reads and barriers, which is why the stage is not sequenced by hand.
+__shared__ __attribute__((aligned(16))) uint16_t midA0[BM * DK], midA1[BM * DK], midA2[BM * DK],
+    midA3[BM * DK];
+__shared__ __attribute__((aligned(16))) uint16_t midB0[DK * BN], midB1[DK * BN], midB2[DK * BN],
+    midB3[DK * BN];
+
+template <int Q>
+__device__ __forceinline__ uint16_t* mid_abuf() {
+  if constexpr (Q == 0) return midA0;
+  else if constexpr (Q == 1) return midA1;
+  else if constexpr (Q == 2) return midA2;
+  else return midA3;
+}
+template <int Q>
+__device__ __forceinline__ uint16_t* mid_bbuf() {
+  if constexpr (Q == 0) return midB0;
+  else if constexpr (Q == 1) return midB1;
+  else if constexpr (Q == 2) return midB2;
+  else return midB3;
+}
+
+template <bool OUT_BF16, bool ACC>
+__global__ __launch_bounds__(kThreads, 2) void mm_mid_kernel(const MmArgs p) {
+  int bm, bn;
+  block_coords(p, bm, bn);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wbase = t & ~63;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const int l32 = lane & 31, h = lane >> 5;
+
+  // loads: 16-byte position i * 256 + t of the stage; chunk c of A row r (64
+  // bytes) sits at c ^ ((r >> 2) & 3), of B row r (256 bytes) at c ^ 4 (r & 3).
+  // Rows past M and columns past N re-read the last ones.
+  const uint16_t* a_src[2];
+  const uint16_t* b_src[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int pos = i * kThreads + t;
+    const int ar = pos >> 2, ac = (pos & 3) ^ ((ar >> 2) & 3);
+    a_src[i] = p.A + static_cast<int64_t>(min(bm * BM + ar, p.M - 1)) * p.lda + ac * 8;
+    const int br = pos >> 4, bc = (pos & 15) ^ ((br & 3) << 2);
+    b_src[i] = p.B + static_cast<int64_t>(br) * p.ldb + min(bn * BN + bc * 8, p.N - 8);
+  }
+  // fragments (byte offsets): A row wm + l32, k chunk 2 sub + h; B transpose
+  // read of rows kb + (lane & 15) / 4 and columns wn + 32 j + 16 ((lane >> 4) & 1)
+  // + 4 (lane & 3), as in mm_dma_kernel
+  const int xa = (l32 >> 2) & 3, arow = (wm + l32) * 64;
+  const int fa[2] = {arow + (h ^ xa) * 16, arow + ((2 + h) ^ xa) * 16};
+  const int brow = (lane & 15) >> 2, e = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+  int fb[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    fb[j] = (8 * h + brow) * 256 + ((wn / 8 + 4 * j + e) ^ (4 * brow)) * 16 + 8 * (lane & 1);
+
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  auto load = [&](int s, uint16_t* Ab, uint16_t* Bb) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      __builtin_amdgcn_global_load_lds(a_src[i] + s * DK, (lds_void*)(Ab + (i * kThreads + wbase) * 8),
+                                       16, 0, 0);
+      __builtin_amdgcn_global_load_lds(b_src[i] + static_cast<int64_t>(s * DK) * p.ldb,
+                                       (lds_void*)(Bb + (i * kThreads + wbase) * 8), 16, 0, 0);
+    }
+  };
+  const int nk = p.K / DK;
+  load(0, midA0, midB0);
+  if (1 < nk) load(1, midA1, midB1);
+  if (2 < nk) load(2, midA2, midB2);
+
+  // stage s in buffer Q: wait for this wave's loads of it (later stages, four
+  // loads each, may be in flight), meet the other waves, which are then also
+  // done with buffer Q - 1, fetch stage s + 3 into that, and multiply
+  auto stage = [&](auto qq, auto steady, int s) {
+    constexpr int q = decltype(qq)::value;
+    constexpr bool STEADY = decltype(steady)::value;
+    const char* Ab = reinterpret_cast<const char*>(mid_abuf<q>());
+    const char* Bb = reinterpret_cast<const char*>(mid_bbuf<q>());
+    if (STEADY || s + 2 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(8));
+    else if (s + 1 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(4));
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    stage_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (STEADY || s + 3 < nk) load(s + 3, mid_abuf<(q + 3) & 3>(), mid_bbuf<(q + 3) & 3>());
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      bf16x8 a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        a[i] = *reinterpret_cast<const bf16x8*>(Ab + fa[sub] + i * 32 * 64);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const char* src = Bb + fb[j] + sub * 16 * 256;
+        const i16x4m lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4m*)src);
+        const i16x4m hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4m*)(src + 4 * 256));
+        const i16x8m w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        b[j] = __builtin_bit_cast(bf16x8, w);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  int s = 0;
+  for (; s + 7 <= nk; s += 4) {
+    stage(I0(), std::true_type(), s);
+    stage(I1(), std::true_type(), s + 1);
+    stage(I2(), std::true_type(), s + 2);
+    stage(I3(), std::true_type(), s + 3);
+  }
+  for (; s + 4 <= nk; s += 4) {
+    stage(I0(), std::false_type(), s);
+    stage(I1(), std::false_type(), s + 1);
+    stage(I2(), std::false_type(), s + 2);
+    stage(I3(), std::false_type(), s + 3);
+  }
+  if (s < nk) stage(I0(), std::false_type(), s);
+  if (s + 1 < nk) stage(I1(), std::false_type(), s + 1);
+  if (s + 2 < nk) stage(I2(), std::false_type(), s + 2);
+
+  const int r0 = bm * BM + wm, c0 = bn * BN + wn;
+  static_for<4>([&](auto ij) {
+    constexpr int i = decltype(ij)::value / 2, j = decltype(ij)::value % 2;
+    if (r0 + i * 32 < p.M && c0 + j * 32 < p.N) {
+      if (p.c_pairs)
+        store_acc_tile_pairs<OUT_BF16, ACC>(p, acc[i][j], r0 + i * 32, c0 + j * 32, lane);
+      else
+        store_acc_tile(p, acc[i][j], r0 + i * 32, c0 + j * 32, lane);
+    }
+  });
+}
+
+// ---------------------------------------------------------------------------
 // bf16 x bfloat8_b with the weights dequantised in LDS ahead of the MFMAs.
 // Tiling, A pipeline, fragment reads and MFMA sequence are mm_dma_kernel's
 // (256x256 block, four waves of 128x128, 32-k stages, A in a ring of four
@@ -1728,34 +1881,77 @@ __global__ __launch_bounds__(kThreads, 1) void mm_dq_kernel(const MmArgs p) {
   });
 }
 
-// Launches the 256x256 kernel when the problem has enough 256x256 blocks to
-// fill the chip; returns false otherwise.
-template <bool BQ>
-bool launch_mm256(MmArgs a, hipStream_t s, int* status) {
+// Launches a 256x256 bfloat8_b kernel when the problem has enough 256x256
+// blocks to fill the chip; returns false otherwise.
+bool launch_mm256_bq(MmArgs a, hipStream_t s, int* status) {
   const int gm = (a.M + LM - 1) / LM, gn = (a.N + LN - 1) / LN;
   if (static_cast<int64_t>(gm) * gn < 192) return false;
   if (static_cast<int64_t>(a.M) * a.ldc >= (int64_t(1) << 31)) return false;  // 32-bit C offsets
   a.grid_m = gm;
   a.grid_n = gn;
-  if constexpr (BQ) {
-    // weights dequantised in LDS: whole 256-column blocks of whole stage
-    // quads, tiles 16-byte aligned
-    if (a.N % LN == 0 && a.K % (4 * DK) == 0 && (reinterpret_cast<uintptr_t>(a.Bq) & 15) == 0 &&
-        static_cast<int64_t>(a.M) * a.lda * 2 < (int64_t(1) << 31) &&
-        static_cast<int64_t>(a.K / 32) * (a.N / 32) * TTLH_BFP8_TILE_BYTES < (int64_t(1) << 31)) {
-      hipLaunchKernelGGL((mm_dq_kernel<true, false>), dim3(a.grid_m * a.grid_n), dim3(kThreads), 0,
-                         s, a);
-      *status = check_launch("mm_dq_kernel");
-      return true;
-    }
-    return launch_mm256_as<true, true, false>(a, s, status);
-  } else {
-    if (a.c_dtype == TTLH_BF16)
-      return a.accumulate ? launch_mm_dma_as<true, true>(a, s, status)
-                          : launch_mm_dma_as<true, false>(a, s, status);
-    return a.accumulate ? launch_mm_dma_as<false, true>(a, s, status)
-                        : launch_mm_dma_as<false, false>(a, s, status);
+  // weights dequantised in LDS: whole 256-column blocks of whole stage
+  // quads, tiles 16-byte aligned
+  if (a.N % LN == 0 && a.K % (4 * DK) == 0 && (reinterpret_cast<uintptr_t>(a.Bq) & 15) == 0 &&
+      static_cast<int64_t>(a.M) * a.lda * 2 < (int64_t(1) << 31) &&
+      static_cast<int64_t>(a.K / 32) * (a.N / 32) * TTLH_BFP8_TILE_BYTES < (int64_t(1) << 31)) {
+    hipLaunchKernelGGL((mm_dq_kernel<true, false>), dim3(a.grid_m * a.grid_n), dim3(kThreads), 0,
+                       s, a);
+    *status = check_launch("mm_dq_kernel");
+    return true;
   }
+  return launch_mm256_as<true, true, false>(a, s, status);
+}
+
+// Modelled times, us, of the two bf16 kernels that stage through LDS, fitted
+// to measurements of 24 problems (2048^3: 128x128 blocks 25 us, 256x256 44;
+// 3168 x 7072 x 3104: 211 and 157; 4096^3: 146 and 112; 3008 x 2784 x 5696:
+// 122 and 130).  256x256: one block per CU, and a partly filled round runs at
+// a higher clock.  128x128: two blocks per CU.
+// `reg`: mm_bf16_kernel, for results that the other two cannot address.
+struct LdsTimes {
+  double dma, mid, reg;
+};
+LdsTimes lds_times(const MmArgs& a) {
+  const double k = a.K / 32.0;
+  const int64_t b128 = int64_t((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+  const double y = b128 / 256.0;
+  LdsTimes t = {1e30, 1e30, 10 + k * std::max(0.57, 0.37 * y)};
+  if (static_cast<int64_t>(a.M) * a.ldc >= (int64_t(1) << 31)) return t;  // 32-bit C offsets
+  const int64_t b256 = int64_t((a.M + LM - 1) / LM) * ((a.N + LN - 1) / LN);
+  const double x = b256 / 256.0;
+  t.dma = 8 + k * (x <= 1 ? 0.53 + 0.25 * x : 1.4 + 0.5 * (x - 1));
+  t.mid = 4 + k * (y <= 1 ? 0.3 : 0.3 * y + (b128 % 256 ? 0.12 : 0.05));
+  if (b256 >= 192) t.mid *= 1.08;  // near a tie the 256x256 kernel, whose model is the steadier
+  return t;
+}
+
+bool launch_dma(MmArgs a, hipStream_t s, int* status) {
+  if (static_cast<int64_t>(a.M) * a.ldc >= (int64_t(1) << 31)) return false;
+  a.grid_m = (a.M + LM - 1) / LM;
+  a.grid_n = (a.N + LN - 1) / LN;
+  if (a.c_dtype == TTLH_BF16)
+    return a.accumulate ? launch_mm_dma_as<true, true>(a, s, status)
+                        : launch_mm_dma_as<true, false>(a, s, status);
+  return a.accumulate ? launch_mm_dma_as<false, true>(a, s, status)
+                      : launch_mm_dma_as<false, false>(a, s, status);
+}
+
+bool launch_mid(MmArgs a, hipStream_t s, int* status) {
+  if (lds_times(a).mid >= 1e30) return false;
+  a.grid_m = (a.M + BM - 1) / BM;
+  a.grid_n = (a.N + BN - 1) / BN;
+  a.c_pairs = (reinterpret_cast<uintptr_t>(a.C) & (a.c_dtype == TTLH_BF16 ? 3 : 7)) == 0 &&
+              a.ldc % 2 == 0;
+  const dim3 grid(a.grid_m * a.grid_n), block(kThreads);
+  if (a.c_dtype == TTLH_BF16) {
+    if (a.accumulate) hipLaunchKernelGGL((mm_mid_kernel<true, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((mm_mid_kernel<true, false>), grid, block, 0, s, a);
+  } else {
+    if (a.accumulate) hipLaunchKernelGGL((mm_mid_kernel<false, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((mm_mid_kernel<false, false>), grid, block, 0, s, a);
+  }
+  *status = check_launch("mm_mid_kernel");
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1876,9 +2072,11 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
     a.K = static_cast<int32_t>(K);
     a.c_dtype = c_dtype;
     a.accumulate = accumulate ? 1 : 0;
-    // a 256-row block would be mostly padding for one or two tiles of rows
-    if (M > 64 && launch_mm256<false>(a, s, &status)) return status;
-    if (launch_direct_bf16(d, scratch, s, &status)) return status;
+    const LdsTimes lds = lds_times(a);
+    if (launch_direct_bf16(d, std::min({lds.dma, lds.mid, lds.reg}), scratch, s, &status))
+      return status;
+    if (lds.dma <= lds.mid && launch_dma(a, s, &status)) return status;
+    if (launch_mid(a, s, &status)) return status;
     a.grid_m = static_cast<int32_t>((M + BM - 1) / BM);
     a.grid_n = static_cast<int32_t>((N + BN - 1) / BN);
     hipLaunchKernelGGL(mm_bf16_kernel<false>, dim3(a.grid_m * a.grid_n), dim3(kThreads), 0, s, a);
@@ -1931,7 +2129,7 @@ int matmul_block(const char* fn, int bits, const void* A, int64_t lda, const voi
   a.accumulate = 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   int status = TTLH_OK;
-  if (bits == 8 && M > 64 && launch_mm256<true>(a, s, &status)) return status;
+  if (bits == 8 && M > 64 && launch_mm256_bq(a, s, &status)) return status;
   DirectArgs d = {};
   d.A = A;
   d.B = Bq;

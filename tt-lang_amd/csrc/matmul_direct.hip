@@ -652,53 +652,36 @@ bool offsets_fit(const DirectArgs& a, int elem) {
 
 }  // namespace
 
-bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status) {
+bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_t s, int* status) {
   if (!offsets_fit(a, 2)) return false;
   set_c_vec(a);
-  // Modelled time of each shape, us: per round of workgroups the chip holds
-  // at once, a fixed part and one per 32-k stage, both fitted to measurements
-  // of 32 problems from 32x512x512 to 4096x512x2048 (the choice was within 8%
-  // of the best measured shape on 28 of them, within 20% on all).
+  // Modelled time of each block shape, us: per round of 256 workgroups a fixed
+  // part and one per 32-k stage of a wave's share, fitted to measurements of 50
+  // problems from 32x32x32 to 4096x512x2048 (the choice was the fastest of the
+  // shapes or within 10% of it, but for a few at 20%).
   const double k = a.K / 32.0;
-  const auto rounds = [](int64_t blocks, int held) {
-    return static_cast<double>((blocks + held - 1) / held);
-  };
-  const int64_t b64 = blocks_of(a, 32, 64), b128 = blocks_of(a, 32, 128), m64 = blocks_of(a, 64, 128),
-                lds = blocks_of(a, 128, 128);
+  const auto rounds = [](int64_t blocks) { return static_cast<double>((blocks + 255) / 256); };
+  const int64_t b64 = blocks_of(a, 32, 64), b128 = blocks_of(a, 32, 128), m64 = blocks_of(a, 64, 128);
   const int p64 = k_parts(b64, a.K, 1024, scratch, s);
   const int p128 = b128 >= 80 ? std::min(2, k_parts(b128, a.K, 1024, scratch, s)) : 1;
-  const double t[6] = {
-      2 + 0.11 * k / p64 * rounds(b64 * p64, 256) + (p64 > 1 ? 2 : 0),
-      2 + 0.153 * k / p128 * rounds(b128 * p128, 256) + (p128 > 1 ? 2 : 0),
-      3 + k * (b128 <= 256 ? 0.17 : 0.267 * std::max(1.0, b128 / 512.0)),
-      3 + 0.237 * k * rounds(m64, 256),
-      (6 + 0.4 * k) * rounds(m64, 512),
-      10 + 0.57 * k * std::max(1.0, 0.65 * rounds(lds, 256)),  // 128x128 through LDS (matmul.hip)
+  const double t[3] = {
+      1 + (1.2 + 0.11 * k / p64) * rounds(b64 * p64) + (p64 > 1 ? 2 : 0),
+      1 + (1.5 + 0.153 * k / p128) * rounds(b128 * p128) + (p128 > 1 ? 2 : 0),
+      1 + (2 + 0.237 * k) * rounds(m64),
   };
-  switch (std::min_element(t, t + 6) - t) {
-    case 0:
-      set_blocks(a, 32, 64, p64, scratch);
-      TTLH_DIRECT((mm_direct_kernel<2, 4, 8, 3, 3>), 8, "mm_direct_kernel");
-      return true;
-    case 1:
-      set_blocks(a, 32, 128, p128, scratch);
-      TTLH_DIRECT((mm_direct_kernel<2, 8, 8, 2, 2>), 8, "mm_direct_kernel");
-      return true;
-    case 2:
-      set_blocks(a, 32, 128, 1, nullptr);
-      TTLH_DIRECT((mm_direct_kernel<2, 8, 4, 3, 2>), 4, "mm_direct_kernel");
-      return true;
-    case 3:
-      set_blocks(a, 64, 128, 1, nullptr);
-      TTLH_DIRECT((mm_direct_kernel<4, 8, 4, 2, 2>), 4, "mm_direct_kernel");
-      return true;
-    case 4:
-      set_blocks(a, 64, 128, 1, nullptr);
-      TTLH_DIRECT((mm_direct_kernel<4, 8, 2, 2, 1>), 2, "mm_direct_kernel");
-      return true;
-    default:
-      return false;
+  const int best = static_cast<int>(std::min_element(t, t + 3) - t);
+  if (t[best] >= other_us) return false;
+  if (best == 0) {
+    set_blocks(a, 32, 64, p64, scratch);
+    TTLH_DIRECT((mm_direct_kernel<2, 4, 8, 3, 3>), 8, "mm_direct_kernel");
+  } else if (best == 1) {
+    set_blocks(a, 32, 128, p128, scratch);
+    TTLH_DIRECT((mm_direct_kernel<2, 8, 8, 2, 2>), 8, "mm_direct_kernel");
+  } else {
+    set_blocks(a, 64, 128, 1, nullptr);
+    TTLH_DIRECT((mm_direct_kernel<4, 8, 4, 2, 2>), 4, "mm_direct_kernel");
   }
+  return true;
 }
 
 bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status) {

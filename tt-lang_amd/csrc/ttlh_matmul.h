@@ -23,7 +23,8 @@ struct DirectArgs {
 // the launch's status in *status, or returns false, having launched nothing,
 // where the caller's other kernels take the problem.  `scratch`: null, or
 // TTLH_MATMUL_SCRATCH_BYTES of device memory (see ttlh_matmul_scratch).
-bool launch_direct_bf16(DirectArgs a, void* scratch, hipStream_t s, int* status);
+// other_us: the modelled time of the caller's best kernel.
+bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_t s, int* status);
 bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status);
 bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status);
 
