@@ -588,14 +588,15 @@ def bfp8_unpack(q: torch.Tensor, rows: int, cols: int, stream=None) -> torch.Ten
     return out
 
 
-# At and above this many rows of A the weight tiles are dequantised once into a
-# bf16 workspace and multiplied by the bf16 GEMM; below it the kernels that
-# decode on the way to the MFMAs, once per 32 or 64 rows of A, are used.  At
-# 512 x 4096 x 4096 the two take the same time (38 us decoding, 8 to 10 us for
-# the unpack and 29 for the GEMM), at 256 x 4096 x 11008 decoding takes 53 us
-# against 25 + 62.
+# From this many rows of A and multiply-adds on, the weight tiles are dequantised
+# once into a bf16 workspace and multiplied by the bf16 GEMM; below, the kernels
+# that decode on the way to the MFMAs, once per 32 or 64 rows of A, are used.
+# Measured, decoding / two passes in us: 256 x 4096 x 11008 53 / 72, 512 x 4096 x
+# 4096 44 / 42, 512 x 4096 x 11008 108 / 89; 1024^3 9.0 / 11.3, 4096 x 512 x 512
+# 9.8 / 12.0, 2048 x 512 x 2048 15.9 / 14.1, 1024 x 2048 x 4096 44 / 34.
 BFP8_TWO_PASS_MIN_M = 512
 BFP4_TWO_PASS_MIN_M = 512
+TWO_PASS_MIN_MACS = 1_500_000_000
 
 
 def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> None:
@@ -609,7 +610,7 @@ def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> None:
 def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None,
                  two_pass: Optional[bool] = None) -> None:
     """c[M,N] = a[M,K] (bf16) @ dequant(bq)[K,N]; bf16 out.  `two_pass`
-    forces the path (None: by M, see BFP8_TWO_PASS_MIN_M); the two-pass
+    forces the path (None: by size, see BFP8_TWO_PASS_MIN_M); the two-pass
     workspace is the cached one of c's device and the stream."""
     _check_device(a, "matmul_bfp8w A")
     _check_device(c, "matmul_bfp8w C")
@@ -622,7 +623,8 @@ def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
     if a.stride(1) != 1 or c.stride(1) != 1:
         raise ValueError("matmul_bfp8w: A and C must be row-major")
     if two_pass is None:  # the two-pass decode reads Bq in 16-byte words
-        two_pass = M >= BFP8_TWO_PASS_MIN_M and bq.data_ptr() % 16 == 0
+        two_pass = (M >= BFP8_TWO_PASS_MIN_M and M * N * K >= TWO_PASS_MIN_MACS
+                    and bq.data_ptr() % 16 == 0)
     if not two_pass:
         _matmul_packed(a, bq, L.TTLH_BFP8, c, M, N, K, stream)
         return
@@ -667,8 +669,8 @@ def bfp4_unpack(q: torch.Tensor, rows: int, cols: int, stream=None) -> torch.Ten
 
 
 def matmul_bfp4w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None) -> None:
-    """c[M,N] = a[M,K] (bf16) @ dequant(bq)[K,N] with bfloat4_b weights; from
-    BFP4_TWO_PASS_MIN_M rows on, the dequantised weights go through a bf16
+    """c[M,N] = a[M,K] (bf16) @ dequant(bq)[K,N] with bfloat4_b weights; in large
+    products (BFP4_TWO_PASS_MIN_M) the dequantised weights go through a bf16
     workspace (the cached one of c's device and the stream)."""
     _check_device(a, "matmul_bfp4w A")
     _check_device(c, "matmul_bfp4w C")
@@ -682,8 +684,8 @@ def matmul_bfp4w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
         raise ValueError("matmul_bfp4w: A and C must be row-major")
     # (operands off their alignment go to the two passes at any M, which refuse
     # them)
-    if (M < BFP4_TWO_PASS_MIN_M and bq.data_ptr() % 8 == 0 and a.data_ptr() % 16 == 0
-            and a.stride(0) % 8 == 0):
+    if ((M < BFP4_TWO_PASS_MIN_M or M * N * K < TWO_PASS_MIN_MACS) and bq.data_ptr() % 8 == 0
+            and a.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0):
         _matmul_packed(a, bq, L.TTLH_BFP4, c, M, N, K, stream)
         return
     ws = _workspace(c.device, stream, K * N * 2)
