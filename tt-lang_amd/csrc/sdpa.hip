@@ -221,8 +221,6 @@ struct Sdpa {
     return __builtin_amdgcn_exp2f(__builtin_fmaf(v, sc, -mx));
   }
 
-  static constexpr float kLazy = 8.0f;
-
   // One KV block kb = it * GROUPS + group, if there is one: the group's next
   // block's K and V are fetched into registers while this one computes S, the
   // softmax and O += V(kb)^T P^T from the group's LDS buffer it & 1, then
@@ -234,7 +232,7 @@ struct Sdpa {
       load_rows<D, RAGGED>(p.K, base, next * BKV, stk, p.S);
       load_rows<D, RAGGED>(p.V, base, next * BKV, stv, p.S);
     }
-    if (kb < nkv) block(kb, Ks[it & 1], Vs[it & 1]);
+    if (GROUPS == 1 || kb < nkv) block(kb, Ks[it & 1], Vs[it & 1]);
     if (next < nkv) {
       store_rows<D, kKPitch<D>>(stk, Ks[(it + 1) & 1]);
       store_rows<D, kVPitch<D>>(stv, Vs[(it + 1) & 1]);
@@ -244,7 +242,11 @@ struct Sdpa {
 
   __device__ __forceinline__ void block(int kb, const uint16_t* Kc, const uint16_t* Vc) {
     f32x16 cur[2];
+    // (the wave with MFMAs goes first where the other wave of its SIMD is in its
+    // softmax: 1 x 32 x 2016 x 128 84.0 -> 81.7 us; no gain under the mask)
+    if constexpr (!CAUSAL && D == 128) __builtin_amdgcn_s_setprio(1);
     scores(Kc, cur);
+    if constexpr (!CAUSAL && D == 128) __builtin_amdgcn_s_setprio(0);
 
     // causal: only blocks that reach past this wave's first query need a
     // mask; ragged: the block that runs past the sequence end masks the kv
@@ -261,28 +263,26 @@ struct Sdpa {
           if (masked(kv)) cur[t][r] = sc >= 0.0f ? -INFINITY : INFINITY;
         }
     }
-    // block extreme of the raw scores: max if the scale is positive, else
-    // min (four chains, so that no add or max waits for all before it)
-    float e4[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) e4[c] = cur[c >> 1][8 * (c & 1)];
+    // block extreme of the raw scores: max if the scale is positive, else min
+    float ex = cur[0][0];
     if (sc >= 0.0f) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 1; r < 8; ++r) e4[c] = fmaxf(e4[c], cur[c >> 1][8 * (c & 1) + r]);
-      e4[0] = xor32_max(fmaxf(fmaxf(e4[0], e4[1]), fmaxf(e4[2], e4[3])));
+        for (int r = 0; r < 16; ++r) ex = fmaxf(ex, cur[t][r]);
+      ex = xor32_max(ex);
     } else {
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 1; r < 8; ++r) e4[c] = fminf(e4[c], cur[c >> 1][8 * (c & 1) + r]);
-      e4[0] = xor32_min(fminf(fminf(e4[0], e4[1]), fminf(e4[2], e4[3])));
+        for (int r = 0; r < 16; ++r) ex = fminf(ex, cur[t][r]);
+      ex = xor32_min(ex);
     }
-    // The running max moves, and O is rescaled, only when a lane's block max
-    // exceeds it by more than 8 (log2 units): P <= 2^8 until then.
-    const float m_blk = e4[0] * sc;
-    if (__any(m_blk > m + kLazy)) {
+    // O is rescaled only when some lane's running max moves.  (Letting it lag
+    // by up to 2^8 saves 2 to 5% of the time, but the largest probability is
+    // then no longer 1, exact in bf16: 2 to 5% more error.)
+    const float m_blk = ex * sc;
+    if (__any(m_blk > m)) {
       const float m_new = fmaxf(m, m_blk);
       const float alpha = m_new == m ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);  // 0 at first
       l *= alpha;
@@ -293,7 +293,7 @@ struct Sdpa {
     // (a lane that has seen only masked or -inf scores keeps m = -inf: its
     // exponentials are 0)
     const float mm = m == -INFINITY ? 0.0f : m;
-    float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float rs = 0.0f;
     if (diag) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -302,7 +302,7 @@ struct Sdpa {
           const int kv = kb * BKV + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
           const float e = masked(kv) ? 0.0f : expo(cur[t][r], mm);
           cur[t][r] = e;
-          r4[r & 3] += e;
+          rs += e;
         }
     } else {
 #pragma unroll
@@ -311,10 +311,10 @@ struct Sdpa {
         for (int r = 0; r < 16; ++r) {
           const float e = expo(cur[t][r], mm);
           cur[t][r] = e;
-          r4[r & 3] += e;
+          rs += e;
         }
     }
-    l += xor32_add((r4[0] + r4[1]) + (r4[2] + r4[3]));
+    l += xor32_add(rs);
 
     // P^T operands: chunk c (16 kv) = tile c/2, accumulators 8(c%2) .. +8
     bf16x8 pb[4];
@@ -328,6 +328,7 @@ struct Sdpa {
       w.w = pk_bf16(cur[t][r0 + 6], cur[t][r0 + 7]);
       pb[c] = __builtin_bit_cast(bf16x8, w);
     }
+    if constexpr (!CAUSAL) __builtin_amdgcn_s_setprio(1);
     // O^T += V^T P^T; the V^T operand of lane (d = 32j + l32, h) holds kv
     // {16c + 4h + i, 16c + 4h + 8 + i}
 #pragma unroll
@@ -342,6 +343,7 @@ struct Sdpa {
                                                        0, 0, 0);
       }
     }
+    if constexpr (!CAUSAL) __builtin_amdgcn_s_setprio(0);
   }
 };
 
@@ -967,9 +969,9 @@ int launch(SdpaArgs a, hipStream_t s) {
   // Two groups of waves: up to one workgroup per CU, and under the causal mask
   // up to two rounds of long blocks, whose shares of a CU would differ most (512
   // blocks of S = 2016: 62 us against 69; of S = 480: 28 against 24; 384
-  // blocks without the mask: 84 against 72).  Two KV blocks do not pay for the
-  // second group.
-  const bool two = a.S > 128 && (blocks <= 256 || (CAUSAL && blocks <= 512 && a.S >= 1024));
+  // blocks without the mask: 84 against 72).  Three KV blocks do not pay for
+  // the second group.
+  const bool two = a.S > 192 && (blocks <= 256 || (CAUSAL && blocks <= 512 && a.S >= 1024));
   const dim3 grid(static_cast<uint32_t>(blocks));
   const bool ragged = a.S % BQ != 0;  // S % 32 == 0 only
   if (two && ragged)
