@@ -13,6 +13,7 @@ import torch
 from oracle import bfp8 as OB
 from oracle import tile_ops as O
 from ttlhip import _lib as L
+from ttlhip import expr as X
 from ttlhip import kernels as Kn
 
 pytestmark = pytest.mark.gpu
@@ -75,6 +76,20 @@ def test_bf16_blocks_of_128(K):
     f0 = f.clone()
     Kn.matmul(a, b, f, accumulate=True)
     _check(f - f0, a, b, False)
+
+
+@pytest.mark.parametrize("M,K,N", [(4096, 32, 3072), (4096, 96, 3104), (32, 64, 49152)])
+def test_sums_in_the_fused_epilogues_order(M, K, N):
+    # problems that the fused epilogue takes give the same bits with and
+    # without it, whichever kernel runs the plain product
+    a, b = _operands(M, K, N, 19)
+    c = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    Kn.matmul(a, b, c)
+    leaf = X.Leaf(0, torch.bfloat16)
+    prog = X.compile_expr(X.Unary("relu", leaf, torch.bfloat16))
+    d = torch.zeros_like(c)
+    Kn.matmul_eltwise(a, b, prog, [None] * len(prog.steps), 0, d, (0, 0, M, N))
+    assert torch.equal(d, torch.relu(c))
 
 
 def test_bf16_blocks_of_128_with_slow_operand_loads():

@@ -2073,7 +2073,12 @@ int matmul_with(const void* A, int a_dtype, int64_t lda, const void* B, int b_dt
     a.c_dtype = c_dtype;
     a.accumulate = accumulate ? 1 : 0;
     const LdsTimes lds = lds_times(a);
-    if (launch_direct_bf16(d, std::min({lds.dma, lds.mid, lds.reg}), scratch, s, &status))
+    // Problems that ttlh_matmul_eltwise takes (>= 192 blocks of 256x256) stay with
+    // the kernels that add in its order, so that its results are those of the
+    // separate launches bit for bit.
+    const int64_t b256 = ((M + LM - 1) / LM) * ((N + LN - 1) / LN);
+    if (b256 < 192 &&
+        launch_direct_bf16(d, std::min({lds.dma, lds.mid, lds.reg}), scratch, s, &status))
       return status;
     if (lds.dma <= lds.mid && launch_dma(a, s, &status)) return status;
     if (launch_mid(a, s, &status)) return status;
