@@ -6,6 +6,7 @@ as for the other GEMM kernels: fp32 sums of K products (1e-6 sqrt(K) of the
 largest result) and, for bf16 results, one rounding (2^-8 of the value)."""
 
 import math
+import threading
 
 import pytest
 import torch
@@ -165,6 +166,51 @@ def test_divided_product_under_capture_and_on_two_streams():
     Kn.release_workspaces()
     Kn.matmul(a, b, c)
     _check(c, a, b, True)
+
+
+def test_scratch_of_a_stream_while_another_thread_captures():
+    # the first product of a stream takes its scratch; that allocation ends
+    # neither in an error nor with the other thread's (global mode) capture
+    a, b = _operands(32, 4096, 256, 11)
+    c, d = (torch.zeros(32, 256, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    Kn.matmul(a, b, c)
+    Kn.release_workspaces()
+    side, errors = torch.cuda.Stream(), []
+
+    def first_product():
+        try:
+            Kn.matmul(a, b, c, stream=side)
+        except Exception as e:  # reported by the main thread
+            errors.append(e)
+
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        Kn.matmul(a, b, d)
+        t = threading.Thread(target=first_product)
+        t.start()
+        t.join()
+    assert not errors, errors
+    g.replay()
+    torch.cuda.synchronize()
+    _check(c, a, b, True)
+    _check(d, a, b, True)
+
+
+def test_scratches_are_bounded(monkeypatch):
+    monkeypatch.setattr(Kn, "_MATMUL_SCRATCH_MAX", 2)
+    Kn.release_workspaces()
+    a, b = _operands(32, 4096, 256, 13)
+    outs = [torch.zeros(32, 256, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+    streams = [torch.cuda.Stream() for _ in outs]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for s, o in zip(streams, outs):
+            Kn.matmul(a, b, o, stream=s)
+            assert len(Kn._MATMUL_SCRATCH) <= 2
+    torch.cuda.synchronize()
+    for o in outs:
+        _check(o, a, b, True)
 
 
 def _packed(w, bits):

@@ -7,7 +7,11 @@
 // (examples/metal_examples/singlecore_matmul/metal/kernels/mm_compute.cpp:28-68,
 // mm_reader.cpp:8-55; blocked variant bmm_large_block_zm.cpp:41-120).
 //
-// MI355X design (bf16):
+// MI355X design.  Which kernel takes a problem is in lds_times and matmul_with
+// below: mm_dma_kernel (256x256 blocks) and mm_mid_kernel (128x128), both fed
+// through LDS by direct-to-LDS loads; the register-direct kernels of
+// matmul_direct.hip for results that do not fill the chip in such blocks; and
+// for operands or results that none of these can address, mm_bf16_kernel:
 //  - one workgroup computes a 128x128 output block (4x4 tiles of 32x32), four
 //    waves in a 2x2 arrangement, each owning 64x64 = 2x2 MFMA tiles of
 //    v_mfma_f32_32x32x16_bf16 with fp32 accumulators (64 per lane);
@@ -24,7 +28,9 @@
 //    regrouped to give each XCD a compact band of output blocks whose A rows
 //    and B columns stay in that XCD's L2;
 //  - the epilogue rounds once to the output dtype (RNE).
-// fp32 inputs take a simpler v_mfma_f32_32x32x2f32 kernel (64x64 blocks).
+// fp32 inputs that the register-direct kernels do not take (operands off their
+// 16- or 8-byte alignment) run a simpler v_mfma_f32_32x32x2f32 kernel (64x64
+// blocks).
 
 #include <algorithm>
 #include <atomic>

@@ -10,6 +10,7 @@ missing GPU raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import functools
 import os
@@ -219,6 +220,21 @@ def synchronize() -> None:
         torch._C._cuda_synchronize()
     else:
         torch.cuda.synchronize()
+
+
+@contextlib.contextmanager
+def relaxed_capture():
+    """Lets this thread allocate while another one captures a graph in the
+    global mode (torch's default), where a hipMalloc anywhere in the process
+    would otherwise end that capture with an error."""
+    exchange = load().hipThreadExchangeStreamCaptureMode  # of the HIP runtime it links
+    mode = C.c_int(2)  # hipStreamCaptureModeRelaxed
+    status = exchange(C.byref(mode))
+    try:
+        yield
+    finally:
+        if status == 0:
+            exchange(C.byref(mode))  # back to the mode it was
 
 
 _DTYPE_CODES = {torch.bfloat16: TTLH_BF16, torch.float32: TTLH_F32}

@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes as C
 import functools
 import struct
+import threading
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -72,9 +73,13 @@ def _workspace(device: torch.device, stream, nbytes: int,
 
 # The matmul's scratch (partial sums of products that divide K among several
 # workgroups, and their counters): a fixed 4 MiB per (device, stream), zeroed
-# once and left to the library.  Never allocated while the stream is being
-# captured; the library does not use it there either, so no graph holds it.
+# once and left to the library; the oldest goes back to the allocator when a
+# 65th stream asks (torch itself hands out 32 per device).  Never allocated while
+# the stream is being captured; the library does not use it there either, so no
+# graph holds it.
 _MATMUL_SCRATCH: dict = {}
+_MATMUL_SCRATCH_MAX = 64
+_MATMUL_SCRATCH_LOCK = threading.Lock()
 
 
 def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Tensor]:
@@ -84,11 +89,16 @@ def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Ten
         s = stream if stream is not None else torch.cuda.current_stream()
         if s.device.index != device.index:
             return None  # the zeroing would not be ordered before the launch
-        with torch.cuda.stream(s):
-            if torch.cuda.is_current_stream_capturing():
-                return None
-            t = torch.zeros(L.MATMUL_SCRATCH_BYTES, dtype=torch.uint8, device=device)
-        t = _MATMUL_SCRATCH.setdefault(key, t)
+        with _MATMUL_SCRATCH_LOCK, torch.cuda.stream(s):
+            t = _MATMUL_SCRATCH.get(key)
+            if t is None:
+                if torch.cuda.is_current_stream_capturing():
+                    return None
+                with L.relaxed_capture():
+                    t = torch.zeros(L.MATMUL_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+                while len(_MATMUL_SCRATCH) >= _MATMUL_SCRATCH_MAX:
+                    del _MATMUL_SCRATCH[next(iter(_MATMUL_SCRATCH))]
+                _MATMUL_SCRATCH[key] = t
     return t
 
 
@@ -96,7 +106,8 @@ def release_workspaces() -> None:
     """Drop the cached workspaces (their memory returns to torch's caching
     allocator once the work queued on them has finished)."""
     _WORKSPACES.clear()
-    _MATMUL_SCRATCH.clear()
+    with _MATMUL_SCRATCH_LOCK:
+        _MATMUL_SCRATCH.clear()
 
 
 def _axis_range(lo: int, n: int, mask: int, off: int):
