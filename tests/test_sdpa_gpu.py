@@ -275,3 +275,17 @@ def test_sdpa_scores_of_minus_infinity(S):
     keep = torch.isfinite(k[0, 0, :, 3])
     ref = O.sdpa_ref(q, k[:, :, keep], v[:, :, keep], 0.09)
     _check(got, ref)
+
+
+@pytest.mark.parametrize("S", [96, 480])
+@pytest.mark.parametrize("D", [64, 128])
+def test_sdpa_infinite_value_in_a_ragged_last_row(S, D):
+    # the rows past the sequence are zeros, not copies of its last one: that
+    # row's infinity reaches its column once, and never as 0 * inf
+    q, k, v = _qkv(1, 2, S, D, 19)
+    ref = O.sdpa_ref(q, k, v, 0.09)
+    v[:, :, S - 1, 5] = float("inf")
+    got = _run(q, k, v, 0.09)
+    assert bool((got[..., 5] == float("inf")).all())
+    rest = [d for d in range(D) if d != 5]
+    _check(got[..., rest], ref[..., rest])

@@ -35,8 +35,10 @@
 //    fewer, a CU would hold one group with nothing to hide its latencies, so
 //    two groups share the workgroup's queries, taking the even and the odd KV
 //    blocks, and their results meet in LDS: 1 x 8 x 4000 x 128 causal 107 ->
-//    76 us, 1 x 16 x 992 x 128 31 -> 24.  Either is bound by the latencies of
-//    its chain S -> softmax -> O (40% of the MFMA time of a block is waiting).
+//    72 us, 1 x 16 x 992 x 128 31 -> 23.5.  Either is bound by the latencies of
+//    its chain S -> softmax -> O; the staging of K and V through registers is a
+//    quarter (1 x 32 x 2048 x 128 causal 50 us: 44 without the loads, 39 without
+//    the LDS stores as well).
 //    A third kernel, which ran the two groups in ping-pong over 256 queries, was
 //    slower than these in every case it took (1 x 32 x 2048 x 128 causal 71 us
 //    against 58, 4 x 32 x 4096 x 64 682 against 646).
@@ -117,24 +119,34 @@ constexpr int kKPitch = D + 8;   // K rows in LDS (elements)
 template <int D>
 constexpr int kVPitch = D + 32;  // V rows in LDS (elements)
 
-// K or V rows kv0 .. kv0 + 63 as 16-byte chunks, D / 32 per thread; with
-// RAGGED, rows from `end` on (past the sequence) read as zeros
+// K or V rows kv0 .. kv0 + 63 as 16-byte chunks, D / 32 per thread.  With
+// RAGGED, the rows from `end` on (past the sequence) read row end - 1 and are
+// zeroed when they are stored: no condition stands around a load (1 x 32 x 2016
+// x 128 causal 54.9 -> 52.9 us, 1 x 32 x 2016 x 64 51.3 -> 47.2; a second,
+// unconditional copy of the loads for whole blocks was slower, 58).
 template <int D, bool RAGGED = false>
 __device__ __forceinline__ void load_rows(const uint16_t* X, int64_t base, int kv0, u32x4 (&r)[D / 32],
                                           int end = 0) {
   const int t = threadIdx.x & (kThreads - 1);
   constexpr int kChunksPerRow = D / 8;
+  const uintptr_t block = reinterpret_cast<uintptr_t>(X + base + static_cast<int64_t>(kv0) * D);
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) {
     const int c = t + i * kThreads;
-    const int row = c / kChunksPerRow, dc = (c % kChunksPerRow) * 8;
-    if (RAGGED && kv0 + row >= end) {
-      r[i] = u32x4{0u, 0u, 0u, 0u};
-      continue;
-    }
-    r[i] = *reinterpret_cast<gu32x4*>(
-        reinterpret_cast<uintptr_t>(X + base + static_cast<int64_t>(kv0 + row) * D + dc));
+    int row = c / kChunksPerRow;
+    if (RAGGED) row = min(row, end - 1 - kv0);
+    const uint32_t off = (row * D + (c % kChunksPerRow) * 8) * 2;
+    r[i] = *reinterpret_cast<gu32x4*>(block + off);
   }
+}
+
+// rows `rows` .. 63 of a block as zeros
+template <int D>
+__device__ __forceinline__ void zero_rows(u32x4 (&r)[D / 32], int rows) {
+  const int t = threadIdx.x & (kThreads - 1);
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+    if ((t + i * kThreads) / (D / 8) >= rows) r[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
 template <int D, int PITCH>
@@ -202,17 +214,31 @@ struct Sdpa {
   float m, l;
   u32x4 stk[D / 32], stv[D / 32];  // K and V rows of the next block
 
-  // S^T = K Q^T for the K block at K_ (raw scores)
+  // S^T = K Q^T for the K block at K_ (raw scores).  The K fragments are read
+  // kAhead before the MFMA that takes them, into the registers that hold the
+  // exponentials later; the scheduling fences keep the compiler from sinking the
+  // reads to their uses, where each pair waits for the LDS (2% under the mask;
+  // eight ahead no faster, and 5% slower at 4 x 32 x 2048 x 64).
   __device__ __forceinline__ void scores(const uint16_t* K_, f32x16 (&sv)[2]) {
+    constexpr int kAhead = 4;
+    const uint16_t* row = K_ + l32 * kKPitch<D> + 8 * h;
+    const auto frag = [&](int i) {
+      return *reinterpret_cast<const bf16x8*>(row + (i / NDC) * 32 * kKPitch<D> + (i % NDC) * 16);
+    };
+    bf16x8 f[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) f[i] = frag(i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) sv[t][r] = 0.0f;
 #pragma unroll
       for (int dc = 0; dc < NDC; ++dc) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(K_ + (32 * t + l32) * kKPitch<D> +
-                                                          dc * 16 + 8 * h);
-        sv[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qop[dc], sv[t], 0, 0, 0);
+        const int i = t * NDC + dc;
+        sv[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i % kAhead], qop[dc], sv[t], 0, 0, 0);
+        if (i + kAhead < 2 * NDC) f[i % kAhead] = frag(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
@@ -232,8 +258,15 @@ struct Sdpa {
       load_rows<D, RAGGED>(p.K, base, next * BKV, stk, p.S);
       load_rows<D, RAGGED>(p.V, base, next * BKV, stv, p.S);
     }
-    if (GROUPS == 1 || kb < nkv) block(kb, Ks[it & 1], Vs[it & 1]);
+    // (causal: the last KV block of a workgroup lies wholly past the queries of
+    // its waves 0 and 1)
+    if ((GROUPS == 1 || kb < nkv) && (!CAUSAL || kb * BKV <= qb * BQ + wave * 32 + 31))
+      block(kb, Ks[it & 1], Vs[it & 1]);
     if (next < nkv) {
+      if (RAGGED && next * BKV + BKV > p.S) {
+        zero_rows<D>(stk, p.S - next * BKV);
+        zero_rows<D>(stv, p.S - next * BKV);
+      }
       store_rows<D, kKPitch<D>>(stk, Ks[(it + 1) & 1]);
       store_rows<D, kVPitch<D>>(stv, Vs[(it + 1) & 1]);
     }
@@ -314,7 +347,7 @@ struct Sdpa {
           rs += e;
         }
     }
-    l += xor32_add(rs);
+    l += rs;  // of this lane's kv: the two halves, whose m is one, meet at the end
 
     // P^T operands: chunk c (16 kv) = tile c/2, accumulators 8(c%2) .. +8
     bf16x8 pb[4];
@@ -390,6 +423,10 @@ __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r) w.o[j][r] = 0.0f;
   if (group < w.nkv) {
+    if (RAGGED && group * BKV + BKV > p.S) {
+      zero_rows<D>(w.stk, p.S - group * BKV);
+      zero_rows<D>(w.stv, p.S - group * BKV);
+    }
     store_rows<D, kKPitch<D>>(w.stk, w.Ks[0]);
     store_rows<D, kVPitch<D>>(w.stv, w.Vs[0]);
   }
@@ -431,7 +468,7 @@ __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel
   if (RAGGED && w.q >= p.S) return;  // wave-uniform (S % 32 == 0); no barrier follows
 
   // O[q][d], d = 32j + 8u + 4h + i: four contiguous bf16 per (j, u)
-  const float inv = 1.0f / w.l;
+  const float inv = 1.0f / xor32_add(w.l);
   uint16_t* orow = p.O + w.base + static_cast<int64_t>(w.q) * D;
 #pragma unroll
   for (int j = 0; j < D / 32; ++j)
