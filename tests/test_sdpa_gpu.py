@@ -289,3 +289,11 @@ def test_sdpa_infinite_value_in_a_ragged_last_row(S, D):
     assert bool((got[..., 5] == float("inf")).all())
     rest = [d for d in range(D) if d != 5]
     _check(got[..., rest], ref[..., rest])
+
+
+@pytest.mark.parametrize("S,D,causal", [(224, 128, True), (416, 64, False), (160, 64, True),
+                                        (480, 128, False)])
+def test_sdpa_ragged_forms_with_slow_loads(S, D, causal):
+    # one and two groups, the last block half past the sequence: its zeros are
+    # written after its loads have landed, however late those are
+    test_sdpa_other_kernels_with_slow_loads(S, D, causal)

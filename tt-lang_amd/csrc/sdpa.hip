@@ -35,21 +35,23 @@
 //    fewer, a CU would hold one group with nothing to hide its latencies, so
 //    two groups share the workgroup's queries, taking the even and the odd KV
 //    blocks, and their results meet in LDS: 1 x 8 x 4000 x 128 causal 107 ->
-//    72 us, 1 x 16 x 992 x 128 31 -> 23.5.  Either is bound by the latencies of
-//    its chain S -> softmax -> O; the staging of K and V through registers is a
-//    quarter (1 x 32 x 2048 x 128 causal 50 us: 44 without the loads, 39 without
-//    the LDS stores as well).
+//    66 us, 1 x 16 x 992 x 128 31 -> 22.5.  Either is bound by the latencies of
+//    its chain S -> softmax -> O.  K and V come by direct-to-LDS loads: through
+//    registers and LDS stores they took a quarter of the time (1 x 32 x 2048 x 128
+//    causal, with nothing to load or store 39 of 50 us); 4 x 32 x 4096 x 128 causal
+//    663 -> 615 us, 4 x 32 x 4096 x 64 647 -> 614.
 //    A third kernel, which ran the two groups in ping-pong over 256 queries, was
 //    slower than these in every case it took (1 x 32 x 2048 x 128 causal 71 us
 //    against 58, 4 x 32 x 4096 x 64 682 against 646).
 //
-// K and V are staged in LDS as loaded (row-major, 16-byte stores).  gfx950's
-// LDS serves 256 bytes (64 banks) per cycle: a ds_read_b128 is conflict-free
-// when each 16 lanes hit 16 distinct 16-byte bank groups, a ds_read_b64 when
-// each 32 lanes do.  Row pitches of D + 8 (K: 16 rows, one chunk each) and
-// D + 32 elements (V: 4 rows x 4 chunks per 32 lanes of a transpose read)
-// meet that.  The next block's K and V are fetched into registers while the
-// current block computes.
+// K and V lie in LDS row-major and unpadded (a direct-to-LDS load writes 64 x 16
+// consecutive bytes), the 16-byte chunks of a row permuted.  gfx950's LDS serves
+// 256 bytes (64 banks) per cycle: a ds_read_b128 is conflict-free when each 16
+// lanes hit 16 distinct 16-byte bank groups, a ds_read_b64 when each 32 lanes do.
+// K (16 rows, one chunk each): chunk c of row r at c ^ (r & 15), for D = 64, where
+// two rows share the banks, at c ^ ((r >> 1) & 7); V (4 rows x 4 chunks per 32
+// lanes of a transpose read): at c ^ 4 (r & 3), for D = 64 at c ^ 4 ((r >> 1) & 1).
+// The next block's loads run while the current block computes.
 // Softmax runs in the log2 domain: exp2(fma(s, scale log2 e, -m)) in
 // sdpa_fwd_kernel, with the block max taken on the raw scores (sign of the
 // scale handled by taking the min instead); the causal mask touches only the blocks
@@ -68,7 +70,6 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef const __attribute__((address_space(1))) u32x4 gu32x4;
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
@@ -114,59 +115,22 @@ __device__ __forceinline__ float xor32_add(float x) {
 // s_waitcnt immediate (gfx9 encoding): at most n global loads outstanding
 constexpr int vmcnt_imm_sdpa(int n) { return 0x0F70 | (n & 0xF) | ((n >> 4) << 14); }
 
-template <int D>
-constexpr int kKPitch = D + 8;   // K rows in LDS (elements)
-template <int D>
-constexpr int kVPitch = D + 32;  // V rows in LDS (elements)
+typedef __attribute__((address_space(3))) void lds_void;
 
-// K or V rows kv0 .. kv0 + 63 as 16-byte chunks, D / 32 per thread.  With
-// RAGGED, the rows from `end` on (past the sequence) read row end - 1 and are
-// zeroed when they are stored: no condition stands around a load (1 x 32 x 2016
-// x 128 causal 54.9 -> 52.9 us, 1 x 32 x 2016 x 64 51.3 -> 47.2; a second,
-// unconditional copy of the loads for whole blocks was slower, 58).
-template <int D, bool RAGGED = false>
-__device__ __forceinline__ void load_rows(const uint16_t* X, int64_t base, int kv0, u32x4 (&r)[D / 32],
-                                          int end = 0) {
-  const int t = threadIdx.x & (kThreads - 1);
-  constexpr int kChunksPerRow = D / 8;
-  const uintptr_t block = reinterpret_cast<uintptr_t>(X + base + static_cast<int64_t>(kv0) * D);
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    const int c = t + i * kThreads;
-    int row = c / kChunksPerRow;
-    if (RAGGED) row = min(row, end - 1 - kv0);
-    const uint32_t off = (row * D + (c % kChunksPerRow) * 8) * 2;
-    r[i] = *reinterpret_cast<gu32x4*>(block + off);
-  }
-}
-
-// rows `rows` .. 63 of a block as zeros
-template <int D>
-__device__ __forceinline__ void zero_rows(u32x4 (&r)[D / 32], int rows) {
-  const int t = threadIdx.x & (kThreads - 1);
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i)
-    if ((t + i * kThreads) / (D / 8) >= rows) r[i] = u32x4{0u, 0u, 0u, 0u};
-}
-
-template <int D, int PITCH>
-__device__ __forceinline__ void store_rows(const u32x4 (&r)[D / 32], uint16_t* dst) {
-  const int t = threadIdx.x & (kThreads - 1);
-  constexpr int kChunksPerRow = D / 8;
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    const int c = t + i * kThreads;
-    const int row = c / kChunksPerRow, dc = (c % kChunksPerRow) * 8;
-    *reinterpret_cast<u32x4*>(dst + row * PITCH + dc) = r[i];
-  }
-}
-
-// 4 consecutive kv rows (from kv0) of column d0 + (lane & 15) of V, as 4
-// bf16 (see the transpose-load rule above)
-template <int D>
-__device__ __forceinline__ i16x4 read_v4(const uint16_t* Vs, int kv0, int d0, int lane) {
-  const uint16_t* a = Vs + (kv0 + ((lane & 15) >> 2)) * kVPitch<D> + d0 + 4 * (lane & 3);
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)a);
+// One direct-to-LDS load per lane: its 16 bytes at byte `off` from the uniform
+// `src` land at the uniform `lds` + 16 lane.  Inline asm, waited for explicitly:
+// the compiler would wait for every LDS read while one it knows of is in flight.
+__device__ __forceinline__ void dma16(uint64_t src, uint32_t off, uint32_t lds) {
+  const uint64_t g =
+      (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(src >> 32)))) << 32) |
+      uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(src))));
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(g)
+      : "memory", "m0");
 }
 
 // the block's queries: q blocks of one (b, h) are kept on one XCD
@@ -204,26 +168,82 @@ struct Sdpa {
   static constexpr int NDC = D / 16;  // 16-wide d chunks of the S^T contraction
 
   const SdpaArgs& p;
-  uint16_t (*Ks)[BKV * kKPitch<D>];
-  uint16_t (*Vs)[BKV * kVPitch<D>];
+  uint16_t (*Ks)[BKV * D];
+  uint16_t (*Vs)[BKV * D];
   int64_t base;
   int qb, wave, lane, l32, h, q, nkv;
   float sc;
   bf16x8 qop[NDC];
   f32x16 o[ND];
   float m, l;
-  u32x4 stk[D / 32], stv[D / 32];  // K and V rows of the next block
+  int row0, k_src, v_src;   // DMA: the thread's first row; its chunks' elements in a row
+  int k_frag, v_frag[ND];   // LDS elements of the K and V fragment reads
+
+  static constexpr int kChunks = D / 8;                // 16-byte chunks in a row
+  static constexpr int kRowsPer = kThreads / kChunks;  // rows that one DMA of the group covers
+  // position of chunk c of row r: c ^ k_swz(r) in K, c ^ v_swz(r) in V
+  static __device__ __forceinline__ int k_swz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
+  static __device__ __forceinline__ int v_swz(int r) {
+    return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+  }
+
+  __device__ __forceinline__ void setup() {
+    const int t = threadIdx.x & (kThreads - 1);
+    row0 = t / kChunks;
+    k_src = ((t % kChunks) ^ k_swz(row0)) * 8;
+    v_src = ((t % kChunks) ^ v_swz(row0)) * 8;
+    k_frag = l32 * D + ((h ^ k_swz(l32)) << 3);
+    const int vr = (lane & 15) >> 2;
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const int chunk = 4 * j + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+      v_frag[j] = (4 * h + vr) * D + ((chunk ^ v_swz(vr)) << 3) + 4 * (lane & 1);
+    }
+  }
+
+  // rows kb * 64 .. + 63 of X into an LDS buffer; with RAGGED, rows past the
+  // sequence are its last row again
+  __device__ __forceinline__ void dma(const uint16_t* X, int chunk, int kb, const uint16_t* buf) {
+    const uint64_t src = reinterpret_cast<uint64_t>(X + base + static_cast<int64_t>(kb) * BKV * D);
+    const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)buf));
+#pragma unroll
+    for (int i = 0; i < BKV / kRowsPer; ++i) {
+      int row = row0 + i * kRowsPer;
+      if (RAGGED) row = min(row, p.S - 1 - kb * BKV);
+      dma16(src, static_cast<uint32_t>(row * D + chunk) * 2u, lds + i * kThreads * 16 + wave * 1024);
+    }
+  }
+
+  // The loads of block kb have landed; with RAGGED, the V rows past the sequence
+  // become zeros (each thread's own chunks), so that 0 * V is 0 there.  (The
+  // scores of such K rows are masked.)
+  __device__ __forceinline__ void landed(int kb, uint16_t* Vb) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm_sdpa(0));
+    asm volatile("" ::: "memory");
+    if (RAGGED && kb * BKV + BKV > p.S) {
+      const int t = threadIdx.x & (kThreads - 1);
+#pragma unroll
+      for (int i = 0; i < BKV / kRowsPer; ++i)
+        if (kb * BKV + row0 + i * kRowsPer >= p.S)
+          *reinterpret_cast<u32x4*>(Vb + (i * kThreads + t) * 8) = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+
+  // 4 consecutive kv rows of one d column each of V's tile j (see the
+  // transpose-load rule above), from row kv + 4 h
+  __device__ __forceinline__ i16x4 read_v4(const uint16_t* Vb, int kv, int j) const {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(Vb + v_frag[j] + kv * D));
+  }
 
   // S^T = K Q^T for the K block at K_ (raw scores).  The K fragments are read
   // kAhead before the MFMA that takes them, into the registers that hold the
   // exponentials later; the scheduling fences keep the compiler from sinking the
   // reads to their uses, where each pair waits for the LDS (2% under the mask;
-  // eight ahead no faster, and 5% slower at 4 x 32 x 2048 x 64).
+  // eight ahead no faster).
   __device__ __forceinline__ void scores(const uint16_t* K_, f32x16 (&sv)[2]) {
     constexpr int kAhead = 4;
-    const uint16_t* row = K_ + l32 * kKPitch<D> + 8 * h;
     const auto frag = [&](int i) {
-      return *reinterpret_cast<const bf16x8*>(row + (i / NDC) * 32 * kKPitch<D> + (i % NDC) * 16);
+      return *reinterpret_cast<const bf16x8*>(K_ + (k_frag ^ ((i % NDC) * 16)) + (i / NDC) * 32 * D);
     };
     bf16x8 f[kAhead];
 #pragma unroll
@@ -248,28 +268,21 @@ struct Sdpa {
   }
 
   // One KV block kb = it * GROUPS + group, if there is one: the group's next
-  // block's K and V are fetched into registers while this one computes S, the
-  // softmax and O += V(kb)^T P^T from the group's LDS buffer it & 1, then
-  // stored into the other buffer (last read before the previous barrier).
+  // block's K and V are on their way to the other LDS buffer (last read before
+  // the previous barrier) while this one computes S, the softmax and
+  // O += V(kb)^T P^T from buffer it & 1.
   template <int GROUPS>
   __device__ __forceinline__ void step(int it, int group) {
     const int kb = it * GROUPS + group, next = kb + GROUPS;
     if (next < nkv) {
-      load_rows<D, RAGGED>(p.K, base, next * BKV, stk, p.S);
-      load_rows<D, RAGGED>(p.V, base, next * BKV, stv, p.S);
+      dma(p.K, k_src, next, Ks[(it + 1) & 1]);
+      dma(p.V, v_src, next, Vs[(it + 1) & 1]);
     }
     // (causal: the last KV block of a workgroup lies wholly past the queries of
     // its waves 0 and 1)
     if ((GROUPS == 1 || kb < nkv) && (!CAUSAL || kb * BKV <= qb * BQ + wave * 32 + 31))
       block(kb, Ks[it & 1], Vs[it & 1]);
-    if (next < nkv) {
-      if (RAGGED && next * BKV + BKV > p.S) {
-        zero_rows<D>(stk, p.S - next * BKV);
-        zero_rows<D>(stv, p.S - next * BKV);
-      }
-      store_rows<D, kKPitch<D>>(stk, Ks[(it + 1) & 1]);
-      store_rows<D, kVPitch<D>>(stv, Vs[(it + 1) & 1]);
-    }
+    if (next < nkv) landed(next, Vs[(it + 1) & 1]);
     __syncthreads();
   }
 
@@ -284,6 +297,21 @@ struct Sdpa {
     // causal: only blocks that reach past this wave's first query need a
     // mask; ragged: the block that runs past the sequence end masks the kv
     // beyond it (masked scores drop out of the block extreme and get exp 0)
+    // the V^T operand i of lane (d = 32j + l32, h), j = i % ND, holds kv
+    // {16c + 4h + i, 16c + 4h + 8 + i}, c = i / ND; the first ones are read here,
+    // under the softmax
+    const auto vfrag = [&](int i) {
+      const i16x4 lo = read_v4(Vc, 16 * (i / ND), i % ND);
+      const i16x4 hi = read_v4(Vc, 16 * (i / ND) + 8, i % ND);
+      const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      return __builtin_bit_cast(bf16x8, w);
+    };
+    constexpr int kAhead = 4;
+    bf16x8 vf[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) vf[i] = vfrag(i);
+    __builtin_amdgcn_sched_barrier(0);
+
     const bool diag = (CAUSAL && kb * BKV + BKV - 1 > qb * BQ + wave * 32) ||
                       (RAGGED && kb * BKV + BKV > p.S);
     auto masked = [&](int kv) { return (CAUSAL && kv > q) || (RAGGED && kv >= p.S); };
@@ -362,19 +390,14 @@ struct Sdpa {
       pb[c] = __builtin_bit_cast(bf16x8, w);
     }
     if constexpr (!CAUSAL) __builtin_amdgcn_s_setprio(1);
-    // O^T += V^T P^T; the V^T operand of lane (d = 32j + l32, h) holds kv
-    // {16c + 4h + i, 16c + 4h + 8 + i}
+    // O^T += V^T P^T, one chunk of 16 kv after the other, so that consecutive
+    // MFMAs are independent
 #pragma unroll
-    for (int j = 0; j < ND; ++j) {
-      const int d0 = 32 * j + 16 * ((lane >> 4) & 1);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const i16x4 lo = read_v4<D>(Vc, 16 * c + 4 * h, d0, lane);
-        const i16x4 hi = read_v4<D>(Vc, 16 * c + 4 * h + 8, d0, lane);
-        const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), pb[c], o[j],
-                                                       0, 0, 0);
-      }
+    for (int i = 0; i < 4 * ND; ++i) {
+      o[i % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % kAhead], pb[i / ND], o[i % ND], 0,
+                                                          0, 0);
+      if (i + kAhead < 4 * ND) vf[i % kAhead] = vfrag(i + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!CAUSAL) __builtin_amdgcn_s_setprio(0);
   }
@@ -386,10 +409,10 @@ struct Sdpa {
 // The last KV block reads rows past S as zeros and masks their scores.
 template <int D, bool CAUSAL, bool RAGGED, int GROUPS>
 __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel(const SdpaArgs p) {
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[GROUPS][2][BKV * kKPitch<D>];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[GROUPS][2][BKV * kVPitch<D>];
+  // K, then V, of each group, two buffers each
+  __shared__ __attribute__((aligned(256))) uint16_t KV[2 * GROUPS][2][BKV * D];
   const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-  Sdpa<D, CAUSAL, RAGGED> w{p, Ks[group], Vs[group]};
+  Sdpa<D, CAUSAL, RAGGED> w{p, KV[group], KV[GROUPS + group]};
   int bh;
   ordered_block<CAUSAL>(p, bh, w.qb);
   w.lane = threadIdx.x & 63;
@@ -409,10 +432,11 @@ __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel
   }
   const int qload = RAGGED ? min(w.q, p.S - 1) : w.q;  // a wave past S reads a valid row
 
+  w.setup();
   // prologue: the group's first K and V block into LDS; Q^T into VGPRs
   if (group < w.nkv) {
-    load_rows<D, RAGGED>(p.K, w.base, group * BKV, w.stk, p.S);
-    load_rows<D, RAGGED>(p.V, w.base, group * BKV, w.stv, p.S);
+    w.dma(p.K, w.k_src, group, w.Ks[0]);
+    w.dma(p.V, w.v_src, group, w.Vs[0]);
   }
 #pragma unroll
   for (int dc = 0; dc < D / 16; ++dc)
@@ -422,18 +446,10 @@ __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel
   for (int j = 0; j < D / 32; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) w.o[j][r] = 0.0f;
-  if (group < w.nkv) {
-    if (RAGGED && group * BKV + BKV > p.S) {
-      zero_rows<D>(w.stk, p.S - group * BKV);
-      zero_rows<D>(w.stv, p.S - group * BKV);
-    }
-    store_rows<D, kKPitch<D>>(w.stk, w.Ks[0]);
-    store_rows<D, kVPitch<D>>(w.stv, w.Vs[0]);
-  }
-  // Q^T must have landed before the loop: otherwise the compiler, merging
-  // the first iteration's state (Q loads in flight) with later ones, makes
-  // every S MFMA of every block wait on the next block's K/V prefetch
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  // (the wait for K and V is one for Q^T too: Q^T must have landed before the
+  // loop, or its MFMAs would wait for the next block's K and V every time)
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm_sdpa(0));
+  if (group < w.nkv) w.landed(group, w.Vs[0]);
   __syncthreads();
 
   const int steps = (w.nkv + GROUPS - 1) / GROUPS;
@@ -443,8 +459,8 @@ __global__ __launch_bounds__(kThreads * GROUPS, 2 / GROUPS) void sdpa_fwd_kernel
     // Group 1 leaves its max, sum and O in LDS (every group is past its last
     // read of K and V); group 0's wave w, which holds the same queries in the
     // same lanes as wave w + 4, adds them.
-    float* part = reinterpret_cast<float*>(&Ks[0][0][0]) + (w.wave * (16 * (D / 32) + 2)) * 64 + w.lane;
-    static_assert(sizeof(Ks) >= 4 * 64 * (16 * (D / 32) + 2) * sizeof(float), "partial O fits K");
+    float* part = reinterpret_cast<float*>(&KV[0][0][0]) + (w.wave * (16 * (D / 32) + 2)) * 64 + w.lane;
+    static_assert(sizeof(KV) >= 4 * 64 * (16 * (D / 32) + 2) * sizeof(float), "partial O fits");
     if (group == 1) {
       part[0] = w.m;
       part[64] = w.l;
@@ -550,8 +566,6 @@ __device__ __forceinline__ uint16_t* w8_vbuf() {
   return w8V[B];
 }
 
-typedef __attribute__((address_space(3))) void w8_lds_void;
-
 struct SdpaW8 {
   static constexpr int D = W8_D, ND = D / 32, NDC = D / 16;
 
@@ -604,7 +618,7 @@ struct SdpaW8 {
     const uint64_t gs =
         (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(g >> 32)))) << 32) |
         uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(g))));
-    const uint32_t buf = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((w8_lds_void*)lds));
+    const uint32_t buf = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds));
     asm volatile(
         "s_mov_b32 m0, %0\n\t"
         "s_nop 0\n\t"
@@ -741,7 +755,7 @@ struct SdpaW8 {
           (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(gq >> 32)))) << 32) |
           uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(gq))));
       const uint32_t buf = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-          (w8_lds_void*)(w8Q[wave] + ins * 512)));
+          (lds_void*)(w8Q[wave] + ins * 512)));
       asm volatile(
           "s_mov_b32 m0, %0\n\t"
           "s_nop 0\n\t"
