@@ -202,15 +202,24 @@ struct Sdpa {
   }
 
   // rows kb * 64 .. + 63 of X into an LDS buffer; with RAGGED, rows past the
-  // sequence are its last row again
+  // sequence are its last row again.  Without, the loads share one offset a lane
+  // that stays the same for the whole loop, their rows in the uniform address
+  // (causal: 1 x 8 x 4096 x 128 65.9 us -> 64.8, 1 x 8 x 2048 x 128 36.5 -> 36.0, 2
+  // x 32 x 2048 x 64 51.3 -> 50.4; no change without the mask.  The same for all
+  // but the last block of a ragged sequence, behind a branch, was slower: 1 x 8 x
+  // 4000 x 128 65.5 -> 66.7).
   __device__ __forceinline__ void dma(const uint16_t* X, int chunk, int kb, const uint16_t* buf) {
     const uint64_t src = reinterpret_cast<uint64_t>(X + base + static_cast<int64_t>(kb) * BKV * D);
     const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)buf));
 #pragma unroll
     for (int i = 0; i < BKV / kRowsPer; ++i) {
-      int row = row0 + i * kRowsPer;
-      if (RAGGED) row = min(row, p.S - 1 - kb * BKV);
-      dma16(src, static_cast<uint32_t>(row * D + chunk) * 2u, lds + i * kThreads * 16 + wave * 1024);
+      const uint32_t at = lds + i * kThreads * 16 + wave * 1024;
+      if constexpr (RAGGED) {
+        const int row = min(row0 + i * kRowsPer, p.S - 1 - kb * BKV);
+        dma16(src, static_cast<uint32_t>(row * D + chunk) * 2u, at);
+      } else {
+        dma16(src + i * kRowsPer * D * 2, static_cast<uint32_t>(row0 * D + chunk) * 2u, at);
+      }
     }
   }
 
