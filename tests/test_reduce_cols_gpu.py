@@ -61,3 +61,15 @@ def test_nan_and_infinity(h):
         assert float(got[9]) == -float("inf")
         ok = torch.tensor([i for i in range(128) if i not in (3, 5, 9)])
         _check(got[ok], x[:, ok], kind)
+
+
+def test_more_columns_than_one_launch_of_strips_holds():
+    # 2^29 columns are 2^23 strips of 512 threads, one thread more than a launch
+    # takes; one column strip fewer is the widest that the strips take
+    for w in (2 ** 29 - 64, 2 ** 29):
+        print(f"column strips 1x{w}", flush=True)
+        x = torch.arange(w, dtype=torch.int32, device="cuda").remainder_(251).bfloat16().view(1, w)
+        out = torch.zeros(1, w, device="cuda")
+        _run(x, "max", (0, 0, 1, w), out)
+        assert torch.equal(out, x.float())
+        del x, out

@@ -1900,17 +1900,19 @@ int reduce_impl(const char* who, const ttlh_instr* prog, const ttlh_operand* in,
     a.splits = static_cast<int32_t>((h + a.rows_per_split - 1) / a.rows_per_split);
     const EltOperand& o0 = a.e.ops[0];
     const int64_t strips = (w + kStripCols - 1) / kStripCols;
-    if (mode == 1 && plain_row(o0) && strips < (int64_t(1) << 24)) {
-      // Shares of at least 1024 rows, at most eight (and at most the
-      // workspace's), while all make up to 512 workgroups: one launch below
-      // 2048 rows (512 x 4096: 3.9 us, 5.5 in two shares, 9.7 in 32-row shares of
-      // 512 columns by the kernel below), 4096^2 in four 11.5 us (one 17, eight
-      // 13; 15 below), 8192^2 in four 27 (two 31; 47 below).
-      const int64_t fill = strips < 512 ? 512 / strips : 1;
-      int64_t sp = h / 1024 < fill ? h / 1024 : fill;
-      if (sp > 8) sp = 8;
-      if (sp > a.splits) sp = a.splits;
-      if (sp < 1) sp = 1;
+    // Shares of at least 1024 rows, at most eight (and at most the workspace's),
+    // while all make up to 512 workgroups: one launch below 2048 rows (512 x 4096:
+    // 3.9 us, 5.5 in two shares, 9.7 in 32-row shares of 512 columns by the kernel
+    // below), 4096^2 in four 11.5 us (one 17, eight 13; 15 below), 8192^2 in four 27
+    // (two 31; 47 below).
+    const int64_t fill = strips < 512 ? 512 / strips : 1;
+    int64_t sp = h / 1024 < fill ? h / 1024 : fill;
+    if (sp > 8) sp = 8;
+    if (sp > a.splits) sp = a.splits;
+    if (sp < 1) sp = 1;
+    // (a launch holds fewer than 2^32 threads: from 2^29 columns on the kernel
+    // below, which takes two columns a thread)
+    if (mode == 1 && plain_row(o0) && strips * sp < (int64_t(1) << 32) / kStripThreads) {
       a.rows_per_split = (h + sp - 1) / sp;
       a.splits = static_cast<int32_t>((h + a.rows_per_split - 1) / a.rows_per_split);
       const uint16_t* const base = static_cast<const uint16_t*>(o0.ptr) +
