@@ -28,7 +28,7 @@ def _check(got, part, kind, scale=1.0):
 @pytest.mark.parametrize("kind", ["sum", "max"])
 @pytest.mark.parametrize("h,w", [(1, 8), (2, 64), (63, 72), (64, 200), (65, 4104), (513, 64),
                                  (1024, 96), (2047, 136), (2048, 64), (4099, 264), (9000, 24),
-                                 (2056, 32768)])
+                                 (2056, 32768), (66000, 72), (1000000, 8)])
 def test_strips(h, w, kind):
     print(f"column strips {h}x{w} {kind}", flush=True)
     x = O.seeded((h, w), "normal", 3).cuda()
@@ -73,3 +73,27 @@ def test_more_columns_than_one_launch_of_strips_holds():
         _run(x, "max", (0, 0, 1, w), out)
         assert torch.equal(out, x.float())
         del x, out
+
+
+def test_tall_and_narrow_operands_fill_the_chip():
+    # the same 64 MB as 8192 x 4096 and as one strip: in eight shares of a strip
+    # the tall one ran on 8 of 256 CUs, 15 times as long as the wide one
+    def best(h, w):
+        x = torch.ones(h, w, dtype=torch.bfloat16, device="cuda")
+        out = torch.zeros(1, w, device="cuda")
+        times = []
+        for _ in range(8):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda._sleep(1000000)  # the host is ahead when the first launch starts
+            start.record()
+            for _ in range(4):
+                _run(x, "sum", (0, 0, h, w), out)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        assert bool((out == h).all())
+        return min(times)
+
+    wide, tall = best(8192, 4096), best(2 ** 20, 32)
+    print(f"column sums of 64 MB: wide {wide * 250:.1f} us, tall {tall * 250:.1f} us", flush=True)
+    assert tall <= 5 * wide

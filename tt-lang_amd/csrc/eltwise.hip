@@ -1900,14 +1900,16 @@ int reduce_impl(const char* who, const ttlh_instr* prog, const ttlh_operand* in,
     a.splits = static_cast<int32_t>((h + a.rows_per_split - 1) / a.rows_per_split);
     const EltOperand& o0 = a.e.ops[0];
     const int64_t strips = (w + kStripCols - 1) / kStripCols;
-    // Shares of at least 1024 rows, at most eight (and at most the workspace's),
-    // while all make up to 512 workgroups: one launch below 2048 rows (512 x 4096:
-    // 3.9 us, 5.5 in two shares, 9.7 in 32-row shares of 512 columns by the kernel
-    // below), 4096^2 in four 11.5 us (one 17, eight 13; 15 below), 8192^2 in four 27
-    // (two 31; 47 below).
-    const int64_t fill = strips < 512 ? 512 / strips : 1;
-    int64_t sp = h / 1024 < fill ? h / 1024 : fill;
-    if (sp > 8) sp = 8;
+    // Shares of at least 1024 rows (at most the workspace's): up to eight while all
+    // make up to 512 workgroups, one launch below 2048 rows (512 x 4096: 3.9 us, 5.5
+    // in two shares, 9.7 in 32-row shares of 512 columns by the kernel below), 4096^2
+    // in four 11.5 us (one 17, eight 13; 15 below), 8192^2 in four 27 (two 31; 47
+    // below).  Few strips take more, up to 256 workgroups: 262144 x 64 in 256 shares
+    // 8.2 us (eight 56; 50 below), 1000000 x 32 16 (eight 234; 166 below), but
+    // 65536 x 1024 in 16 24.7 (32 26.1), 32768 x 2048 in eight 24.4 (16 25.0).
+    int64_t sp = strips < 512 ? 512 / strips : 1;
+    if (sp > 8) sp = strips < 32 ? 256 / strips : 8;
+    if (sp > h / 1024) sp = h / 1024;
     if (sp > a.splits) sp = a.splits;
     if (sp < 1) sp = 1;
     // (a launch holds fewer than 2^32 threads: from 2^29 columns on the kernel
