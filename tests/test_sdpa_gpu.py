@@ -277,6 +277,34 @@ def test_sdpa_scores_of_minus_infinity(S):
     _check(got, ref)
 
 
+@pytest.mark.parametrize("H,S", [(3, 256), (3, 2048), (17, 2048), (130, 256)])
+def test_sdpa_leading_scores_of_minus_infinity(H, S):
+    # with few blocks sdpa_fwd_kernel, with more than 256 sdpa_w8_kernel.  Even
+    # queries score -inf on the first keys (-3e38 times 64), odd ones do not see
+    # that column; every finite score is near -270, far below where exp underflows
+    # next to a maximum that would have stayed at 0.  Head 1 has three keys left, all
+    # at the end, and head 2 none: its even rows are 0 / 0.
+    print(f"sdpa -inf {H}x{S}", flush=True)
+    q, k, v = _qkv(1, H, S, 128, 23)
+    q[..., 3] = 0.0
+    q[:, :, ::2, 3] = 64.0
+    q[..., 5], k[..., 5] = 1.0, -3008.0
+    k[..., 3] = 0.0
+    k[:, :, :40, 3] = k[:, :, 64:160, 3] = -3e38
+    k[:, 1, :S - 3, 3] = -3e38
+    k[:, 2, :, 3] = -3e38
+    got = _run(q, k, v, 0.09)
+    for h in (0, 1, 2, H - 1):
+        keep = k[0, h, :, 3] == 0
+        even, odd = q[:, h:h + 1, ::2].clone(), q[:, h:h + 1, 1::2]
+        _check(got[:, h:h + 1, 1::2], O.sdpa_ref(odd, k[:, h:h + 1], v[:, h:h + 1], 0.09))
+        if bool(keep.any()):
+            _check(got[:, h:h + 1, ::2],
+                   O.sdpa_ref(even, k[:, h:h + 1, keep], v[:, h:h + 1, keep], 0.09))
+        else:
+            assert bool(torch.isnan(got[:, h, ::2]).all())
+
+
 @pytest.mark.parametrize("S", [96, 480])
 @pytest.mark.parametrize("D", [64, 128])
 def test_sdpa_infinite_value_in_a_ragged_last_row(S, D):

@@ -587,6 +587,7 @@ struct SdpaW8 {
   f32x16 negm;              // -m in every element: where each S accumulation starts
   u32x4 pw[2][2];           // [parity][kv chunk]: P(i - 1), P(i - 2) as bf16 pairs
   float m, l;               // running max (log2 units), this lane's share of the row sum
+  float limit;              // block sum above which the wave goes to rescale() (uniform)
   int k_src, v_src;         // per-lane DMA source offsets (elements)
   int v_frag[ND];           // LDS offsets of the V transpose reads
   uint32_t lds_wave;        // the wave's byte offset in a K / V buffer (uniform)
@@ -661,6 +662,10 @@ struct SdpaW8 {
   // 2^8) sends the wave to rescale(), which moves m by the block max where
   // that exceeds kLazy.  Otherwise every P = exp2(s - m) <= 2^12, which fp32
   // O and l absorb.  Row maxima use v_maximum3 (NaN-propagating).
+  // A query whose scores have all been -inf has no maximum yet: its m stays 0, its
+  // P and l are 0, and as long as a wave holds one, limit is below every sum, so
+  // that rescale() sees each block and takes the first finite maximum as it is,
+  // downwards too.
   static constexpr float kLazy = 8.0f;
   static constexpr float kSumLimit = 4096.0f;
   float rsum_;
@@ -691,6 +696,12 @@ struct SdpaW8 {
     rsum_ = g == 0 ? e0 + e1 : rsum_ + (e0 + e1);
   }
 
+  // (readfirstlane: in a scalar register, which the check's compare takes for free)
+  __device__ __forceinline__ void set_limit(bool every_block) {
+    limit = __int_as_float(__builtin_amdgcn_readfirstlane(
+        __float_as_int(every_block ? -1.0f : kSumLimit)));
+  }
+
   // The rare path for P(i - 1) (its scores in sp): move m by the block max d
   // where that exceeds kLazy, recompute P(i - 1), scale O (blocks <= i - 2)
   // and l by 2^-d, shift S(i) (accumulated from the old -m, now in sv) and
@@ -706,8 +717,11 @@ struct SdpaW8 {
     // SHIFT_S: S(i) was accumulated from the old -m (main steps); otherwise
     // S(i) is a new block's raw first block or absent, and -m is reset
     const float bm = xor32_max(max16(sp));
-    const float d = bm > kLazy ? bm : 0.0f;
-    const float alpha = __builtin_amdgcn_exp2f(-d);
+    const bool unset = xor32_add(l) == 0.0f;  // no score above -inf so far: O is 0 too
+    const bool none = bm == -INFINITY;
+    const float d = unset ? (none ? 0.0f : bm) : bm > kLazy ? bm : 0.0f;
+    const float alpha = unset ? 1.0f : __builtin_amdgcn_exp2f(-d);
+    set_limit(__any(unset && none));
     m += d;
     float rs = 0.0f;
 #pragma unroll
@@ -863,7 +877,7 @@ struct SdpaW8 {
     });
     if constexpr (DO_SM) {
       if constexpr (CHECK) {
-        if (__builtin_expect(__any(rsum_ > kSumLimit), 0)) rescale<PAR ^ 1, SHIFT>(sp);
+        if (__builtin_expect(__any(rsum_ > limit), 0)) rescale<PAR ^ 1, SHIFT>(sp);
       }
       l += rsum_;
     }
@@ -904,9 +918,13 @@ struct SdpaW8 {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // a block's S(0) (raw) is in sv: m = its maximum, S(0) and -m rebased
+  // a block's S(0) (raw) is in sv: m = its maximum (0 if that is -inf), S(0) and
+  // -m rebased
   __device__ __forceinline__ void start_block() {
     m = xor32_max(max16(sv));
+    const bool unset = m == -INFINITY;
+    set_limit(__any(unset));
+    m = unset ? 0.0f : m;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       sv[r] -= m;
