@@ -471,6 +471,13 @@ int ttlh_matmul_bfp4w_ws(const void* A, int64_t lda, const void* Bq4, void* C,
 int ttlh_sdpa_fwd(const void* Q, const void* K, const void* V, void* O,
                   int64_t B, int64_t H, int64_t S, int64_t D, float scale,
                   int causal, void* stream);
+/* The kernel that ttlh_sdpa_fwd runs for a problem it takes (for tests and
+ * profiles; the choice is by size alone): one or two groups of four waves a
+ * workgroup, or the eight-wave kernel. */
+#define TTLH_SDPA_ONE_GROUP 1
+#define TTLH_SDPA_TWO_GROUPS 2
+#define TTLH_SDPA_EIGHT_WAVES 8
+int ttlh_sdpa_fwd_form(int64_t B, int64_t H, int64_t S, int64_t D, int causal);
 
 /* ------------------------------------------------------------------------ */
 const char* ttlh_last_error(void);

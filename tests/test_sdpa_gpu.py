@@ -16,6 +16,7 @@ import pytest
 import torch
 
 from oracle import tile_ops as O
+from ttlhip import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -26,6 +27,16 @@ def _run(q, k, v, scale, causal=False):
     K.sdpa_fwd(q.cuda(), k.cuda(), v.cuda(), out, scale, causal)
     torch.cuda.synchronize()
     return out.cpu()
+
+
+# ttlh_sdpa_fwd_form: one or two groups of four waves (sdpa_fwd_kernel), eight
+# waves (sdpa_w8_kernel).  A test that is there for one of them asks, so that a
+# change of the choice cannot take its subject from it unseen.
+ONE_GROUP, TWO_GROUPS, EIGHT_WAVES = 1, 2, 8
+
+
+def _form(B, H, S, D=128, causal=False):
+    return L.load().ttlh_sdpa_fwd_form(B, H, S, D, int(causal))
 
 
 def _qkv(B, H, S, D, seed):
@@ -41,8 +52,7 @@ def _check(out, ref):
 @pytest.mark.parametrize("B,H,S,D", [(1, 1, 128, 128), (2, 3, 256, 128), (1, 2, 384, 64),
                                     (1, 2, 768, 128)])
 def test_sdpa_matches_reference(B, H, S, D):
-    # S = 256, 512 (below), 768 leave 0, 2 and 4 steps after the eight-wave
-    # kernel's six-step loop (its K / V rings have three buffers)
+    # few heads: sdpa_fwd_kernel whatever S is
     q, k, v = _qkv(B, H, S, D, 1)
     scale = 1.0 / math.sqrt(D)
     _check(_run(q, k, v, scale), O.sdpa_ref(q, k, v, scale))
@@ -77,6 +87,7 @@ def test_sdpa_one_hot_value_selects_probabilities():
 
 def test_sdpa_config5_sampled_heads():
     B, H, S, D = 4, 32, 4096, 128
+    assert _form(B, H, S) == EIGHT_WAVES
     q, k, v = _qkv(B, H, S, D, 21)
     scale = 1.0 / math.sqrt(D)
     out = _run(q, k, v, scale)
@@ -103,8 +114,8 @@ def test_sdpa_negative_and_zero_scale(scale, causal, D):
 
 @pytest.mark.parametrize("B,H,S", [(1, 3, 1024), (3, 1, 512)])
 def test_sdpa_several_query_blocks(B, H, S):
-    # several 256-query workgroups per head and several KV double-buffer
-    # cycles; V = 1 in the second head (or batch) pins the row sums exactly
+    # several query blocks per head and several cycles through the KV buffers; V = 1
+    # in the second head (or batch) pins the row sums exactly
     q, k, v = _qkv(B, H, S, 128, 61)
     v[-1, -1] = 1.0
     scale = 1.0 / math.sqrt(128)
@@ -130,6 +141,7 @@ def test_sdpa_blocks_uneven_over_the_workgroups():
     # CU: workgroups walk one or two blocks (the eight-wave kernel's
     # persistent grid); sampled heads of every part of the sequence
     B, H, S, D = 1, 75, 1024, 128
+    assert _form(B, H, S) == EIGHT_WAVES
     q, k, v = _qkv(B, H, S, D, 71)
     scale = 1.0 / math.sqrt(D)
     out = _run(q, k, v, scale)
@@ -138,17 +150,20 @@ def test_sdpa_blocks_uneven_over_the_workgroups():
         _check(out[sl], O.sdpa_ref(q[sl], k[sl], v[sl], scale))
 
 
-@pytest.mark.parametrize("B,H,S,seed", [(1, 4, 1024, 3), (1, 4, 1024, 4), (1, 2, 256, 5)])
+@pytest.mark.parametrize("B,H,S,seed", [(1, 4, 1024, 3), (1, 4, 1024, 4), (1, 2, 256, 5),
+                                        (1, 34, 1024, 6), (2, 17, 1024, 7), (1, 130, 256, 8),
+                                        (1, 70, 1024, 9)])
 def test_sdpa_last_blocks_with_slow_kv_loads(B, H, S, seed):
     # K and V in pinned host memory: every K / V load crosses PCIe and takes
-    # far longer than a step.  Every workgroup's last query block stages no
-    # Q for a next block, and its end-of-step wait must still cover the
-    # previous step's K / V loads, whose first fragments the next step
-    # prefetches: a wait that counted the skipped Q loads read stale
-    # fragments here (max error 0.28-0.59 of the output's range at
-    # [1, 4, 1024, 128]), and now and then with device memory.
-    from ttlhip import _lib as L
+    # far longer than a step.  From 17 heads on the eight-wave kernel: every
+    # workgroup's last query block (its only one, or with 70 heads its second)
+    # stages no Q for a next block, and its end-of-step wait must still cover the
+    # previous step's K / V loads, whose first fragments the next step prefetches.
+    # A wait that counted the skipped Q loads reads stale fragments (max error
+    # 0.28-0.59 of the output's range at [1, 4, 1024, 128] when that ran there),
+    # now and then with device memory too.
     D = 128
+    assert _form(B, H, S) == (EIGHT_WAVES if H >= 17 else TWO_GROUPS)
     g = torch.Generator().manual_seed(seed)
     q, k, v = (torch.randn(B, H, S, D, generator=g).bfloat16() for _ in range(3))
     kh, vh = k.pin_memory(), v.pin_memory()
@@ -157,7 +172,31 @@ def test_sdpa_last_blocks_with_slow_kv_loads(B, H, S, seed):
     L.call("ttlh_sdpa_fwd", qd.data_ptr(), kh.data_ptr(), vh.data_ptr(), out.data_ptr(), B, H, S,
            D, 0.1, 0, L.stream_ptr())
     torch.cuda.synchronize()
-    _check(out.cpu(), O.sdpa_ref(q, k, v, 0.1))
+    out = out.cpu()
+    for h in range(0, H, 1 if H < 10 else 7):
+        sl = (slice(None), slice(h, h + 1))
+        _check(out[sl], O.sdpa_ref(q[sl], k[sl], v[sl], 0.1))
+
+
+@pytest.mark.parametrize("H,S", [(130, 256), (43, 768), (33, 1024)])
+@pytest.mark.parametrize("scale", [0.09, -0.09, 0.0])
+def test_sdpa_eight_waves(H, S, scale):
+    # the eight-wave kernel with the fewest steps of a block (8, no pass of its
+    # inner loop), one query block a workgroup and two; V = 1 in head 1 pins the row
+    # sums, a one-hot V in head 2 shows the probabilities themselves
+    print(f"sdpa eight waves {H}x{S} scale {scale}", flush=True)
+    assert _form(1, H, S) == EIGHT_WAVES
+    q, k, v = _qkv(1, H, S, 128, 91)
+    v[0, 1] = 1.0
+    v[0, 2] = 0.0
+    v[0, 2, torch.arange(128), torch.arange(128)] = 1.0
+    out = _run(q, k, v, scale)
+    assert float((out[0, 1].float() - 1.0).abs().max()) <= 2 ** -7
+    p = torch.softmax((q[0, 2].double() @ k[0, 2].double().T) * scale, -1)
+    assert float((out[0, 2].double() - p[:, :128]).abs().max()) <= 1e-2 * float(p.max())
+    for h in (0, 3, H // 2, H - 1):
+        sl = (slice(None), slice(h, h + 1))
+        _check(out[sl], O.sdpa_ref(q[sl], k[sl], v[sl], scale))
 
 
 @pytest.mark.parametrize("jump", [False, True])
@@ -187,6 +226,7 @@ def test_sdpa_running_max_growth_in_later_blocks_of_a_workgroup():
     # growing along kv, one late key far above the rest) happen in every block,
     # so a block's rescale state must not leak into the next
     B, H, S, D = 1, 260, 512, 128
+    assert _form(B, H, S) == EIGHT_WAVES
     q = torch.zeros(B, H, S, D)
     q[..., 0] = 1.0
     q[..., 1] = torch.linspace(-1, 1, S)
@@ -234,10 +274,10 @@ def test_sdpa_ragged_negative_and_zero_scale(scale):
 @pytest.mark.parametrize("S,D,causal", [(384, 128, False), (256, 64, False), (96, 128, False),
                                         (512, 128, True), (256, 64, True)])
 def test_sdpa_other_kernels_with_slow_loads(S, D, causal):
-    # the kernels other than the eight-wave one (ping-pong, 4-wave, ragged,
-    # causal) with Q, K and V in pinned host memory: loads far slower than
-    # any step of their pipelines
-    from ttlhip import _lib as L
+    # sdpa_fwd_kernel (one and two groups, whole and ragged, with and without
+    # the mask) with Q, K and V in pinned host memory: loads far slower than any
+    # step of its pipeline
+    assert _form(1, 2, S, D, causal) == (TWO_GROUPS if S > 192 else ONE_GROUP)
     g = torch.Generator().manual_seed(S + D)
     q, k, v = (torch.randn(1, 2, S, D, generator=g).bfloat16() for _ in range(3))
     qh, kh, vh = q.pin_memory(), k.pin_memory(), v.pin_memory()
@@ -285,6 +325,7 @@ def test_sdpa_leading_scores_of_minus_infinity(H, S):
     # next to a maximum that would have stayed at 0.  Head 1 has three keys left, all
     # at the end, and head 2 none: its even rows are 0 / 0.
     print(f"sdpa -inf {H}x{S}", flush=True)
+    assert _form(1, H, S) == (TWO_GROUPS if H == 3 else EIGHT_WAVES)
     q, k, v = _qkv(1, H, S, 128, 23)
     q[..., 3] = 0.0
     q[:, :, ::2, 3] = 64.0

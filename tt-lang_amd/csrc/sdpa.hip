@@ -1019,6 +1019,21 @@ __global__ __launch_bounds__(W8_THREADS, 1) void sdpa_w8_kernel(const SdpaArgs p
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
 }
 
+// The kernel for `blocks` blocks of 128 queries.
+int form_of(int64_t blocks, int64_t S, int64_t D, bool causal) {
+  // (256 blocks of 128 queries and fewer leave sdpa_w8_kernel half the CUs:
+  // 1 x 8 x 2048 x 128 46.6 us against 40 to 42 in sdpa_fwd_kernel)
+  if (D == W8_D && !causal && S % W8_BQ == 0 && blocks > 256) return TTLH_SDPA_EIGHT_WAVES;
+  // Two groups of waves: up to one workgroup per CU, and under the causal mask
+  // up to two rounds of long blocks, whose shares of a CU would differ most (512
+  // blocks of S = 2016: 62 us against 69; of S = 480: 28 against 24; 384
+  // blocks without the mask: 84 against 72).  Three KV blocks do not pay for
+  // the second group.
+  return S > 192 && (blocks <= 256 || (causal && blocks <= 512 && S >= 1024))
+             ? TTLH_SDPA_TWO_GROUPS
+             : TTLH_SDPA_ONE_GROUP;
+}
+
 template <int D, bool CAUSAL>
 int launch(SdpaArgs a, hipStream_t s) {
   // heads dispatched together: a divisor of an XCD's share of the heads whose
@@ -1028,10 +1043,8 @@ int launch(SdpaArgs a, hipStream_t s) {
   a.heads_together = 1;
   for (int g = 1; g <= share && g <= fit; ++g)
     if (share % g == 0) a.heads_together = g;
-  const int64_t blocks = static_cast<int64_t>(a.nbh) * a.nqb;
-  // (256 blocks of 128 queries and fewer leave sdpa_w8_kernel half the CUs:
-  // 1 x 8 x 2048 x 128 46.6 us against 40 to 42 in sdpa_fwd_kernel)
-  if (D == W8_D && !CAUSAL && a.S % W8_BQ == 0 && blocks > 256) {
+  const int form = form_of(static_cast<int64_t>(a.nbh) * a.nqb, a.S, D, CAUSAL);
+  if (form == TTLH_SDPA_EIGHT_WAVES) {
     SdpaArgs b = a;
     b.nqb = a.S / W8_BQ;
     // persistent: one workgroup per CU (at most), each walking its blocks
@@ -1044,13 +1057,8 @@ int launch(SdpaArgs a, hipStream_t s) {
     hipLaunchKernelGGL(sdpa_w8_kernel, dim3(grid), dim3(W8_THREADS), 0, s, b);
     return check_launch("sdpa_w8_kernel");
   }
-  // Two groups of waves: up to one workgroup per CU, and under the causal mask
-  // up to two rounds of long blocks, whose shares of a CU would differ most (512
-  // blocks of S = 2016: 62 us against 69; of S = 480: 28 against 24; 384
-  // blocks without the mask: 84 against 72).  Three KV blocks do not pay for
-  // the second group.
-  const bool two = a.S > 192 && (blocks <= 256 || (CAUSAL && blocks <= 512 && a.S >= 1024));
-  const dim3 grid(static_cast<uint32_t>(blocks));
+  const bool two = form == TTLH_SDPA_TWO_GROUPS;
+  const dim3 grid(static_cast<uint32_t>(static_cast<int64_t>(a.nbh) * a.nqb));
   const bool ragged = a.S % BQ != 0;  // S % 32 == 0 only
   if (two && ragged)
     hipLaunchKernelGGL((sdpa_fwd_kernel<D, CAUSAL, true, 2>), grid, dim3(2 * kThreads), 0, s, a);
@@ -1095,4 +1103,8 @@ extern "C" int ttlh_sdpa_fwd(const void* Q, const void* K, const void* V, void* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (D == 128) return causal ? launch<128, true>(a, s) : launch<128, false>(a, s);
   return causal ? launch<64, true>(a, s) : launch<64, false>(a, s);
+}
+
+extern "C" int ttlh_sdpa_fwd_form(int64_t B, int64_t H, int64_t S, int64_t D, int causal) {
+  return form_of(B * H * ((S + BQ - 1) / BQ), S, D, causal != 0);
 }

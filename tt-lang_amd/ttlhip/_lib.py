@@ -142,6 +142,7 @@ SIGNATURES = {
     "ttlh_matmul_bfp4w_ws": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),
     "ttlh_matmul_bfp8w_ws": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),
     "ttlh_sdpa_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, C.c_float, _int, _vp]),
+    "ttlh_sdpa_fwd_form": (_int, [_i64, _i64, _i64, _i64, _int]),
     "ttlh_last_error": (C.c_char_p, []),
     "ttlh_version": (_int, []),
 }
