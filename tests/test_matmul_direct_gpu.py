@@ -79,6 +79,29 @@ def test_bf16_blocks_of_128(K):
     _check(f - f0, a, b, False)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,K,N", [(3328, 1024, 3072), (4064, 512, 4064)])
+def test_blocks_of_256_into_a_result_off_its_pairs(M, K, N, dtype):
+    # mm_dma_kernel (below and above 192 blocks, whole and cut) writes two columns at
+    # once, also where a column slice or an odd pitch leaves them unaligned
+    print(f"unaligned pairs {M}x{K}x{N} {dtype}", flush=True)
+    a, b = _operands(M, K, N, 29)
+    c = torch.empty(M, N, dtype=dtype, device="cuda")
+    Kn.matmul(a, b, c)
+    _check(c, a, b, dtype == torch.bfloat16)
+    odd = torch.full((M, N + 3), 7.0, dtype=dtype, device="cuda")
+    Kn.matmul(a, b, odd[:, 1:N + 1])
+    assert torch.equal(odd[:, 1:N + 1], c)
+    assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())
+    c0 = O.seeded((M, N), "normal", 30, dtype).cuda()
+    wide = c0.clone()
+    Kn.matmul(a, b, wide, accumulate=True)
+    odd[:, 1:N + 1] = c0
+    Kn.matmul(a, b, odd[:, 1:N + 1], accumulate=True)
+    assert torch.equal(odd[:, 1:N + 1], wide)
+    assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())
+
+
 @pytest.mark.parametrize("M,K,N", [(4096, 32, 3072), (4096, 96, 3104), (32, 64, 49152)])
 def test_sums_in_the_fused_epilogues_order(M, K, N):
     # problems that the fused epilogue takes give the same bits with and
@@ -262,3 +285,20 @@ def test_packed_decode_is_exact(K, bits):
     _matmul_packed(torch.eye(K, dtype=torch.bfloat16, device="cuda"), q.cuda(), c, bits)
     w = _unpacked(q, K, N, bits)
     assert torch.equal(c.cpu().float(), w.float())
+
+
+@pytest.mark.parametrize("K,N", [(128, 3072), (96, 3104)])
+def test_packed_weights_in_blocks_of_256_into_a_result_off_its_pairs(K, N):
+    # mm_dq_kernel and mm256_kernel, as above
+    M = 4096
+    print(f"unaligned pairs packed {M}x{K}x{N}", flush=True)
+    a = O.seeded((M, K), "normal", 33, torch.bfloat16, std=K ** -0.5).cuda()
+    q = OB.pack_c(O.seeded((K, N), "normal", 34, torch.float32))
+    qd = q.cuda()
+    c = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    _matmul_packed(a, qd, c, 8)
+    _check(c, a, OB.unpack_c(q, K, N), True)
+    odd = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device="cuda")
+    _matmul_packed(a, qd, odd[:, 1:N + 1], 8)
+    assert torch.equal(odd[:, 1:N + 1], c)
+    assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())

@@ -297,7 +297,12 @@ __device__ __forceinline__ void store_acc_tile(const MmArgs& p, const f32x16& t,
 // rows; DPP swaps of each row pair give the even lane rows 8 (r / 4) +
 // 4 (lane / 32) + r % 4 for even r and the odd lane those for odd r, both as
 // (column 2c, column 2c + 1) pairs: 8 packed stores per lane instead of 16
-// 2-byte ones.  Offsets are 32-bit (the launcher checks M * ldc < 2^31).
+// 2-byte ones.  Offsets are 32-bit (the launcher checks M * ldc < 2^31).  C
+// need only be aligned to its elements (an odd pitch, a column slice): the pair
+// types say so, and the store stays one instruction (gfx950 under HSA takes
+// unaligned global accesses, which the compiler relies on here).
+typedef uint32_t bf16_pair __attribute__((aligned(2)));
+typedef float f32_pair __attribute__((ext_vector_type(2), aligned(4)));
 template <bool BF16OUT, bool ACC>
 __device__ __forceinline__ void store_acc_tile_pairs(const MmArgs& p, const f32x16& t, int r0,
                                                      int c0, int lane) {
@@ -317,7 +322,7 @@ __device__ __forceinline__ void store_acc_tile_pairs(const MmArgs& p, const f32x
     const uint32_t off = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.ldc) +
                          static_cast<uint32_t>(col);
     if constexpr (BF16OUT) {
-      uint32_t* c = reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.C) + off);
+      bf16_pair* c = reinterpret_cast<bf16_pair*>(static_cast<uint16_t*>(p.C) + off);
       float a = lo, b = hi;
       if constexpr (ACC) {
         const uint32_t old = *c;
@@ -326,9 +331,8 @@ __device__ __forceinline__ void store_acc_tile_pairs(const MmArgs& p, const f32x
       }
       *c = cvt_pk_bf16x2(a, b);
     } else {
-      typedef float f32x2 __attribute__((ext_vector_type(2)));
-      f32x2* c = reinterpret_cast<f32x2*>(static_cast<float*>(p.C) + off);
-      f32x2 v = {lo, hi};
+      f32_pair* c = reinterpret_cast<f32_pair*>(static_cast<float*>(p.C) + off);
+      f32_pair v = {lo, hi};
       if constexpr (ACC) v += *c;
       *c = v;
     }
