@@ -302,3 +302,19 @@ def test_packed_weights_in_blocks_of_256_into_a_result_off_its_pairs(K, N):
     _matmul_packed(a, qd, odd[:, 1:N + 1], 8)
     assert torch.equal(odd[:, 1:N + 1], c)
     assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M", [32, 96])
+def test_packed_weights_and_rows_far_apart(M, bits):
+    # rows of A 2^24 elements apart: past the decoding kernels' 32-bit offsets, so
+    # bfloat8_b goes to mm_bf16_kernel's decoding form, bfloat4_b to the two passes
+    K, N, pitch = 160, 96, 2 ** 24
+    print(f"packed {bits} pitch {pitch} M {M}", flush=True)
+    buf = torch.empty((M - 1) * pitch + K, dtype=torch.bfloat16, device="cuda")
+    a = buf.as_strided((M, K), (pitch, 1))
+    a.copy_(O.seeded((M, K), "normal", 35, torch.bfloat16, std=K ** -0.5))
+    q = _packed(O.seeded((K, N), "normal", 36, torch.float32), bits)
+    c = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    _matmul_packed(a, q.cuda(), c, bits)
+    _check(c, a, _unpacked(q, K, N, bits), True)

@@ -610,12 +610,13 @@ BFP4_TWO_PASS_MIN_M = 512
 TWO_PASS_MIN_MACS = 1_500_000_000
 
 
-def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> None:
+def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> int:
     sp = L.stream_ptr(stream)
     scratch = _matmul_scratch(c.device, stream, sp)
-    L.call("ttlh_matmul_scratch", a.data_ptr(), L.TTLH_BF16, a.stride(0), bq.data_ptr(), code, N,
-           c.data_ptr(), L.TTLH_BF16, c.stride(0), M, N, K, 0,
-           scratch.data_ptr() if scratch is not None else 0, L.MATMUL_SCRATCH_BYTES, sp)
+    return L.load().ttlh_matmul_scratch(
+        a.data_ptr(), L.TTLH_BF16, a.stride(0), bq.data_ptr(), code, N, c.data_ptr(), L.TTLH_BF16,
+        c.stride(0), M, N, K, 0, scratch.data_ptr() if scratch is not None else 0,
+        L.MATMUL_SCRATCH_BYTES, sp)
 
 
 def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None,
@@ -637,7 +638,7 @@ def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
         two_pass = (M >= BFP8_TWO_PASS_MIN_M and M * N * K >= TWO_PASS_MIN_MACS
                     and bq.data_ptr() % 16 == 0)
     if not two_pass:
-        _matmul_packed(a, bq, L.TTLH_BFP8, c, M, N, K, stream)
+        L.check("ttlh_matmul_scratch", _matmul_packed(a, bq, L.TTLH_BFP8, c, M, N, K, stream))
         return
     nbytes = int(L.load().ttlh_matmul_bfp8w_workspace_bytes(M, N, K))
     ws = _workspace(c.device, stream, nbytes)
@@ -694,11 +695,14 @@ def matmul_bfp4w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None
     if a.stride(1) != 1 or c.stride(1) != 1:
         raise ValueError("matmul_bfp4w: A and C must be row-major")
     # (operands off their alignment go to the two passes at any M, which refuse
-    # them)
+    # them, and so do those that the decoding kernel refuses: it addresses A's rows
+    # with 32 bits, so not from strides of 2^24 on)
     if ((M < BFP4_TWO_PASS_MIN_M or M * N * K < TWO_PASS_MIN_MACS) and bq.data_ptr() % 8 == 0
             and a.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0):
-        _matmul_packed(a, bq, L.TTLH_BFP4, c, M, N, K, stream)
-        return
+        status = _matmul_packed(a, bq, L.TTLH_BFP4, c, M, N, K, stream)
+        if status != L.TTLH_EUNSUPPORTED:
+            L.check("ttlh_matmul_scratch", status)
+            return
     ws = _workspace(c.device, stream, K * N * 2)
     L.call("ttlh_matmul_bfp4w_ws", a.data_ptr(), a.stride(0), bq.data_ptr(), c.data_ptr(),
            c.stride(0), M, N, K, ws.data_ptr(), K * N * 2, L.stream_ptr(stream))
