@@ -83,12 +83,14 @@ _MATMUL_SCRATCH_LOCK = threading.Lock()
 
 
 def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Tensor]:
+    # (default streams of all devices have handle 0: the stream must be one of the
+    # tensors' device, or the launch would share the counters of another stream)
+    if (stream.device.index if stream is not None else torch._C._cuda_getDevice()) != device.index:
+        return None
     key = (device.index, sp)
     t = _MATMUL_SCRATCH.get(key)
     if t is None:
         s = stream if stream is not None else torch.cuda.current_stream()
-        if s.device.index != device.index:
-            return None  # the zeroing would not be ordered before the launch
         with _MATMUL_SCRATCH_LOCK, torch.cuda.stream(s):
             t = _MATMUL_SCRATCH.get(key)
             if t is None:
