@@ -333,9 +333,11 @@ int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B,
  * zeroed once before its first use and then left to the library (NULL: none).
  * Problems with few outputs then divide K among several workgroups per output
  * block; sums are added in a fixed order, so results repeat exactly.  Launches
- * that share a scratch must be ordered (one stream); while the stream is being
- * captured the scratch is not used.  No counterpart in the reference (its
- * kernels own a core's SRAM). */
+ * that share a scratch must be ordered (one stream).  While the stream is being
+ * captured the scratch is not used: there, and without one (ttlh_matmul too),
+ * a workgroup takes the parts of its block in turn, which is slower and gives
+ * the same bits.  No counterpart in the reference (its kernels own a core's
+ * SRAM). */
 #define TTLH_BFP8 8
 #define TTLH_BFP4 4
 #define TTLH_MATMUL_SCRATCH_BYTES (4198400)

@@ -160,8 +160,8 @@ def test_bf16_accumulate_f32(M, K, N):
 
 
 def test_divided_product_under_capture_and_on_two_streams():
-    # under capture K is not divided (a replay may run beside launches that use
-    # the scratch); two streams have a scratch each
+    # under capture one workgroup takes all parts of K (a replay may run beside
+    # launches that use the scratch); two streams have a scratch each
     a, b = _operands(32, 4096, 256, 9)
     c = torch.zeros(32, 256, dtype=torch.bfloat16, device="cuda")
     Kn.matmul(a, b, c)
@@ -318,3 +318,41 @@ def test_packed_weights_and_rows_far_apart(M, bits):
     c = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
     _matmul_packed(a, q.cuda(), c, bits)
     _check(c, a, _unpacked(q, K, N, bits), True)
+
+
+@pytest.mark.parametrize("kind", [torch.bfloat16, torch.float32, 8, 4])
+@pytest.mark.parametrize("M,K,N", [(32, 2048, 96), (32, 11008, 288), (64, 4096, 1504),
+                                   (96, 4000, 3968), (160, 2080, 2080)])
+def test_divided_products_bits_are_their_sizes(M, K, N, kind):
+    # K in two and four parts of 32x64, 32x128 and (fp32) 32x32 blocks, and cut
+    # blocks: the same bits with a workgroup for each part, under capture and without
+    # a scratch at all
+    print(f"parts {M}x{K}x{N} {kind}", flush=True)
+    if kind in (8, 4):
+        a = O.seeded((M, K), "normal", 41, torch.bfloat16, std=K ** -0.5).cuda()
+        b = _packed(O.seeded((K, N), "normal", 42, torch.float32), kind).cuda()
+        dt, code = torch.bfloat16, kind
+
+        def run(out):
+            _matmul_packed(a, b, out, kind)
+    else:
+        a, b = _operands(M, K, N, 41, kind)
+        dt, code = kind, L.dtype_code(kind)
+
+        def run(out):
+            Kn.matmul(a, b, out)
+    eager, captured, bare = (torch.zeros(M, N, dtype=dt, device="cuda") for _ in range(3))
+    run(eager)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run(captured)
+    for _ in range(3):
+        captured.zero_()
+        g.replay()
+        run(eager)
+        torch.cuda.synchronize()
+        assert torch.equal(captured, eager)
+    L.call("ttlh_matmul_scratch", a.data_ptr(), L.dtype_code(a.dtype), K, b.data_ptr(), code, N,
+           bare.data_ptr(), L.dtype_code(dt), N, M, N, K, 0, 0, 0, L.stream_ptr())
+    assert torch.equal(bare, eager)

@@ -116,25 +116,58 @@ __device__ __forceinline__ f32x4 get_part(const float* d) {
   return __builtin_bit_cast(f32x4, w);
 }
 
-// The sum over the waves' partial blocks in LDS (rows at a pitch of PITCH
-// floats), in wave order, and the store of the block.
-template <int BM, int BN, int PITCH, int WK, int THREADS>
+// Chunk c (four results of a row) of the sum over the waves' blocks in LDS (rows
+// at a pitch of PITCH floats), in wave order.
+template <int BM, int BN, int PITCH, int WK>
+__device__ __forceinline__ f32x4 wave_sum(const float* part, int c) {
+  const float* q = part + c / (BN / 4) * PITCH + (c % (BN / 4)) * 4;
+  f32x4 s = *reinterpret_cast<const f32x4*>(q);
+#pragma unroll
+  for (int w = 1; w < WK; ++w) s += *reinterpret_cast<const f32x4*>(q + w * BM * PITCH);
+  return s;
+}
+
+// The block's result: of each of the p.splits parts of K, part_of(split) leaves
+// the waves' blocks in LDS, behind a barrier; their sums are added in split order.
+// WHOLE: this workgroup takes all parts, one after the other (where there is no
+// scratch to meet in); the results are the same bits.
+template <int BM, int BN, int PITCH, int WK, int THREADS, bool WHOLE, typename F>
 __device__ __forceinline__ void reduce_store(const DirectArgs& p, const float* part, int bm, int bn,
-                                             int split) {
+                                             int split, F part_of) {
   constexpr int kChunks = BM * BN / 4;
   const int m0 = bm * BM, n0 = bn * BN;
+  const auto store = [&](int c, f32x4 v) {
+    const int row = m0 + c / (BN / 4), col = n0 + (c % (BN / 4)) * 4;
+    if (row < p.M && col < p.N) store4(p, row, col, v);
+  };
+  if constexpr (WHOLE) {
+    constexpr int kPer = (kChunks + THREADS - 1) / THREADS;
+    const int t = threadIdx.x;
+    f32x4 sum[kPer];
+    for (int s = 0; s < p.splits; ++s) {
+      part_of(s);
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (t + i * THREADS < kChunks) {
+          const f32x4 v = wave_sum<BM, BN, PITCH, WK>(part, t + i * THREADS);
+          sum[i] = s == 0 ? v : sum[i] + v;
+        }
+      __syncthreads();  // the next part writes over these
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      if (t + i * THREADS < kChunks) store(t + i * THREADS, sum[i]);
+    return;
+  }
+  part_of(split);
   const int block = bn * p.grid_m + bm;
   float* mine = p.partial + static_cast<int64_t>(block * p.splits + split) * (BM * BN);
   for (int c = threadIdx.x; c < kChunks; c += THREADS) {
-    const int r = c / (BN / 4), col = (c % (BN / 4)) * 4;
-    f32x4 s = *reinterpret_cast<const f32x4*>(part + r * PITCH + col);
-#pragma unroll
-    for (int w = 1; w < WK; ++w)
-      s += *reinterpret_cast<const f32x4*>(part + w * BM * PITCH + r * PITCH + col);
+    const f32x4 s = wave_sum<BM, BN, PITCH, WK>(part, c);
     if (p.splits > 1)
       put_part(mine + 4 * c, s);
-    else if (m0 + r < p.M && n0 + col < p.N)
-      store4(p, m0 + r, n0 + col, s);
+    else
+      store(c, s);
   }
   if (p.splits == 1) return;
   // The workgroup that arrives last at this block's counter adds the parts,
@@ -154,11 +187,10 @@ __device__ __forceinline__ void reduce_store(const DirectArgs& p, const float* p
   if (!last) return;
   const float* parts = p.partial + static_cast<int64_t>(block) * p.splits * (BM * BN);
   for (int c = threadIdx.x; c < kChunks; c += THREADS) {
-    const int r = c / (BN / 4), col = (c % (BN / 4)) * 4;
     f32x4 s = get_part(parts + 4 * c);
     for (int w = 1; w < p.splits; ++w)
       s += get_part(parts + static_cast<int64_t>(w) * (BM * BN) + 4 * c);
-    if (m0 + r < p.M && n0 + col < p.N) store4(p, m0 + r, n0 + col, s);
+    store(c, s);
   }
 }
 
@@ -188,7 +220,7 @@ template <typename V>
 __device__ __forceinline__ uint32_t word(const V& v, int i) { return v[i]; }
 __device__ __forceinline__ uint32_t word(const uint32_t& v, int) { return v; }
 
-template <int MT, int NPL, int WK, int D, int OCC>
+template <int MT, int NPL, int WK, int D, int OCC, bool WHOLE = false>
 __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArgs p) {
   constexpr int BM = 16 * MT, BN = 16 * NPL, PITCH = BN + 4;
   __shared__ __attribute__((aligned(16))) float part[WK * BM * PITCH];
@@ -211,85 +243,87 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
   const uint32_t b_off = 2 * (static_cast<uint32_t>(8 * kg) * static_cast<uint32_t>(p.ldb) +
                               min(n0 + NPL * l16, p.N - NPL));
 
-  f32x4 acc[MT][NPL];
+  const auto part_of = [&](int part_id) {
+    f32x4 acc[MT][NPL];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NPL; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < NPL; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const int stages = p.K / 32, first = split * WK + wave, step = p.splits * WK;
-  typedef BfStage<MT, NPL, D> Stage;
-  auto load = [&](Stage& s, int i) {  // the wave's i-th stage
-    const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 32;
-    const uint32_t bo = opaque(b_off);
-    const uint16_t* ak = A + k0;
-    const uint16_t* bk = B + k0 * p.ldb;
+    const int stages = p.K / 32, first = part_id * WK + wave, step = p.splits * WK;
+    typedef BfStage<MT, NPL, D> Stage;
+    auto load = [&](Stage& s, int i) {  // the wave's i-th stage
+      const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 32;
+      const uint32_t bo = opaque(b_off);
+      const uint16_t* ak = A + k0;
+      const uint16_t* bk = B + k0 * p.ldb;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      s.b[j] = gload<typename Stage::vec>(bk + static_cast<int64_t>(j) * p.ldb, bo);
+      for (int j = 0; j < 8; ++j)
+        s.b[j] = gload<typename Stage::vec>(bk + static_cast<int64_t>(j) * p.ldb, bo);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
-  };
-  auto compute = [&](const Stage& s) {
+      for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
+    };
+    auto compute = [&](const Stage& s) {
 #pragma unroll
-    for (int c = 0; c < NPL; ++c) {
-      u32x4 f;
+      for (int c = 0; c < NPL; ++c) {
+        u32x4 f;
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const uint32_t x = word(s.b[2 * d], c >> 1), y = word(s.b[2 * d + 1], c >> 1);
-        f[d] = (c & 1) ? perm_hi(x, y) : perm_lo(x, y);
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t x = word(s.b[2 * d], c >> 1), y = word(s.b[2 * d + 1], c >> 1);
+          f[d] = (c & 1) ? perm_hi(x, y) : perm_lo(x, y);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, f), acc[m][c], 0, 0, 0);
       }
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, f), acc[m][c], 0, 0, 0);
-    }
-  };
+    };
 
-  const int n = stages > first ? (stages - first + step - 1) / step : 0;
-  Stage st[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    load(st[d], d);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  int i = 0;
-  for (; i + 2 * D <= n; i += D) {
+    const int n = stages > first ? (stages - first + step - 1) / step : 0;
+    Stage st[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      compute(st[d]);
-      __builtin_amdgcn_sched_barrier(0);
-      load(st[d], i + D + d);
+      load(st[d], d);
       __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    int i = 0;
+    for (; i + 2 * D <= n; i += D) {
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (i + d < n) compute(st[d]);
-    if (i + D + d < n) load(st[d], i + D + d);
-  }
-#pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (i + D + d < n) compute(st[d]);
-
-  // lane holds of MFMA (m, c): column NPL l16 + c, rows 16 m + 4 kg + r
-  float* mine = part + wave * BM * PITCH + (4 * kg) * PITCH + NPL * l16;
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float* d = mine + (16 * m + r) * PITCH;
-      if constexpr (NPL == 2) {
-        *reinterpret_cast<f32x2*>(d) = f32x2{acc[m][0][r], acc[m][1][r]};
-      } else {
-#pragma unroll
-        for (int c = 0; c < NPL; c += 4)
-          *reinterpret_cast<f32x4*>(d + c) =
-              f32x4{acc[m][c][r], acc[m][c + 1][r], acc[m][c + 2][r], acc[m][c + 3][r]};
+      for (int d = 0; d < D; ++d) {
+        compute(st[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(st[d], i + D + d);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  __syncthreads();
-  reduce_store<BM, BN, PITCH, WK, 64 * WK>(p, part, bm, bn, split);
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (i + d < n) compute(st[d]);
+      if (i + D + d < n) load(st[d], i + D + d);
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (i + D + d < n) compute(st[d]);
+
+    // lane holds of MFMA (m, c): column NPL l16 + c, rows 16 m + 4 kg + r
+    float* mine = part + wave * BM * PITCH + (4 * kg) * PITCH + NPL * l16;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float* d = mine + (16 * m + r) * PITCH;
+        if constexpr (NPL == 2) {
+          *reinterpret_cast<f32x2*>(d) = f32x2{acc[m][0][r], acc[m][1][r]};
+        } else {
+#pragma unroll
+          for (int c = 0; c < NPL; c += 4)
+            *reinterpret_cast<f32x4*>(d + c) =
+                f32x4{acc[m][c][r], acc[m][c + 1][r], acc[m][c + 2][r], acc[m][c + 3][r]};
+        }
+      }
+    __syncthreads();
+  };
+  reduce_store<BM, BN, PITCH, WK, 64 * WK, WHOLE>(p, part, bm, bn, split, part_of);
 }
 
 // ---------------------------------------------------------------------------
@@ -336,7 +370,7 @@ __device__ __forceinline__ u32x2 spread_nibbles(uint32_t w) {
   return u32x2{(x | (x << 4)) & 0x87878787u, (y | (y << 4)) & 0x87878787u};
 }
 
-template <int MT, int NT, int BITS, int WK, int D, int OCC>
+template <int MT, int NT, int BITS, int WK, int D, int OCC, bool WHOLE = false>
 __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_bq_kernel(const DirectArgs p) {
   constexpr int BM = 16 * MT, BN = 32 * NT, PITCH = BN + 4;
   constexpr int kTile = BITS == 8 ? TTLH_BFP8_TILE_BYTES : TTLH_BFP4_TILE_BYTES;
@@ -378,108 +412,110 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_bq_kernel(const Direct
   // transpose read of k rows 8 kg + 4 half .. + 3: lane addresses row l16 / 4,
   // columns 4 (l16 % 4) ..
   uint8_t* const get = lds + wave * kStageLds + (4 * kg + (l16 >> 2)) * kRow + 8 * (l16 & 3);
+  float* const part = reinterpret_cast<float*>(lds);
 
-  f32x4 acc[MT][2 * NT];
+  const auto part_of = [&](int part_id) {
+    f32x4 acc[MT][2 * NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2 * NT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < 2 * NT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const int stages = p.K / 32, first = split * WK + wave, step = p.splits * WK;
-  typedef BqStage<MT, NT, BITS> Stage;
-  auto load = [&](Stage& s, int i) {
-    const int64_t st = min(first + i * step, stages - 1);
-    const uint16_t* ak = A + st * 32;
-    const uint8_t* qk = Q + st * (static_cast<int64_t>(tiles_n) * kTile);
+    const int stages = p.K / 32, first = part_id * WK + wave, step = p.splits * WK;
+    typedef BqStage<MT, NT, BITS> Stage;
+    auto load = [&](Stage& s, int i) {
+      const int64_t st = min(first + i * step, stages - 1);
+      const uint16_t* ak = A + st * 32;
+      const uint8_t* qk = Q + st * (static_cast<int64_t>(tiles_n) * kTile);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if constexpr (BITS == 8) {
-        s.q[t] = gload<u32x4a8>(qk, opaque(q_off[t]));
-      } else {
-        const u32x2 v = gload<u32x2>(qk, opaque(q_off[t]));
-        s.q[t].x = v.x;
-        s.q[t].y = v.y;
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (BITS == 8) {
+          s.q[t] = gload<u32x4a8>(qk, opaque(q_off[t]));
+        } else {
+          const u32x2 v = gload<u32x2>(qk, opaque(q_off[t]));
+          s.q[t].x = v.x;
+          s.q[t].y = v.y;
+        }
+        s.e[t] = gload<uint8_t>(qk, opaque(e_off[t]));
       }
-      s.e[t] = gload<uint8_t>(qk, opaque(e_off[t]));
-    }
 #pragma unroll
-    for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
-  };
-  typedef short i16x4 __attribute__((ext_vector_type(4)));
-  typedef short i16x8 __attribute__((ext_vector_type(8)));
-  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-  auto compute = [&](const Stage& s) {
+      for (int m = 0; m < MT; ++m) s.a[m] = gload<u32x4>(ak, opaque(a_off[m]));
+    };
+    typedef short i16x4 __attribute__((ext_vector_type(4)));
+    typedef short i16x8 __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    auto compute = [&](const Stage& s) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      u32x4 v = s.q[t];
-      if constexpr (BITS == 4) {
-        const u32x2 x = spread_nibbles(v.x), y = spread_nibbles(v.y);
-        v = u32x4{x.x, x.y, y.x, y.y};
+      for (int t = 0; t < NT; ++t) {
+        u32x4 v = s.q[t];
+        if constexpr (BITS == 4) {
+          const u32x2 x = spread_nibbles(v.x), y = spread_nibbles(v.y);
+          v = u32x4{x.x, x.y, y.x, y.y};
+        }
+        const int shift = static_cast<int>(s.e[t]) - kBias;
+        uint32_t o[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t m = v[i] & 0x7f7f7f7fu;
+          o[2 * i] = decode_pair(v[i], m, shift, false);
+          o[2 * i + 1] = decode_pair(v[i], m, shift, true);
+        }
+        *reinterpret_cast<u32x4*>(put + 64 * t) = u32x4{o[0], o[1], o[2], o[3]};
+        *reinterpret_cast<u32x4*>(put + 64 * t + 16) = u32x4{o[4], o[5], o[6], o[7]};
       }
-      const int shift = static_cast<int>(s.e[t]) - kBias;
-      uint32_t o[8];
+      // (the wave reads what it wrote itself: LDS operations of one wave
+      // complete in order, so no barrier)
+      asm volatile("" ::: "memory");
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t m = v[i] & 0x7f7f7f7fu;
-        o[2 * i] = decode_pair(v[i], m, shift, false);
-        o[2 * i + 1] = decode_pair(v[i], m, shift, true);
+      for (int j = 0; j < 2 * NT; ++j) {
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 32 * j));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 16 * kRow + 32 * j));
+        const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, w), acc[m][j], 0, 0, 0);
       }
-      *reinterpret_cast<u32x4*>(put + 64 * t) = u32x4{o[0], o[1], o[2], o[3]};
-      *reinterpret_cast<u32x4*>(put + 64 * t + 16) = u32x4{o[4], o[5], o[6], o[7]};
-    }
-    // (the wave reads what it wrote itself: LDS operations of one wave
-    // complete in order, so no barrier)
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int j = 0; j < 2 * NT; ++j) {
-      const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 32 * j));
-      const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(get + 16 * kRow + 32 * j));
-      const i16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, s.a[m]), __builtin_bit_cast(bf16x8, w), acc[m][j], 0, 0, 0);
-    }
-    asm volatile("" ::: "memory");
-  };
+      asm volatile("" ::: "memory");
+    };
 
-  const int n = stages > first ? (stages - first + step - 1) / step : 0;
-  Stage st[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    load(st[d], d);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  int i = 0;
-  for (; i + 2 * D <= n; i += D) {
+    const int n = stages > first ? (stages - first + step - 1) / step : 0;
+    Stage st[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      compute(st[d]);
-      __builtin_amdgcn_sched_barrier(0);
-      load(st[d], i + D + d);
+      load(st[d], d);
       __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    int i = 0;
+    for (; i + 2 * D <= n; i += D) {
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (i + d < n) compute(st[d]);
-    if (i + D + d < n) load(st[d], i + D + d);
-  }
+      for (int d = 0; d < D; ++d) {
+        compute(st[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(st[d], i + D + d);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (i + D + d < n) compute(st[d]);
+    for (int d = 0; d < D; ++d) {
+      if (i + d < n) compute(st[d]);
+      if (i + D + d < n) load(st[d], i + D + d);
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (i + D + d < n) compute(st[d]);
 
-  __syncthreads();  // the stage buffers become the partial blocks
-  float* part = reinterpret_cast<float*>(lds);
-  float* d = part + wave * BM * PITCH + (4 * kg) * PITCH + l16;
+    __syncthreads();  // the stage buffers become the partial blocks
+    float* d = part + wave * BM * PITCH + (4 * kg) * PITCH + l16;
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int j = 0; j < 2 * NT; ++j)
+      for (int j = 0; j < 2 * NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) d[(16 * m + r) * PITCH + 16 * j] = acc[m][j][r];
-  __syncthreads();
-  reduce_store<BM, BN, PITCH, WK, 64 * WK>(p, part, bm, bn, split);
+        for (int r = 0; r < 4; ++r) d[(16 * m + r) * PITCH + 16 * j] = acc[m][j][r];
+    __syncthreads();
+  };
+  reduce_store<BM, BN, PITCH, WK, 64 * WK, WHOLE>(p, part, bm, bn, split, part_of);
 }
 
 // ---------------------------------------------------------------------------
@@ -494,7 +530,7 @@ struct FStage {
   float b[2][4][NT];
 };
 
-template <int MT, int NT, int WM, int WN, int WK, int OCC>
+template <int MT, int NT, int WM, int WN, int WK, int OCC, bool WHOLE = false>
 __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void mm_direct_f32_kernel(const DirectArgs p) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, PITCH = BN + 4, D = 2;
   constexpr int kWaves = WM * WN * WK;
@@ -516,90 +552,92 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void mm_direct_f32_kernel(c
   const uint32_t b_off = 4 * (static_cast<uint32_t>(4 * h) * static_cast<uint32_t>(p.ldb) +
                               min(n0 + 32 * NT * wn + NT * l32, p.N - NT));
 
-  f32x16 acc[MT][NT];
+  const auto part_of = [&](int part_id) {
+    f32x16 acc[MT][NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int stages = p.K / 16, first = split * WK + wk, step = p.splits * WK;
-  typedef FStage<MT, NT> Stage;
-  auto load = [&](Stage& s, int i) {  // stage of 16 k
-    const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 16;
-    const uint32_t bo = opaque(b_off);
+    const int stages = p.K / 16, first = part_id * WK + wk, step = p.splits * WK;
+    typedef FStage<MT, NT> Stage;
+    auto load = [&](Stage& s, int i) {  // stage of 16 k
+      const int64_t k0 = static_cast<int64_t>(min(first + i * step, stages - 1)) * 16;
+      const uint32_t bo = opaque(b_off);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const float* bk = B + (k0 + 8 * g) * p.ldb;
+      for (int g = 0; g < 2; ++g) {
+        const float* bk = B + (k0 + 8 * g) * p.ldb;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float* src = bk + static_cast<int64_t>(j) * p.ldb;
-        if constexpr (NT == 2) {
-          const f32x2 v = gload<f32x2>(src, bo);
-          s.b[g][j][0] = v[0];
-          s.b[g][j][1] = v[1];
-        } else {
-          s.b[g][j][0] = gload<float>(src, bo);
+        for (int j = 0; j < 4; ++j) {
+          const float* src = bk + static_cast<int64_t>(j) * p.ldb;
+          if constexpr (NT == 2) {
+            const f32x2 v = gload<f32x2>(src, bo);
+            s.b[g][j][0] = v[0];
+            s.b[g][j][1] = v[1];
+          } else {
+            s.b[g][j][0] = gload<float>(src, bo);
+          }
         }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) s.a[g][m] = gload<f32x4>(A + k0 + 8 * g, opaque(a_off[m]));
       }
+    };
+    auto compute = [&](const Stage& s) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m) s.a[g][m] = gload<f32x4>(A + k0 + 8 * g, opaque(a_off[m]));
-    }
-  };
-  auto compute = [&](const Stage& s) {
+      for (int g = 0; g < 2; ++g)
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+          for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int c = 0; c < NT; ++c)
-            acc[m][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[g][m][j], s.b[g][j][c], acc[m][c],
-                                                             0, 0, 0);
-  };
+            for (int c = 0; c < NT; ++c)
+              acc[m][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[g][m][j], s.b[g][j][c], acc[m][c],
+                                                               0, 0, 0);
+    };
 
-  const int n = stages > first ? (stages - first + step - 1) / step : 0;
-  Stage st[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    load(st[d], d);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  int i = 0;
-  for (; i + 2 * D <= n; i += D) {
+    const int n = stages > first ? (stages - first + step - 1) / step : 0;
+    Stage st[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      compute(st[d]);
-      __builtin_amdgcn_sched_barrier(0);
-      load(st[d], i + D + d);
+      load(st[d], d);
       __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    int i = 0;
+    for (; i + 2 * D <= n; i += D) {
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (i + d < n) compute(st[d]);
-    if (i + D + d < n) load(st[d], i + D + d);
-  }
+      for (int d = 0; d < D; ++d) {
+        compute(st[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(st[d], i + D + d);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (i + D + d < n) compute(st[d]);
+    for (int d = 0; d < D; ++d) {
+      if (i + d < n) compute(st[d]);
+      if (i + D + d < n) load(st[d], i + D + d);
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (i + D + d < n) compute(st[d]);
 
-  // lane holds of MFMA (m, c): column NT l32 + c, rows 8 (r / 4) + 4 h + r % 4
-  float* d = part + wk * BM * PITCH + (32 * MT * wm + 4 * h) * PITCH + 32 * NT * wn + NT * l32;
+    // lane holds of MFMA (m, c): column NT l32 + c, rows 8 (r / 4) + 4 h + r % 4
+    float* d = part + wk * BM * PITCH + (32 * MT * wm + 4 * h) * PITCH + 32 * NT * wn + NT * l32;
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float* dst = d + (32 * m + 8 * (r >> 2) + (r & 3)) * PITCH;
-      if constexpr (NT == 2)
-        *reinterpret_cast<f32x2*>(dst) = f32x2{acc[m][0][r], acc[m][1][r]};
-      else
-        *dst = acc[m][0][r];
-    }
-  __syncthreads();
-  reduce_store<BM, BN, PITCH, WK, 64 * kWaves>(p, part, bm, bn, split);
+      for (int r = 0; r < 16; ++r) {
+        float* dst = d + (32 * m + 8 * (r >> 2) + (r & 3)) * PITCH;
+        if constexpr (NT == 2)
+          *reinterpret_cast<f32x2*>(dst) = f32x2{acc[m][0][r], acc[m][1][r]};
+        else
+          *dst = acc[m][0][r];
+      }
+    __syncthreads();
+  };
+  reduce_store<BM, BN, PITCH, WK, 64 * kWaves, WHOLE>(p, part, bm, bn, split, part_of);
 }
 
 // ---------------------------------------------------------------------------
@@ -607,18 +645,24 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void mm_direct_f32_kernel(c
 
 // Parts of K for `blocks` output blocks of which the chip holds 256 at once
 // (one per CU): as many as fill it, at most four, while every wave keeps
-// `min_k` of K.  One part without scratch, or while the stream is being
-// captured: a replay may run beside other launches that use the scratch.
-int k_parts(int64_t blocks, int K, int min_k, void* scratch, hipStream_t s) {
+// `min_k` of K.  Where the parts are not each a workgroup's (below), one
+// workgroup takes them in turn: a product's bits depend on its sizes alone.
+int k_parts(int64_t blocks, int K, int min_k) {
   int parts = 1;
   while (parts < 4 && blocks * parts * 2 <= 256 && K >= min_k * parts * 2) parts *= 2;
-  if (parts == 1 || !scratch) return 1;
+  return parts;
+}
+
+// Whether the launch may use the scratch.  Not while the stream is being
+// captured: a replay may run beside other launches that use it.
+bool usable(void* scratch, hipStream_t s) {
+  if (!scratch) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();  // not this launch's error
-    return 1;
+    return false;
   }
-  return st == hipStreamCaptureStatusNone ? parts : 1;
+  return st == hipStreamCaptureStatusNone;
 }
 
 void set_blocks(DirectArgs& a, int bm, int bn, int splits, void* scratch) {
@@ -650,6 +694,18 @@ bool offsets_fit(const DirectArgs& a, int elem) {
     *status = check_launch(name);                                                             \
   } while (0)
 
+// The same with a.splits parts of K: a workgroup each, or (whole) one for all
+#define TTLH_DIRECT_PARTS(kernel, whole, waves, name)                                         \
+  do {                                                                                        \
+    if (a.splits == 1 || usable(scratch, s)) {                                                \
+      TTLH_DIRECT(kernel, waves, name);                                                       \
+    } else {                                                                                  \
+      hipLaunchKernelGGL(HIP_KERNEL_NAME whole, dim3(a.grid_m * a.grid_n),                    \
+                         dim3(64 * (waves)), 0, s, a);                                        \
+      *status = check_launch(name);                                                           \
+    }                                                                                         \
+  } while (0)
+
 }  // namespace
 
 bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_t s, int* status) {
@@ -662,8 +718,8 @@ bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_
   const double k = a.K / 32.0;
   const auto rounds = [](int64_t blocks) { return static_cast<double>((blocks + 255) / 256); };
   const int64_t b64 = blocks_of(a, 32, 64), b128 = blocks_of(a, 32, 128), m64 = blocks_of(a, 64, 128);
-  const int p64 = k_parts(b64, a.K, 1024, scratch, s);
-  const int p128 = b128 >= 80 ? std::min(2, k_parts(b128, a.K, 1024, scratch, s)) : 1;
+  const int p64 = k_parts(b64, a.K, 1024);
+  const int p128 = b128 >= 80 ? std::min(2, k_parts(b128, a.K, 1024)) : 1;
   const double t[3] = {
       1 + (1.2 + 0.11 * k / p64) * rounds(b64 * p64) + (p64 > 1 ? 2 : 0),
       1 + (1.5 + 0.153 * k / p128) * rounds(b128 * p128) + (p128 > 1 ? 2 : 0),
@@ -673,10 +729,12 @@ bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_
   if (t[best] >= other_us) return false;
   if (best == 0) {
     set_blocks(a, 32, 64, p64, scratch);
-    TTLH_DIRECT((mm_direct_kernel<2, 4, 8, 3, 3>), 8, "mm_direct_kernel");
+    TTLH_DIRECT_PARTS((mm_direct_kernel<2, 4, 8, 3, 3>), (mm_direct_kernel<2, 4, 8, 3, 3, true>), 8,
+                      "mm_direct_kernel");
   } else if (best == 1) {
     set_blocks(a, 32, 128, p128, scratch);
-    TTLH_DIRECT((mm_direct_kernel<2, 8, 8, 2, 2>), 8, "mm_direct_kernel");
+    TTLH_DIRECT_PARTS((mm_direct_kernel<2, 8, 8, 2, 2>), (mm_direct_kernel<2, 8, 8, 2, 2, true>), 8,
+                      "mm_direct_kernel");
   } else {
     set_blocks(a, 64, 128, 1, nullptr);
     TTLH_DIRECT((mm_direct_kernel<4, 8, 4, 2, 2>), 4, "mm_direct_kernel");
@@ -699,9 +757,13 @@ bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, i
     else TTLH_DIRECT((mm_direct_bq_kernel<4, 2, 4, 4, 2, 2>), 4, "mm_direct_bq_kernel");
     return true;
   }
-  set_blocks(a, 32, 64, k_parts(blocks_of(a, 32, 64), a.K, 1024, scratch, s), scratch);
-  if (bits == 8) TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>), 8, "mm_direct_bq_kernel");
-  else TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>), 8, "mm_direct_bq_kernel");
+  set_blocks(a, 32, 64, k_parts(blocks_of(a, 32, 64), a.K, 1024), scratch);
+  if (bits == 8)
+    TTLH_DIRECT_PARTS((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>),
+                      (mm_direct_bq_kernel<2, 2, 8, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
+  else
+    TTLH_DIRECT_PARTS((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>),
+                      (mm_direct_bq_kernel<2, 2, 4, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
   return true;
 }
 
@@ -720,8 +782,9 @@ bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status) 
     set_blocks(a, 128, 128, 1, nullptr);
     TTLH_DIRECT((mm_direct_f32_kernel<2, 2, 2, 2, 2, 2>), 8, "mm_direct_f32_kernel");
   } else if (small <= 128) {
-    set_blocks(a, 32, 32, k_parts(small, a.K, 256, scratch, s), scratch);
-    TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4>), 8, "mm_direct_f32_kernel");
+    set_blocks(a, 32, 32, k_parts(small, a.K, 256), scratch);
+    TTLH_DIRECT_PARTS((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4>),
+                      (mm_direct_f32_kernel<1, 1, 1, 1, 8, 4, true>), 8, "mm_direct_f32_kernel");
   } else if (small <= 512) {
     set_blocks(a, 32, 32, 1, nullptr);
     TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 4, 4>), 4, "mm_direct_f32_kernel");
