@@ -687,24 +687,16 @@ bool offsets_fit(const DirectArgs& a, int elem) {
   return 128 * a.lda * elem < (int64_t(1) << 32) && (24 * a.ldb + a.N) * elem < (int64_t(1) << 32);
 }
 
-#define TTLH_DIRECT(kernel, waves, name)                                                      \
-  do {                                                                                        \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME kernel, dim3(a.grid_m * a.grid_n * a.splits),          \
-                       dim3(64 * (waves)), 0, s, a);                                          \
-    *status = check_launch(name);                                                             \
+#define TTLH_DIRECT_GRID(kernel, blocks, waves, name)                                          \
+  do {                                                                                         \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME kernel, dim3(blocks), dim3(64 * (waves)), 0, s, a);     \
+    *status = check_launch(name);                                                              \
   } while (0)
-
-// The same with a.splits parts of K: a workgroup each, or (whole) one for all
-#define TTLH_DIRECT_PARTS(kernel, whole, waves, name)                                         \
-  do {                                                                                        \
-    if (a.splits == 1 || usable(scratch, s)) {                                                \
-      TTLH_DIRECT(kernel, waves, name);                                                       \
-    } else {                                                                                  \
-      hipLaunchKernelGGL(HIP_KERNEL_NAME whole, dim3(a.grid_m * a.grid_n),                    \
-                         dim3(64 * (waves)), 0, s, a);                                        \
-      *status = check_launch(name);                                                           \
-    }                                                                                         \
-  } while (0)
+// a workgroup for each part of each block, and (kernels with WHOLE) one a block
+#define TTLH_DIRECT(kernel, waves, name) \
+  TTLH_DIRECT_GRID(kernel, a.grid_m * a.grid_n * a.splits, waves, name)
+#define TTLH_DIRECT_WHOLE(kernel, waves, name) \
+  TTLH_DIRECT_GRID(kernel, a.grid_m * a.grid_n, waves, name)
 
 }  // namespace
 
@@ -727,14 +719,18 @@ bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_
   };
   const int best = static_cast<int>(std::min_element(t, t + 3) - t);
   if (t[best] >= other_us) return false;
-  if (best == 0) {
+  const int parts = best == 0 ? p64 : best == 1 ? p128 : 1;
+  if (parts > 1 && !usable(scratch, s)) {
+    // (also where the parts would be of 32x128 blocks, which use half as many
+    // CUs here: the bits are those of the parts, not of the blocks' width)
+    set_blocks(a, 32, 64, parts, nullptr);
+    TTLH_DIRECT_WHOLE((mm_direct_kernel<2, 4, 8, 3, 3, true>), 8, "mm_direct_kernel");
+  } else if (best == 0) {
     set_blocks(a, 32, 64, p64, scratch);
-    TTLH_DIRECT_PARTS((mm_direct_kernel<2, 4, 8, 3, 3>), (mm_direct_kernel<2, 4, 8, 3, 3, true>), 8,
-                      "mm_direct_kernel");
+    TTLH_DIRECT((mm_direct_kernel<2, 4, 8, 3, 3>), 8, "mm_direct_kernel");
   } else if (best == 1) {
     set_blocks(a, 32, 128, p128, scratch);
-    TTLH_DIRECT_PARTS((mm_direct_kernel<2, 8, 8, 2, 2>), (mm_direct_kernel<2, 8, 8, 2, 2, true>), 8,
-                      "mm_direct_kernel");
+    TTLH_DIRECT((mm_direct_kernel<2, 8, 8, 2, 2>), 8, "mm_direct_kernel");
   } else {
     set_blocks(a, 64, 128, 1, nullptr);
     TTLH_DIRECT((mm_direct_kernel<4, 8, 4, 2, 2>), 4, "mm_direct_kernel");
@@ -758,12 +754,15 @@ bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, i
     return true;
   }
   set_blocks(a, 32, 64, k_parts(blocks_of(a, 32, 64), a.K, 1024), scratch);
-  if (bits == 8)
-    TTLH_DIRECT_PARTS((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>),
-                      (mm_direct_bq_kernel<2, 2, 8, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
-  else
-    TTLH_DIRECT_PARTS((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>),
-                      (mm_direct_bq_kernel<2, 2, 4, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
+  if (a.splits > 1 && !usable(scratch, s)) {
+    if (bits == 8)
+      TTLH_DIRECT_WHOLE((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
+    else
+      TTLH_DIRECT_WHOLE((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3, true>), 8, "mm_direct_bq_kernel");
+    return true;
+  }
+  if (bits == 8) TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 8, 8, 3, 3>), 8, "mm_direct_bq_kernel");
+  else TTLH_DIRECT((mm_direct_bq_kernel<2, 2, 4, 8, 3, 3>), 8, "mm_direct_bq_kernel");
   return true;
 }
 
@@ -783,8 +782,10 @@ bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status) 
     TTLH_DIRECT((mm_direct_f32_kernel<2, 2, 2, 2, 2, 2>), 8, "mm_direct_f32_kernel");
   } else if (small <= 128) {
     set_blocks(a, 32, 32, k_parts(small, a.K, 256), scratch);
-    TTLH_DIRECT_PARTS((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4>),
-                      (mm_direct_f32_kernel<1, 1, 1, 1, 8, 4, true>), 8, "mm_direct_f32_kernel");
+    if (a.splits > 1 && !usable(scratch, s))
+      TTLH_DIRECT_WHOLE((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4, true>), 8, "mm_direct_f32_kernel");
+    else
+      TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 8, 4>), 8, "mm_direct_f32_kernel");
   } else if (small <= 512) {
     set_blocks(a, 32, 32, 1, nullptr);
     TTLH_DIRECT((mm_direct_f32_kernel<1, 1, 1, 1, 4, 4>), 4, "mm_direct_f32_kernel");
