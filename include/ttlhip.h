@@ -342,6 +342,9 @@ int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* B,
 #define TTLH_BFP4 4
 #define TTLH_MATMUL_SCRATCH_BYTES (4198400)
 
+/* TTLH_MATMUL_SCRATCH_BYTES, or 0 where no product of these sizes uses it. */
+int64_t ttlh_matmul_scratch_bytes(int a_dtype, int b_dtype, int64_t M,
+                                  int64_t N, int64_t K);
 int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,
                         int b_dtype, int64_t ldb, void* C, int c_dtype,
                         int64_t ldc, int64_t M, int64_t N, int64_t K,

@@ -236,6 +236,31 @@ def test_scratches_are_bounded(monkeypatch):
         _check(o, a, b, True)
 
 
+def test_scratch_only_where_k_may_be_divided(monkeypatch):
+    # large products, short sums and packed weights' two passes take none; without
+    # memory for one the product runs all the same, with the same bits
+    Kn.release_workspaces()
+    for M, K, N, dt in [(1024, 4096, 1024, torch.bfloat16), (32, 1024, 256, torch.bfloat16),
+                        (512, 2048, 512, torch.float32)]:
+        a, b = _operands(M, K, N, 45, dt)
+        Kn.matmul(a, b, torch.zeros(M, N, dtype=dt, device="cuda"))
+        assert not Kn._MATMUL_SCRATCH
+    a, b = _operands(32, 4096, 256, 46)
+    c, d = (torch.zeros(32, 256, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+
+    def no_memory(*args, **kwargs):
+        raise torch.OutOfMemoryError("no memory for the scratch")
+
+    with monkeypatch.context() as m:
+        m.setattr(Kn.torch, "zeros", no_memory)
+        Kn.matmul(a, b, c)
+    assert not Kn._MATMUL_SCRATCH
+    Kn.matmul(a, b, d)
+    assert len(Kn._MATMUL_SCRATCH) == 1
+    assert torch.equal(c, d)
+    _check(d, a, b, True)
+
+
 def _packed(w, bits):
     return OB.pack_c(w) if bits == 8 else OB.pack4_c(w)
 

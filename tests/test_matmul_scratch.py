@@ -3,8 +3,10 @@ a GPU: the cached tensors are stand-ins."""
 
 from types import SimpleNamespace
 
+import pytest
 import torch
 
+from ttlhip import _lib as L
 from ttlhip import kernels as Kn
 
 
@@ -24,3 +26,18 @@ def test_a_scratch_is_its_own_devices(monkeypatch):
     for current, expect in ((0, mine), (1, None)):
         monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current, raising=False)
         assert Kn._matmul_scratch(d0, None, 0) is expect
+
+
+@pytest.mark.parametrize("a,b,M,N,K,uses", [
+    (L.TTLH_BF16, L.TTLH_BF16, 32, 4096, 11008, True),
+    (L.TTLH_BF16, L.TTLH_BF16, 32, 16384, 2048, True),
+    (L.TTLH_BF16, L.TTLH_BF16, 32, 4096, 2016, False),   # a wave would keep too little of K
+    (L.TTLH_BF16, L.TTLH_BF16, 1024, 1024, 11008, False),
+    (L.TTLH_F32, L.TTLH_F32, 256, 256, 512, True),
+    (L.TTLH_F32, L.TTLH_F32, 2048, 2048, 2048, False),
+    (L.TTLH_BF16, L.TTLH_BFP8, 32, 4096, 4096, True),
+    (L.TTLH_BF16, L.TTLH_BFP4, 32, 11008, 4096, False),
+    (L.TTLH_BF16, L.TTLH_BF16, 0, 32, 32, False)])
+def test_which_products_ask_for_it(a, b, M, N, K, uses):
+    need = L.load().ttlh_matmul_scratch_bytes(a, b, M, N, K)
+    assert need == (L.MATMUL_SCRATCH_BYTES if uses else 0)

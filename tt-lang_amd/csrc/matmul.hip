@@ -2173,6 +2173,12 @@ extern "C" int ttlh_matmul(const void* A, int a_dtype, int64_t lda, const void* 
                      stream);
 }
 
+extern "C" int64_t ttlh_matmul_scratch_bytes(int a_dtype, int b_dtype, int64_t M, int64_t N,
+                                             int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 30)) return 0;
+  return may_divide_k(a_dtype, b_dtype, M, N, K) ? TTLH_MATMUL_SCRATCH_BYTES : 0;
+}
+
 extern "C" int ttlh_matmul_scratch(const void* A, int a_dtype, int64_t lda, const void* B,
                                    int b_dtype, int64_t ldb, void* C, int c_dtype, int64_t ldc,
                                    int64_t M, int64_t N, int64_t K, int accumulate, void* scratch,

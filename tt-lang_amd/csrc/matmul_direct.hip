@@ -700,6 +700,16 @@ bool offsets_fit(const DirectArgs& a, int elem) {
 
 }  // namespace
 
+bool may_divide_k(int a_dtype, int b_dtype, int64_t M, int64_t N, int64_t K) {
+  DirectArgs a = {};
+  a.M = static_cast<int32_t>(M);
+  a.N = static_cast<int32_t>(N);
+  const int k = static_cast<int>(K);
+  if (a_dtype == TTLH_F32) return k_parts(blocks_of(a, 32, 32), k, 256) > 1;
+  if (b_dtype == TTLH_BFP8 || b_dtype == TTLH_BFP4) return k_parts(blocks_of(a, 32, 64), k, 1024) > 1;
+  return k_parts(blocks_of(a, 32, 128), k, 1024) > 1;  // few enough 32x64 blocks are few of these
+}
+
 bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_t s, int* status) {
   if (!offsets_fit(a, 2)) return false;
   set_c_vec(a);

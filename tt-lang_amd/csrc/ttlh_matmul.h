@@ -27,5 +27,7 @@ struct DirectArgs {
 bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_t s, int* status);
 bool launch_direct_f32(DirectArgs a, void* scratch, hipStream_t s, int* status);
 bool launch_direct_block(DirectArgs a, int bits, void* scratch, hipStream_t s, int* status);
+// false: none of them divides K in a product of these sizes
+bool may_divide_k(int a_dtype, int b_dtype, int64_t M, int64_t N, int64_t K);
 
 }  // namespace ttlh

@@ -126,6 +126,7 @@ SIGNATURES = {
                                         _i64, _i64, _vp]),
     "ttlh_matmul": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64, _i64,
                            _int, _vp]),
+    "ttlh_matmul_scratch_bytes": (_i64, [_int, _int, _i64, _i64, _i64]),
     "ttlh_matmul_scratch": (_int, [_vp, _int, _i64, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64,
                                    _i64, _int, _vp, _i64, _vp]),
     "ttlh_matmul_eltwise": (_int, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp,

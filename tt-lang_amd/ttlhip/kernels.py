@@ -74,12 +74,18 @@ def _workspace(device: torch.device, stream, nbytes: int,
 # The matmul's scratch (partial sums of products that divide K among several
 # workgroups, and their counters): a fixed 4 MiB per (device, stream), zeroed
 # once and left to the library; the oldest goes back to the allocator when a
-# 65th stream asks (torch itself hands out 32 per device).  Never allocated while
-# the stream is being captured; the library does not use it there either, so no
-# graph holds it.
+# 65th stream asks (torch itself hands out 32 per device).  Only for products that
+# may divide K, and never allocated while the stream is being captured; the library
+# does not use it there either, so no graph holds it.  Without it (here: no memory
+# left, too) a product takes longer and has the same bits.
 _MATMUL_SCRATCH: dict = {}
 _MATMUL_SCRATCH_MAX = 64
 _MATMUL_SCRATCH_LOCK = threading.Lock()
+
+
+@functools.lru_cache(maxsize=1024)
+def _matmul_scratch_bytes(a_code: int, b_code: int, M: int, N: int, K: int) -> int:
+    return int(L.load().ttlh_matmul_scratch_bytes(a_code, b_code, M, N, K))
 
 
 def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Tensor]:
@@ -96,12 +102,27 @@ def _matmul_scratch(device: torch.device, stream, sp: int) -> Optional[torch.Ten
             if t is None:
                 if torch.cuda.is_current_stream_capturing():
                     return None
-                with L.relaxed_capture():
-                    t = torch.zeros(L.MATMUL_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+                try:
+                    with L.relaxed_capture():
+                        t = torch.zeros(L.MATMUL_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+                except torch.OutOfMemoryError:
+                    return None
                 while len(_MATMUL_SCRATCH) >= _MATMUL_SCRATCH_MAX:
                     del _MATMUL_SCRATCH[next(iter(_MATMUL_SCRATCH))]
                 _MATMUL_SCRATCH[key] = t
     return t
+
+
+def _launch_matmul(a, a_code: int, b, b_code: int, ldb: int, c, c_code: int, M: int, N: int, K: int,
+                   accumulate: int, stream) -> int:
+    sp = L.stream_ptr(stream)
+    scratch = None
+    if _matmul_scratch_bytes(a_code, b_code, M, N, K):
+        scratch = _matmul_scratch(c.device, stream, sp)
+    return L.load().ttlh_matmul_scratch(
+        a.data_ptr(), a_code, a.stride(0), b.data_ptr(), b_code, ldb, c.data_ptr(), c_code,
+        c.stride(0), M, N, K, accumulate, scratch.data_ptr() if scratch is not None else 0,
+        L.MATMUL_SCRATCH_BYTES, sp)
 
 
 def release_workspaces() -> None:
@@ -439,12 +460,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, accumulate: bool =
     K2, N = b.shape
     if K2 != K or tuple(c.shape) != (M, N):
         raise ValueError(f"matmul shapes {tuple(a.shape)} @ {tuple(b.shape)} -> {tuple(c.shape)}")
-    sp = L.stream_ptr(stream)
-    scratch = _matmul_scratch(c.device, stream, sp)
-    L.call("ttlh_matmul_scratch", a.data_ptr(), L.dtype_code(a.dtype), a.stride(0), b.data_ptr(),
-           L.dtype_code(b.dtype), b.stride(0), c.data_ptr(), L.dtype_code(c.dtype), c.stride(0),
-           M, N, K, int(bool(accumulate)), scratch.data_ptr() if scratch is not None else 0,
-           L.MATMUL_SCRATCH_BYTES, sp)
+    L.check("ttlh_matmul_scratch",
+            _launch_matmul(a, L.dtype_code(a.dtype), b, L.dtype_code(b.dtype), b.stride(0), c,
+                           L.dtype_code(c.dtype), M, N, K, int(bool(accumulate)), stream))
 
 
 # Ops the fused GEMM epilogue (ttlh_matmul_eltwise) runs: + - * / max min
@@ -613,12 +631,7 @@ TWO_PASS_MIN_MACS = 1_500_000_000
 
 
 def _matmul_packed(a, bq, code: int, c, M: int, N: int, K: int, stream) -> int:
-    sp = L.stream_ptr(stream)
-    scratch = _matmul_scratch(c.device, stream, sp)
-    return L.load().ttlh_matmul_scratch(
-        a.data_ptr(), L.TTLH_BF16, a.stride(0), bq.data_ptr(), code, N, c.data_ptr(), L.TTLH_BF16,
-        c.stride(0), M, N, K, 0, scratch.data_ptr() if scratch is not None else 0,
-        L.MATMUL_SCRATCH_BYTES, sp)
+    return _launch_matmul(a, L.TTLH_BF16, bq, code, N, c, L.TTLH_BF16, M, N, K, 0, stream)
 
 
 def matmul_bfp8w(a: torch.Tensor, bq: torch.Tensor, c: torch.Tensor, stream=None,
