@@ -102,6 +102,28 @@ def test_blocks_of_256_into_a_result_off_its_pairs(M, K, N, dtype):
     assert bool((odd[:, 0] == 7).all()) and bool((odd[:, N + 1:] == 7).all())
 
 
+@pytest.mark.parametrize("M,K,N,pitch", [(4096, 96, 3072, 2 ** 19 + 8), (4096, 32, 3104, 2 ** 19 + 5),
+                                        (32, 2048, 96, 2 ** 26 + 1)])
+def test_bf16_results_past_32_bit_offsets(M, K, N, pitch):
+    # the result spans 2^31 elements and more: mm_bf16_kernel in place of the kernels
+    # with 32-bit offsets of C (192 blocks of 256x256 and more), and the
+    # register-direct kernels, whose offsets have 64
+    print(f"far results {M}x{K}x{N} pitch {pitch}", flush=True)
+    a, b = _operands(M, K, N, 37)
+    buf = torch.full(((M - 1) * pitch + N + 2,), 7.0, dtype=torch.bfloat16, device="cuda")
+    c = buf[1:].as_strided((M, N), (pitch, 1), 1)
+    Kn.matmul(a, b, c)
+    _check(c, a, b, True)
+    c0 = O.seeded((M, N), "normal", 38, torch.bfloat16).cuda()
+    c.copy_(c0)
+    Kn.matmul(a, b, c, accumulate=True)
+    exact = a.cpu().double() @ b.cpu().double() + c0.cpu().double()
+    bound = 1e-6 * math.sqrt(K) * float(exact.abs().max()) + exact.abs() * 2.0 ** -8
+    assert bool(((c.cpu().double() - exact).abs() <= bound).all())
+    around = buf.as_strided((M, N + 2), (pitch, 1), 0)
+    assert bool((around[:, 0] == 7).all()) and bool((around[:, N + 1] == 7).all())
+
+
 @pytest.mark.parametrize("M,K,N", [(4096, 32, 3072), (4096, 96, 3104), (32, 64, 49152)])
 def test_sums_in_the_fused_epilogues_order(M, K, N):
     # problems that the fused epilogue takes give the same bits with and
