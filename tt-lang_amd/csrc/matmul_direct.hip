@@ -30,8 +30,6 @@ typedef u32x4 u32x4a8 __attribute__((aligned(8)));  // packed tiles may be 8-byt
 template <int N>
 struct WordVec;
 template <>
-struct WordVec<1> { typedef uint32_t type; };
-template <>
 struct WordVec<2> { typedef u32x2 type; };
 template <>
 struct WordVec<4> { typedef u32x4 type; };
@@ -171,10 +169,14 @@ __device__ __forceinline__ void reduce_store(const DirectArgs& p, const float* p
   }
   if (p.splits == 1) return;
   // The workgroup that arrives last at this block's counter adds the parts,
-  // in split order; nobody waits for anybody.  Every wave's parts are at the
-  // coherence point (vmcnt 0) before the barrier, so before thread 0 counts
-  // them in; a device-scope fence would do the same by writing back the whole
-  // L2 (measured: 20 us a launch).
+  // in split order; nobody waits for anybody.  That the parts come before the
+  // counter is an assumption about the hardware, not a rule of the memory model:
+  // both are relaxed device-scope accesses, and a wave counts in only after
+  // vmcnt(0) and a barrier.  A device-scope store is written through, and its
+  // acknowledgement is taken to mean that it has reached the device's coherence
+  // point, where the last workgroup's loads read.  A release fence would say the
+  // same in the model's terms, by writing back the whole L2 (measured: 20 us a
+  // launch).
   __shared__ int last;
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
@@ -215,10 +217,6 @@ struct BfStage {
   u32x4 a[MT];
   vec b[8];
 };
-
-template <typename V>
-__device__ __forceinline__ uint32_t word(const V& v, int i) { return v[i]; }
-__device__ __forceinline__ uint32_t word(const uint32_t& v, int) { return v; }
 
 template <int MT, int NPL, int WK, int D, int OCC, bool WHOLE = false>
 __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArgs p) {
@@ -269,7 +267,7 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
         u32x4 f;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-          const uint32_t x = word(s.b[2 * d], c >> 1), y = word(s.b[2 * d + 1], c >> 1);
+          const uint32_t x = s.b[2 * d][c >> 1], y = s.b[2 * d + 1][c >> 1];
           f[d] = (c & 1) ? perm_hi(x, y) : perm_lo(x, y);
         }
 #pragma unroll
@@ -312,14 +310,10 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float* d = mine + (16 * m + r) * PITCH;
-        if constexpr (NPL == 2) {
-          *reinterpret_cast<f32x2*>(d) = f32x2{acc[m][0][r], acc[m][1][r]};
-        } else {
 #pragma unroll
-          for (int c = 0; c < NPL; c += 4)
-            *reinterpret_cast<f32x4*>(d + c) =
-                f32x4{acc[m][c][r], acc[m][c + 1][r], acc[m][c + 2][r], acc[m][c + 3][r]};
-        }
+        for (int c = 0; c < NPL; c += 4)
+          *reinterpret_cast<f32x4*>(d + c) =
+              f32x4{acc[m][c][r], acc[m][c + 1][r], acc[m][c + 2][r], acc[m][c + 3][r]};
       }
     __syncthreads();
   };
@@ -716,7 +710,10 @@ bool launch_direct_bf16(DirectArgs a, double other_us, void* scratch, hipStream_
   // Modelled time of each block shape, us: per round of 256 workgroups a fixed
   // part and one per 32-k stage of a wave's share, fitted to measurements of 50
   // problems from 32x32x32 to 4096x512x2048 (the choice was the fastest of the
-  // shapes or within 10% of it, but for a few at 20%).
+  // shapes or within 10% of it, but for a few at 20%).  There is no term for
+  // memory: where B's bytes bound all shapes alike the times are too short (32 x
+  // 11008 x 4096 13.7 us, measured 21.8), and a choice against another kernel near
+  // a tie is not borne out by them.
   const double k = a.K / 32.0;
   const auto rounds = [](int64_t blocks) { return static_cast<double>((blocks + 255) / 256); };
   const int64_t b64 = blocks_of(a, 32, 64), b128 = blocks_of(a, 32, 128), m64 = blocks_of(a, 64, 128);
