@@ -327,8 +327,9 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_kernel(const DirectArg
 // byte l, so the 16 elements that it decodes share one shift; it writes them
 // as bf16 to the wave's own LDS, from where ds_read_b64_tr_b16 gives the
 // MFMA's B operand (lane l of 16: column l of four 32-byte row pieces).
-// Decoding bounds this kernel (3.6 VALU instructions an element), not the
-// packed bytes' 8 to 9 us.
+// Decoding takes most of the time (3.6 VALU instructions an element; VALU on 57%
+// of a SIMD's cycles at 32 x 4096 x 11008, MFMA on 13%), not the packed bytes' 8 to
+// 9 us.
 template <int MT, int NT, int BITS>
 struct BqStage {
   u32x4 a[MT];
@@ -371,8 +372,9 @@ __global__ __launch_bounds__(64 * WK, OCC) void mm_direct_bq_kernel(const Direct
   constexpr int kBias = BITS == 8 ? 133 : 129;
   // decoded stage: k row r at position (r & 3) + 4 (r >> 3) + 16 ((r >> 2) & 1),
   // which puts the rows of one transpose read on consecutive positions; the
-  // pitch is an odd number of 32-byte pieces, so 32 lanes' pieces fall in
-  // different banks
+  // pitch is an odd number of 32-byte pieces, so 32 lanes' pieces of a read fall
+  // in different banks (in a write two lanes of 16 share theirs; the LDS is busy
+  // 15% of the time)
   constexpr int kRow = 64 * NT + 32, kStageLds = 32 * kRow;
   constexpr int kPart = BM * PITCH * 4;
   __shared__ __attribute__((aligned(16))) uint8_t lds[WK * (kPart > kStageLds ? kPart : kStageLds)];

@@ -51,6 +51,7 @@
 // K (16 rows, one chunk each): chunk c of row r at c ^ (r & 15), for D = 64, where
 // two rows share the banks, at c ^ ((r >> 1) & 7); V (4 rows x 4 chunks per 32
 // lanes of a transpose read): at c ^ 4 (r & 3), for D = 64 at c ^ 4 ((r >> 1) & 1).
+// (No bank conflict is counted in any form.)
 // The next block's loads run while the current block computes.
 // Softmax runs in the log2 domain: exp2(fma(s, scale log2 e, -m)) in
 // sdpa_fwd_kernel, with the block max taken on the raw scores (sign of the
